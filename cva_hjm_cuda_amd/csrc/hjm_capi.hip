@@ -204,6 +204,7 @@ int plan_init(hjm_plan p, const hjm_market* market, const hjm_swap* swap, const 
     std::vector<uint16_t> wf;
     std::vector<double> wf64;
     if (p->use_mfma) {
+        int scale = 0;
         if (cfg->precision == HJM_FP64) {
             HJM_HIP(mfma64_kernels_prepare(), HJM_ERR_DEVICE);
             build_mfma64_block_map(market->drifts, market->volatilities, cfg->dt, swap->dtau,
@@ -214,7 +215,8 @@ int plan_init(hjm_plan p, const hjm_market* market, const hjm_swap* swap, const 
                     HJM_ERR_DEVICE);
         } else {
             HJM_HIP(mfma_kernels_prepare(), HJM_ERR_DEVICE);
-            build_mfma_block_map(market->drifts, market->volatilities, cfg->dt, swap->dtau, wf);
+            scale = build_mfma_block_map(market->spot_rates, market->drifts, market->volatilities,
+                                         cfg->dt, swap->dtau, ref_mfma_tiles(D), wf);
             HJM_TRY(dev_alloc(&p->d_wfrag, wf.size()));
             HJM_HIP(hipMemcpyAsync(p->d_wfrag, wf.data(), wf.size() * sizeof(uint16_t),
                                    hipMemcpyHostToDevice, p->stream),
@@ -226,10 +228,11 @@ int plan_init(hjm_plan p, const hjm_market* market, const hjm_swap* swap, const 
         mg.path0 = cfg->path_offset;
         mg.seed_lo = g.seed_lo;
         mg.seed_hi = g.seed_hi;
-        mg.dt = cfg->dt;
+        mg.dt = ldexp(cfg->dt, -scale);
+        mg.down = ldexpf(1.f, -scale);
         for (int j = 0; j < kTenors; ++j) {
-            mg.a0[j] = g.a0[j];
-            mg.spot[j] = (float)market->spot_rates[j];
+            mg.a0[j] = ldexp(g.a0[j], scale);
+            mg.spot[j] = ldexpf((float)market->spot_rates[j], scale);
             mg.spot64[j] = market->spot_rates[j];
         }
     }

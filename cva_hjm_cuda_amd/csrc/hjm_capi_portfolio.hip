@@ -310,11 +310,12 @@ int pplan_init(hjm_portfolio_plan p, const hjm_market* market, const hjm_portfol
         HJM_HIP(hipMemcpy(p->d_normals, cfg->host_normals, n * sizeof(double), hipMemcpyHostToDevice),
                 HJM_ERR_DEVICE);
     }
+    int scale = 0;
     if (p->use_mfma) {
         HJM_HIP(mfma_kernels_prepare(), HJM_ERR_DEVICE);
         std::vector<uint16_t> wf;
-        build_mfma_block_map(market->drifts, market->volatilities, cfg->dt, pf->dtau, wf,
-                             MfmaMap::kPortfolio);
+        scale = build_mfma_block_map(market->spot_rates, market->drifts, market->volatilities, cfg->dt,
+                                     pf->dtau, kMfmaPfMTiles, wf, MfmaMap::kPortfolio);
         HJM_TRY(dev_alloc(&p->d_wfrag, wf.size()));
         HJM_HIP(hipMemcpy(p->d_wfrag, wf.data(), wf.size() * sizeof(uint16_t), hipMemcpyHostToDevice),
                 HJM_ERR_DEVICE);
@@ -335,9 +336,10 @@ int pplan_init(hjm_portfolio_plan p, const hjm_market* market, const hjm_portfol
         mg.path0 = cfg->path_offset;
         mg.seed_lo = g.seed_lo;
         mg.seed_hi = g.seed_hi;
-        mg.dt = cfg->dt;
+        mg.dt = ldexp(cfg->dt, -scale);
+        mg.down = ldexpf(1.f, -scale);
         for (int j = 0; j < kTenors; ++j) {
-            mg.spot[j] = (float)market->spot_rates[j];
+            mg.spot[j] = ldexpf((float)market->spot_rates[j], scale);
             mg.spot64[j] = market->spot_rates[j];
         }
     }

@@ -54,7 +54,9 @@ struct RefGrid {
     double a0[kTenors];  // frozen block-0 integral: spot_j summed stride times (FP64)
 };
 
-// Matrix-core FP32 path kernel (reference semantics, 50-step blocks).
+// Matrix-core path kernels (50-step blocks). The FP32 kernels hold the curve and the
+// integrals times 2^k (build_mfma_block_map): spot and a0 carry that factor, dt its inverse,
+// and `down` = 2^-k scales the curve values that leave the kernel; all of it exact.
 struct MfmaGrid {
     int ndates;
     int pad;
@@ -64,6 +66,7 @@ struct MfmaGrid {
     double dt;
     double a0[kTenors];   // frozen block-0 integrals (FP64)
     float spot[kTenors];
+    float down;
     double spot64[kTenors];  // the FP64 kernel's initial curve
 };
 

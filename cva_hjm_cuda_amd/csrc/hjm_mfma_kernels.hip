@@ -1,8 +1,13 @@
 // hjm_mfma_kernels.hip -- FP32 path, valuation and adjoint-seed kernels on the matrix cores.
 //
 // Each 50-step block is the affine map [f_out; integral rows] = W [f_in; phi; 1]
-// (hjm_mfma_plan.h), computed with v_mfma_f32_16x16x32_bf16 as six products of three-way
-// bf16 splits (W's parts precomputed, the operand split exactly in registers), which
+// (hjm_mfma_plan.h), computed on the matrix cores with split operands: the curve columns with
+// v_mfma_f32_16x16x32_bf16 as six products of three-way bf16 splits (W's parts precomputed,
+// the operand split exactly in registers), the shock columns with v_mfma_f32_16x16x32_f16 as
+// three products of two-way fp16 splits (22 bits of a term that is a few percent of the
+// curve; 258 products per wave-block at 5 M-tiles against 408 with bf16 throughout, and 1.5
+// instead of 5.5 VALU instructions to split a shock: the 10y path kernel at 131072 paths went
+// from 0.51 to 0.42 ms, its results' error against FP64 unchanged). The split products
 // keeps FP32 accuracy while running on the matrix cores concurrently with the VALU
 // (FP32 MFMA on gfx950 shares the vector pipeline and gains nothing over it). A wave owns
 // 32 paths = 2 N-tiles of 16 (the portfolio kernel's shape is a launch choice). The
@@ -35,6 +40,8 @@ namespace hjm {
 
 typedef float f4_t __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u4_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ f4_t mfma_bf16(u4_t a, u4_t b, f4_t c)
@@ -73,6 +80,42 @@ __device__ __forceinline__ Split8 split8(const float* x)
     return s;
 }
 
+__device__ __forceinline__ f4_t mfma_f16(u4_t a, u4_t b, f4_t c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8_t, a),
+                                                  __builtin_bit_cast(h8_t, b), c, 0, 0, 0);
+}
+
+// Two fp16 parts of 8 FP32 values, each rounded to nearest: h + l = x to 2^-22 |x| + 2^-25
+// (the low part's subnormals end there).
+struct SplitH8 {
+    u4_t h, l;
+};
+
+// Three instructions per pair: v_cvt_pk_f16_f32, then the low parts by v_fma_mixlo/mixhi_f16
+// (1.5 per value; the exact three-way bf16 split takes 5.5). The operands are opaque where the
+// compiler would otherwise fold: a product feeding the conversions would be fused into one
+// of them and not the other, and the low part would then belong to another high part; the
+// pair is converted once; x - h stays an FMA with the opaque factor -1.
+__device__ __forceinline__ SplitH8 split8h(const float* x)
+{
+    SplitH8 s;
+    float neg1 = -1.f;
+    asm("" : "+s"(neg1));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        float a = x[2 * j], b = x[2 * j + 1];
+        asm("" : "+v"(a), "+v"(b));
+        h2_t h = {(_Float16)a, (_Float16)b};
+        asm("" : "+v"(h));
+        const h2_t l = {(_Float16)__builtin_fmaf((float)h[0], neg1, a),
+                        (_Float16)__builtin_fmaf((float)h[1], neg1, b)};
+        s.h[j] = __builtin_bit_cast(uint32_t, h);
+        s.l[j] = __builtin_bit_cast(uint32_t, l);
+    }
+    return s;
+}
+
 // reference kernel: 8 waves of 2 N-tiles (16 paths each); the portfolio kernel's shape
 // is a template choice (MfmaShape)
 constexpr int kNT = 2;
@@ -88,23 +131,22 @@ __host__ __device__ constexpr int shock_chunk_last_quad(int s)
 // Issue plan: the matrix-core work of the block is spread over the quads that generate
 // shocks, so that their RNG (VALU) runs beside a share of the MFMAs: chunk c's M-tiles
 // [m0, m1) go to quad q. Quads 3, 7 and 11 make no Philox call (their shocks come from
-// calls made earlier) and get no MFMA work; curve chunks 0, 1 are ready at the start,
-// shock chunk s once its last shock's call is made (quads 1, 4, 6, 9, 12); shock chunk 4
-// completes with the last quad and runs after it.
+// calls made earlier) and get no MFMA work; curve chunks 0, 1 (six products a tile) are
+// ready at the start, shock chunk s (three products) once its last shock's call is made
+// (quads 1, 4, 6, 9, 12); shock chunk 4 completes with the last quad and runs after it.
 struct IssueSlot {
     int chunk, m0, m1;
 };
 template <int MT>
-__host__ __device__ constexpr IssueSlot issue_slot(int q, int half)
+__host__ __device__ constexpr IssueSlot issue_slot(int q)
 {
     const int split = (MT + 1) / 2;
-    (void)half;
     switch (q) {
     case 0: return {0, 0, split};
     case 1: return {0, split, MT};
-    case 2: return {1, 0, MT};
-    case 4: return {2, 0, split};
-    case 5: return {2, split, MT};
+    case 2: return {1, 0, split};
+    case 4: return {1, split, MT};
+    case 5: return {2, 0, MT};
     case 6: return {3, 0, split};
     case 8: return {3, split, MT};
     case 9: return {4, 0, split};
@@ -123,12 +165,12 @@ __device__ __forceinline__ void for_each_index(F& f, std::integer_sequence<int, 
 
 // One 50-step block: acc = W x [fin; shocks of steps b*50 .. b*50+49; 1]. kStore: also
 // write the block's normals to zs[step][factor][path] (FP32) for a later reverse sweep.
-// kTwoAcc: the five small split products (Wh xm, Wm xh, Wh xl, Wl xh, Wm xm) accumulate
-// apart from Wh xh and join it once at the end. The matrix cores drop the low bits of
-// products far below the accumulator (measured: C = 1 plus 32 products of 2^-27 returns 1;
-// small positive contributions are lost, small negative ones kept), which biases a
-// single accumulator holding the curve (FP32 vs FP64: EE 1.4e-6 -> 3.2e-7 on the 10y
-// precision workload with two). It costs 4 registers per tile and N-tile.
+// kTwoAcc: the small split products (all but Wh xh) accumulate apart from Wh xh and join it
+// once at the end. The matrix cores drop the low bits of products far below the accumulator
+// (measured: C = 1 plus 32 products of 2^-27 returns 1; small positive contributions are
+// lost, small negative ones kept), which biases a single accumulator holding the curve (FP32
+// vs FP64: EE 1.4e-6 -> 3.2e-7 on the 10y precision workload with two). It costs 4 registers
+// per tile and N-tile.
 template <int MT, int NT, bool kStore, bool kInterleave, bool kTwoAcc>
 __device__ __forceinline__ void mfma_block(const u4_t* __restrict__ lds_w, const float (&fin)[NT][16],
                                            f4_t (&acc)[MT][NT], const MfmaGrid& g,
@@ -149,41 +191,50 @@ __device__ __forceinline__ void mfma_block(const u4_t* __restrict__ lds_w, const
     for (int m = 0; m < MT2; ++m)
 #pragma unroll
         for (int n = 0; n < NT; ++n) acc2[m][n] = f4_t{0.f, 0.f, 0.f, 0.f};
-    // M-tiles [m0, m1) of chunk c, less the structurally zero curve chunks (the reference
-    // and portfolio maps share tiles 0..3, whose zeros agree; c and m are constants once
-    // unrolled)
-    auto tiles = [&](int c, int m0, int m1, const Split8 (&xs)[NT]) {
+    // one product for the N-tiles in turn (consecutive MFMAs then write different
+    // accumulators): large = Wh xh, otherwise into the small products' accumulator
+    auto product = [&](int m, bool large, u4_t a, auto fn) {
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            if (kTwoAcc && !large) acc2[kTwoAcc ? m : 0][n] = fn(a, n, acc2[kTwoAcc ? m : 0][n]);
+            else acc[m][n] = fn(a, n, acc[m][n]);
+        }
+    };
+    // M-tiles [m0, m1) of curve chunk c, less the structurally zero ones (the reference and
+    // portfolio maps share tiles 0..3, whose zeros agree; c and m are constants once
+    // unrolled), and of a shock chunk
+    auto curve_tiles = [&](int c, int m0, int m1, const Split8 (&xs)[NT]) {
 #pragma unroll
         for (int m = m0; m < m1; ++m) {
             if (mfma_chunk_zero(m, c, false)) continue;
-            const u4_t* a = lds_w + ((m * kMfmaChunks + c) * kMfmaParts) * kWave + off;
+            const u4_t* a = lds_w + mfma_frag(m, c, 0) * kWave + off;
             const u4_t ah = a[0], am = a[kWave], al = a[2 * kWave];
-#pragma unroll
-            for (int n = 0; n < NT; ++n) {
-                f4_t v;
-                if constexpr (kTwoAcc) {
-                    acc[m][n] = mfma_bf16(ah, xs[n].h, acc[m][n]);
-                    v = acc2[m][n];
-                } else {
-                    v = mfma_bf16(ah, xs[n].h, acc[m][n]);
-                }
-                v = mfma_bf16(ah, xs[n].m, v);
-                v = mfma_bf16(am, xs[n].h, v);
-                v = mfma_bf16(ah, xs[n].l, v);
-                v = mfma_bf16(al, xs[n].h, v);
-                v = mfma_bf16(am, xs[n].m, v);
-                if constexpr (kTwoAcc) acc2[m][n] = v;
-                else acc[m][n] = v;
-            }
+            product(m, true, ah, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].h, v); });
+            product(m, false, ah, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].m, v); });
+            product(m, false, am, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].h, v); });
+            product(m, false, ah, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].l, v); });
+            product(m, false, al, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].h, v); });
+            product(m, false, am, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].m, v); });
         }
     };
-    // split operands of the 7 chunks: curve chunks from fin (registers 8 c .. 8 c + 7),
-    // shock chunk s from values 8 s .. 8 s + 7 of z
-    Split8 xs[kMfmaChunks][NT];
+    auto shock_tiles = [&](int c, int m0, int m1, const SplitH8 (&xs)[NT]) {
+#pragma unroll
+        for (int m = m0; m < m1; ++m) {
+            const u4_t* a = lds_w + mfma_frag(m, c, 0) * kWave + off;
+            const u4_t ah = a[0], al = a[kWave];
+            product(m, true, ah, [&](u4_t w, int n, f4_t v) { return mfma_f16(w, xs[n].h, v); });
+            product(m, false, ah, [&](u4_t w, int n, f4_t v) { return mfma_f16(w, xs[n].l, v); });
+            product(m, false, al, [&](u4_t w, int n, f4_t v) { return mfma_f16(w, xs[n].h, v); });
+        }
+    };
+    // split operands: curve chunks from fin (registers 8 c .. 8 c + 7), shock chunk s from
+    // values 8 s .. 8 s + 7 of z
+    Split8 xc[2][NT];
+    SplitH8 xs[kMfmaChunks - 2][NT];
 #pragma unroll
     for (int c = 0; c < 2; ++c)
 #pragma unroll
-        for (int n = 0; n < NT; ++n) xs[c][n] = split8(&fin[n][8 * c]);
+        for (int n = 0; n < NT; ++n) xc[c][n] = split8(&fin[n][8 * c]);
     // shocks: value v = 3 q + k of lane group grp is factor k of step 4 q + grp; step 50
     // (lane group 2, q = 12) carries the constant 1 of the drift in factor 0.
     float z[NT][8 * (kMfmaChunks - 2)];
@@ -229,16 +280,17 @@ __device__ __forceinline__ void mfma_block(const u4_t* __restrict__ lds_w, const
         for (int s = 0; s < kMfmaChunks - 2; ++s)
             if (q == shock_chunk_last_quad(s))
 #pragma unroll
-                for (int n = 0; n < NT; ++n) xs[2 + s][n] = split8(&z[n][8 * s]);
+                for (int n = 0; n < NT; ++n) xs[s][n] = split8h(&z[n][8 * s]);
         // this quad's share of the matrix work (its operands are complete); it runs on
         // the matrix cores beside the RNG of this and the other waves
-        constexpr IssueSlot is = issue_slot<MT>(q, 0);
+        constexpr IssueSlot is = issue_slot<MT>(q);
         if constexpr (is.chunk >= 0) {
-            tiles(is.chunk, is.m0, is.m1, xs[is.chunk]);
+            if constexpr (is.chunk < 2) curve_tiles(is.chunk, is.m0, is.m1, xc[is.chunk]);
+            else shock_tiles(is.chunk, is.m0, is.m1, xs[is.chunk - 2]);
             if constexpr (kInterleave) {
                 // within the quad: one MFMA, then a share of the RNG's VALU instructions
 #pragma unroll
-                for (int i = 0; i < (is.m1 - is.m0) * NT * 6; ++i) {
+                for (int i = 0; i < (is.m1 - is.m0) * NT * (is.chunk < 2 ? 6 : 3); ++i) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                     __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);
                 }
@@ -248,7 +300,7 @@ __device__ __forceinline__ void mfma_block(const u4_t* __restrict__ lds_w, const
         if constexpr (kInterleave) __builtin_amdgcn_sched_barrier(0);
     };
     for_each_index(quad, std::make_integer_sequence<int, kMfmaQuads>{});
-    tiles(kMfmaChunks - 1, 0, MT, xs[kMfmaChunks - 1]);
+    shock_tiles(kMfmaChunks - 1, 0, MT, xs[kMfmaChunks - 3]);
     if constexpr (kTwoAcc) {
 #pragma unroll
         for (int m = 0; m < MT; ++m)
@@ -269,7 +321,7 @@ __global__ __launch_bounds__(kMfmaBlock) void ref_paths_mfma_kernel(const MfmaGr
 {
     constexpr int kInt = MT - 3;  // M-tiles holding integral rows (tile 3 holds both kinds)
     extern __shared__ u4_t lds_w[];
-    for (int t = threadIdx.x; t < MT * kMfmaChunks * kMfmaParts * kWave; t += kMfmaBlock)
+    for (int t = threadIdx.x; t < MT * kMfmaTileFrags * kWave; t += kMfmaBlock)
         lds_w[t] = wfrag[t];
     __syncthreads();
 
@@ -313,7 +365,7 @@ __global__ __launch_bounds__(kMfmaBlock) void ref_paths_mfma_kernel(const MfmaGr
 #pragma unroll
         for (int n = 0; n < kNT; ++n)
             if (live[n]) {
-                num_x[P + path[n]] = (double)g.spot[1];
+                num_x[P + path[n]] = (double)(g.spot[1] * g.down);
                 num_y[P + path[n]] = exp(-g.a0[1] * g.dt);
             }
     }
@@ -359,7 +411,7 @@ __global__ __launch_bounds__(kMfmaBlock) void ref_paths_mfma_kernel(const MfmaGr
                     cv = Ck[n][t2];
                 }
             if (live[n]) {
-                if (grp == gx) num_x[(int64_t)slot * P + path[n]] = (double)xv;
+                if (grp == gx) num_x[(int64_t)slot * P + path[n]] = (double)(xv * g.down);
                 if (grp == ga)
                     num_y[(int64_t)slot * P + path[n]] = exp(-((double)av - (double)cv) * g.dt);
             }
@@ -427,7 +479,7 @@ __global__ __launch_bounds__(WAVES * kWave) void pf_paths_mfma_kernel(const Mfma
                     for (int r = 0; r < 4; ++r) {
                         const int R = 16 * m + 4 * grp + r;
                         if (R < kTenors)
-                            curves[((int64_t)e * kTenors + R) * P + path[n]] = fin[n][4 * m + r];
+                            curves[((int64_t)e * kTenors + R) * P + path[n]] = fin[n][4 * m + r] * g.down;
                     }
                 if (sum_lane) logb[(int64_t)e * P + path[n]] = lnB[n];
             }
@@ -448,7 +500,7 @@ __global__ __launch_bounds__(WAVES * kWave) void pf_paths_mfma_kernel(const Mfma
 }
 
 // The portfolio path kernel's instantiated launch shapes {N-tiles per wave, waves}: {2, 8},
-// {2, 12}, {1, 12}, {1, 16} (the block map's 84 KB of LDS allow one workgroup per CU;
+// {2, 12}, {1, 12}, {1, 16} (64 KB of block map in LDS;
 // 2 N-tiles take about 164 VGPRs, at most 3 waves per SIMD).
 constexpr int kPathShapes = 4;
 template <bool kStore, bool kPersist>

@@ -11,7 +11,7 @@
 //   portfolio semantics (52 rows, 4 M-tiles): row 51 holds the short rate's left-point sum
 //       sum_{r=0}^{S-1} f_r[0] = (sum_{r=0}^{S-1} T^r f_in)[0]
 //                               + sum_t (sum_{q=0}^{S-2-t} T^q (m dt + V s_t))[0].
-// The kernel computes W x [f_in; phi; 1] with v_mfma_f32_16x16x32_bf16. K has 224 entries
+// The kernel computes W x [f_in; phi; 1] with v_mfma_f32_16x16x32_{bf16,f16}. K has 224 entries
 // in 7 chunks of 32; in chunk c lane group g = lane / 16 supplies slots i = 0..7, the
 // K index being 32 c + 8 g + i:
 //   chunks 0, 1: curve row R = 16 (2c + i/4) + 4 g + i%4 (zero column where R > 50): the
@@ -19,11 +19,14 @@
 //   chunks 2..6 (s = c - 2): value v = 8 s + i of lane group g, which generates the steps
 //     t = 4 q + g, q = 0..12: v = 3 q + k is factor k of step t (t < 50); at t = 50
 //     (g = 2, q = 12) factor 0 is the constant 1 carrying the drift; other slots are zero.
-// W (FP64) is split into three bf16 parts W = Wh + Wm + Wl (round to nearest); the kernel
-// splits its FP32 operand x exactly (truncation: xh + xm + xl = x) and accumulates the six
-// products Wh xh + Wh xm + Wm xh + Wh xl + Wl xh + Wm xm in FP32, which leaves an error of
-// the order of FP32 rounding.
-// Fragment [m][c][part][lane][i] = part of W[16 m + lane % 16][32 c + 8 (lane / 16) + i].
+// The curve columns of W (FP64) are split into three bf16 parts W = Wh + Wm + Wl (round to
+// nearest); the kernel splits the curve exactly (truncation: xh + xm + xl = x) and accumulates
+// the six products Wh xh + Wh xm + Wm xh + Wh xl + Wl xh + Wm xm in FP32, which leaves an
+// error of the order of FP32 rounding. The shock columns take two fp16 parts on either side
+// (11 bits each, to nearest) and three products Wh xh + Wh xl + Wl xh: what they leave out is
+// below 2^-21 of a shock's contribution, which is itself a few percent of the curve, with
+// either sign -- under the curve's own FP32 rounding, at half the products.
+// Fragment (m, c, part)[lane][i] = part of W[16 m + lane % 16][32 c + 8 (lane / 16) + i].
 #pragma once
 #include <math.h>
 #include <stdint.h>
@@ -42,13 +45,21 @@ constexpr int kMfmaPfMTiles = 4;  // portfolio map: 52 output rows -> 4 x 16
 constexpr int kMfmaQuads = 13;    // steps 4 q + g, q = 0..12, per lane group
 constexpr int kMfmaChunks = 7;    // 2 curve chunks + 5 shock chunks of 32 K entries
 constexpr int kMfmaK = 32 * kMfmaChunks;  // 224
-constexpr int kMfmaParts = 3;     // bf16 parts of W
-// bf16 elements of one kernel's fragments
-constexpr int kMfmaFragElems = kMfmaMTiles * kMfmaChunks * kMfmaParts * kWave * 8;
-constexpr int kMfmaPfFragElems = kMfmaPfMTiles * kMfmaChunks * kMfmaParts * kWave * 8;
+constexpr int kMfmaParts = 3;      // bf16 parts of W's curve columns (and of -gamma)
+constexpr int kMfmaShockParts = 2; // fp16 parts of W's shock columns
+// fragments (64 lanes x 8 16-bit elements) of one M-tile: curve chunks 0, 1 in three bf16
+// parts, shock chunks 2..6 in two fp16 parts
+constexpr int kMfmaTileFrags = 2 * kMfmaParts + (kMfmaChunks - 2) * kMfmaShockParts;  // 16
+__host__ __device__ constexpr int mfma_frag(int m, int c, int part)
+{
+    return m * kMfmaTileFrags +
+           (c < 2 ? c * kMfmaParts : 2 * kMfmaParts + (c - 2) * kMfmaShockParts) + part;
+}
+// 16-bit elements of one kernel's fragments
+constexpr int kMfmaPfFragElems = kMfmaPfMTiles * kMfmaTileFrags * kWave * 8;
 // LDS bytes of the first mt M-tiles' fragments (the reference kernel stages only its live
 // tiles)
-constexpr int ref_mfma_lds_bytes(int mt) { return mt * kMfmaChunks * kMfmaParts * kWave * 8 * 2; }
+constexpr int ref_mfma_lds_bytes(int mt) { return mt * kMfmaTileFrags * kWave * 8 * 2; }
 
 enum class MfmaMap { kReference, kPortfolio };
 
@@ -116,80 +127,67 @@ inline std::vector<double> mfma_block_map_dense(const double* drift, const doubl
     const int n = kTenors, S = kMfmaStride;
     const int rows = pf ? n + 1 : 2 * n;
     const double c = dt / dtau, sq = sqrt(dt);
-    auto matmul = [n](const std::vector<double>& A, const std::vector<double>& B) {
-        std::vector<double> C((size_t)n * n, 0.0);
-        for (int i = 0; i < n; ++i)
-            for (int k = 0; k < n; ++k) {
-                const double a = A[(size_t)i * n + k];
-                if (a == 0.0) continue;
-                for (int j = 0; j < n; ++j) C[(size_t)i * n + j] += a * B[(size_t)k * n + j];
-            }
-        return C;
+    // y = T x for one column of values `step` apart: T has two entries a row
+    auto apply = [n, c](const double* x, double* y, int step) {
+        for (int j = 0; j < n - 1; ++j)
+            for (int m = 0; m < step; ++m)
+                y[j * step + m] = (1.0 - c) * x[j * step + m] + c * x[(j + 1) * step + m];
+        for (int m = 0; m < step; ++m)
+            y[(n - 1) * step + m] = -c * x[(n - 2) * step + m] + (1.0 + c) * x[(n - 1) * step + m];
     };
-    std::vector<double> T((size_t)n * n, 0.0);
-    for (int j = 0; j < n - 1; ++j) {
-        T[(size_t)j * n + j] = 1.0 - c;
-        T[(size_t)j * n + j + 1] = c;
-    }
-    T[(size_t)(n - 1) * n + n - 1] = 1.0 + c;
-    T[(size_t)(n - 1) * n + n - 2] = -c;
-    // Tp[s] = T^s, Cs[s] = sum_{q=0}^{s} T^q
-    std::vector<std::vector<double>> Tp(S + 1), Cs(S + 1);
-    Tp[0].assign((size_t)n * n, 0.0);
-    for (int j = 0; j < n; ++j) Tp[0][(size_t)j * n + j] = 1.0;
-    Cs[0] = Tp[0];
+    // T^S, sum_{q=1}^{S} T^q and row 0 of sum_{q=0}^{S-1} T^q
+    std::vector<double> Tp((size_t)n * n, 0.0), next((size_t)n * n), Sum((size_t)n * n, 0.0);
+    std::vector<double> first(n, 0.0);
+    for (int j = 0; j < n; ++j) Tp[(size_t)j * n + j] = 1.0;
     for (int s = 1; s <= S; ++s) {
-        Tp[s] = matmul(T, Tp[s - 1]);
-        Cs[s] = Cs[s - 1];
-        for (size_t i = 0; i < Cs[s].size(); ++i) Cs[s][i] += Tp[s][i];
+        for (int m = 0; m < n; ++m) first[m] += Tp[m];
+        apply(Tp.data(), next.data(), n);
+        Tp.swap(next);
+        for (size_t i = 0; i < Sum.size(); ++i) Sum[i] += Tp[i];
     }
-    auto mv = [n](const std::vector<double>& M, const double* v, int j) {
-        double s = 0.0;
-        for (int i = 0; i < n; ++i) s += M[(size_t)j * n + i] * v[i];
-        return s;
-    };
-    std::vector<double> mdt(n);
-    for (int i = 0; i < n; ++i) mdt[i] = drift[i] * dt;
     std::vector<double> W((size_t)rows * kMfmaK, 0.0);
+    int shock_k[kMfmaStride][3] = {}, const_k = 0;
     for (int k = 0; k < kMfmaK; ++k) {
         const MfmaColumn col = mfma_column(k);
-        auto put = [&](int row, double v) { W[(size_t)row * kMfmaK + k] = v; };
-        if (col.kind == MfmaColumn::kCurve) {
-            const int R = col.row;
-            for (int j = 0; j < n; ++j) put(j, Tp[S][(size_t)j * n + R]);
-            if (pf) {
-                put(n, Cs[S - 1][R]);
-            } else {
-                for (int j = 0; j < n; ++j) {
-                    double sa = 0.0;
-                    for (int q = 1; q <= S; ++q) sa += Tp[q][(size_t)j * n + R];
-                    put(n + j, sa);
-                }
-            }
-        } else if (col.kind == MfmaColumn::kShock) {
-            const int t = col.step;
-            std::vector<double> sv(n);
-            for (int i = 0; i < n; ++i) sv[i] = sq * vols[col.factor * n + i];
-            for (int j = 0; j < n; ++j) put(j, mv(Tp[S - 1 - t], sv.data(), j));
-            if (pf) {
-                if (t <= S - 2) put(n, mv(Cs[S - 2 - t], sv.data(), 0));
-            } else {
-                for (int j = 0; j < n; ++j) put(n + j, mv(Cs[S - 1 - t], sv.data(), j));
-            }
-        } else if (col.kind == MfmaColumn::kConst) {
-            for (int j = 0; j < n; ++j) {
-                double sf = 0.0, sa = 0.0;
-                for (int tt = 0; tt < S; ++tt) {
-                    sf += mv(Tp[S - 1 - tt], mdt.data(), j);
-                    if (!pf) sa += mv(Cs[S - 1 - tt], mdt.data(), j);
-                    else if (j == 0 && tt <= S - 2) sa += mv(Cs[S - 2 - tt], mdt.data(), 0);
-                }
-                put(j, sf);
-                if (!pf) put(n + j, sa);
-                else if (j == 0) put(n, sa);
-            }
-        }
+        if (col.kind == MfmaColumn::kShock) shock_k[col.step][col.factor] = k;
+        if (col.kind == MfmaColumn::kConst) const_k = k;
+        if (col.kind != MfmaColumn::kCurve) continue;
+        for (int j = 0; j < n; ++j) W[(size_t)j * kMfmaK + k] = Tp[(size_t)j * n + col.row];
+        if (pf) W[(size_t)n * kMfmaK + k] = first[col.row];
+        else
+            for (int j = 0; j < n; ++j) W[(size_t)(n + j) * kMfmaK + k] = Sum[(size_t)j * n + col.row];
     }
+    // A vector v added at step t reaches the block's end as T^{S-1-t} v and its integral as
+    // sum_{q <= S-1-t} T^q v (the left-point sum: q <= S-2-t, tenor 0): walked from the last
+    // step back, u = T^q v and its running sum.
+    auto walk = [&](const double* v, auto put) {
+        std::vector<double> u(v, v + n), acc(n, 0.0), t(n);
+        for (int q = 0; q < S; ++q) {
+            const double left = acc[0];
+            for (int j = 0; j < n; ++j) acc[j] += u[j];
+            put(S - 1 - q, u.data(), acc.data(), left);
+            apply(u.data(), t.data(), 1);
+            u.swap(t);
+        }
+    };
+    std::vector<double> v(n);
+    for (int f = 0; f < 3; ++f) {
+        for (int i = 0; i < n; ++i) v[i] = sq * vols[f * n + i];
+        walk(v.data(), [&](int t, const double* u, const double* acc, double left) {
+            const int k = shock_k[t][f];
+            for (int j = 0; j < n; ++j) W[(size_t)j * kMfmaK + k] = u[j];
+            if (pf) W[(size_t)n * kMfmaK + k] = left;
+            else
+                for (int j = 0; j < n; ++j) W[(size_t)(n + j) * kMfmaK + k] = acc[j];
+        });
+    }
+    for (int i = 0; i < n; ++i) v[i] = drift[i] * dt;
+    walk(v.data(), [&](int, const double* u, const double* acc, double left) {
+        for (int j = 0; j < n; ++j) W[(size_t)j * kMfmaK + const_k] += u[j];
+        if (pf) W[(size_t)n * kMfmaK + const_k] += left;
+        else
+            for (int j = 0; j < n; ++j) W[(size_t)(n + j) * kMfmaK + const_k] += acc[j];
+    });
     return W;
 }
 
@@ -211,29 +209,78 @@ inline double bf16_value(uint16_t b)
     return (double)f;
 }
 
-// Fragments of the three bf16 parts of W in the kernel's A-operand order.
-inline void build_mfma_block_map(const double* drift, const double* vols, double dt, double dtau,
-                                 std::vector<uint16_t>& frag, MfmaMap map = MfmaMap::kReference)
+// fp16 bits of x rounded to nearest (ties to even); |x| < 65504
+inline uint16_t fp16_rne(float x)
+{
+    uint32_t u;
+    memcpy(&u, &x, 4);
+    const uint32_t sign = (u >> 16) & 0x8000u;
+    u &= 0x7fffffffu;
+    if (u < 0x38800000u) {   // below 2^-14: subnormal, quantum 2^-24
+        const float m = nearbyintf(ldexpf(x < 0.f ? -x : x, 24));
+        return (uint16_t)(sign | (uint32_t)m);
+    }
+    u += 0xfffu + ((u >> 13) & 1u);
+    return (uint16_t)(sign | ((u >> 13) - (112u << 10)));
+}
+
+inline double fp16_value(uint16_t h)
+{
+    const uint32_t e = (h >> 10) & 31u, m = h & 1023u;
+    if (!e) return ((h & 0x8000u) ? -0x1p-24 : 0x1p-24) * m;
+    const uint32_t u = ((uint32_t)(h & 0x8000u) << 16) | ((e + 112u) << 23) | (m << 13);
+    float f;
+    memcpy(&f, &u, 4);
+    return (double)f;
+}
+
+// Fragments of W in the kernel's A-operand order: the curve columns as three bf16 parts, the
+// shock columns (and the drift constant's) times 2^k as two fp16 parts rounded to nearest.
+// Returns k: the power of two that brings the largest shock entry to [2^12, 2^13), where
+// both parts of every entry within 2^-26 of it are normal fp16 numbers (without the scale
+// the entries, 1e-4 .. 1e-2, would leave their low parts to subnormals). The kernels hold the
+// curve and the integrals times 2^k too, so both kinds of products share an accumulator;
+// k is also bounded by the curve's size (max |spot| 2^k <= 2^40), and 0 without shocks.
+// mtiles: the M-tiles built (the reference kernel's live ones).
+inline int build_mfma_block_map(const double* spot, const double* drift, const double* vols, double dt,
+                                double dtau, int mtiles, std::vector<uint16_t>& frag,
+                                MfmaMap map = MfmaMap::kReference)
 {
     const bool pf = map == MfmaMap::kPortfolio;
-    const int mtiles = pf ? kMfmaPfMTiles : kMfmaMTiles;
     const int rows = pf ? kTenors + 1 : 2 * kTenors;
     const std::vector<double> W = mfma_block_map_dense(drift, vols, dt, dtau, map);
-    frag.assign((size_t)mtiles * kMfmaChunks * kMfmaParts * kWave * 8, 0);
+    double top = 0.0, curve = 0.0;
+    for (int row = 0; row < rows; ++row)
+        for (int k = 64; k < kMfmaK; ++k) top = std::max(top, fabs(W[(size_t)row * kMfmaK + k]));
+    for (int j = 0; j < kTenors; ++j) curve = std::max(curve, fabs(spot[j]));
+    int scale = 0;
+    if (top > 0.0) {
+        scale = std::max(-120, std::min(120, 12 - ilogb(top)));
+        if (curve > 0.0) scale = std::min(scale, std::max(12 - ilogb(top) - 40, 39 - ilogb(curve)));
+    }
+    const double up = ldexp(1.0, scale);
+    frag.assign((size_t)mtiles * kMfmaTileFrags * kWave * 8, 0);
     for (int m = 0; m < mtiles; ++m)
         for (int c = 0; c < kMfmaChunks; ++c)
             for (int l = 0; l < kWave; ++l)
                 for (int i = 0; i < 8; ++i) {
                     const int row = 16 * m + l % 16, k = 32 * c + 8 * (l / 16) + i;
                     const double w = row < rows ? W[(size_t)row * kMfmaK + k] : 0.0;
-                    const uint16_t h = bf16_rne(w);
-                    const double r1 = w - bf16_value(h);
-                    const uint16_t mm = bf16_rne(r1);
-                    const uint16_t lo = bf16_rne(r1 - bf16_value(mm));
-                    const uint16_t parts[3] = {h, mm, lo};
-                    for (int p = 0; p < kMfmaParts; ++p)
-                        frag[((((size_t)m * kMfmaChunks + c) * kMfmaParts + p) * kWave + l) * 8 + i] = parts[p];
+                    uint16_t parts[3] = {0, 0, 0};
+                    if (c < 2) {
+                        parts[0] = bf16_rne(w);
+                        const double r1 = w - bf16_value(parts[0]);
+                        parts[1] = bf16_rne(r1);
+                        parts[2] = bf16_rne(r1 - bf16_value(parts[1]));
+                    } else {
+                        parts[0] = fp16_rne((float)(w * up));
+                        parts[1] = fp16_rne((float)(w * up - fp16_value(parts[0])));
+                    }
+                    const int np = c < 2 ? kMfmaParts : kMfmaShockParts;
+                    for (int p = 0; p < np; ++p)
+                        frag[((size_t)mfma_frag(m, c, p) * kWave + l) * 8 + i] = parts[p];
                 }
+    return scale;
 }
 
 // The FP64 block map for v_mfma_f64_16x16x4f64 (ref_paths_mfma64_kernel). One instruction

@@ -209,7 +209,7 @@ typedef struct {
 /* Launch shapes of the portfolio plan's kernels (0 in a field: its default). The VALU
  * path kernel (FP64, host normals, or path_kernel = VECTOR) uses block_size and
  * blocks_per_cu; the matrix-core FP32 path kernel path_tiles, path_waves and
- * blocks_per_cu (0 or 1: its block map fills 84 KB of LDS, one workgroup per CU); the
+ * blocks_per_cu (0 or 1: one workgroup per CU); the
  * matrix-core valuation value_tiles, value_waves and value_stage. The FP64 matrix-core
  * path kernel (FP64 with path_kernel = MATRIX) has a fixed shape. Results do not depend
  * on the shapes. hjm_portfolio_autotune measures them. */
