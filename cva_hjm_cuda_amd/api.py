@@ -127,6 +127,8 @@ def _declare(lib):
     lib.hjm_status_string.restype = C.c_char_p
     lib.hjm_status_string.argtypes = [i]
     lib.hjm_device_count.argtypes = [C.POINTER(i)]
+    lib.hjm_release_cached_memory.argtypes = []
+    lib.hjm_release_cached_memory.restype = None
     lib.hjm_cva_weights.argtypes = [i, d, d, d, _dp]
     lib.hjm_hjm_drift.argtypes = [_dp, d, _dp]
     lib.hjm_plan_create.argtypes = [C.POINTER(C.c_void_p), C.POINTER(_Market), C.POINTER(_Swap),
@@ -247,6 +249,11 @@ def device_count() -> int:
     n = C.c_int(0)
     _check(library().hjm_device_count(C.byref(n)), "hjm_device_count")
     return n.value
+
+
+def release_cached_memory() -> None:
+    """Return the device memory the library keeps between calls (hjm_release_cached_memory)."""
+    library().hjm_release_cached_memory()
 
 
 # ---- reference-semantics simulation ------------------------------------------------

@@ -370,6 +370,7 @@ int hjm_calibrate_pca(const hjm_calibration* c, hjm_calibration_results* r)
         for (size_t w = 0; w < W && rc == HJM_OK; ++w)
             rc = hjm_hjm_drift(&ld[w * F * kN], c->dtau, r->drifts + w * kN);
     }
+    (void)hipStreamSynchronize(nullptr);
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
     dev_free(d_curves);

@@ -50,8 +50,9 @@ int ref_grid(double expiry, double dtau, double dt, int* stride, int* nsteps, in
 
 struct hjm_plan_s {
     int device = 0;
-    hipStream_t stream = nullptr;
-    hipEvent_t ev[5] = {};
+    ContextHolder ctx;
+    hipStream_t stream = nullptr;   // the context's, as are the events and h_res
+    hipEvent_t* ev = nullptr;
     int precision = HJM_FP64;
     bool host_rng = false;
     bool do_pfe = false;
@@ -85,6 +86,7 @@ void plan_release(hjm_plan p)
     int prev = -1;
     (void)hipGetDevice(&prev);
     (void)hipSetDevice(p->device);
+    const bool clean = p->ctx.quiesce();
     dev_free(p->d_normals);
     dev_free(p->d_wfrag);
     dev_free(p->d_wfrag64);
@@ -94,10 +96,8 @@ void plan_release(hjm_plan p)
     dev_free(p->d_partials);
     dev_free(p->d_sums);
     dev_free(p->d_selws);
-    if (p->h_res) (void)hipHostFree(p->h_res);
-    for (auto& e : p->ev)
-        if (e) (void)hipEventDestroy(e);
-    if (p->stream) (void)hipStreamDestroy(p->stream);
+    p->ctx.give();
+    if (!clean) pool_release_all();
     if (prev >= 0) (void)hipSetDevice(prev);
     delete p;
 }
@@ -181,21 +181,19 @@ int plan_init(hjm_plan p, const hjm_market* market, const hjm_swap* swap, const 
 
     DeviceGuard guard;
     HJM_TRY(guard.set(cfg->device));
-    HJM_HIP(hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking), HJM_ERR_DEVICE);
-    for (auto& ev : p->ev) HJM_HIP(hipEventCreate(&ev), HJM_ERR_DEVICE);
+    HJM_TRY(p->ctx.take(cfg->device, sizeof(double) * (kStatSlots + kTenors)));
+    p->stream = p->ctx.c->stream;
+    p->ev = p->ctx.c->ev;
+    p->h_res = static_cast<double*>(p->ctx.c->host);
+    // rows: numeraire slots 1 .. D, exposure dates 0 .. D-1; the others are never read
     const size_t slots = (size_t)kTenors * cfg->paths;
     HJM_TRY(dev_alloc(&p->d_nx, slots));
     HJM_TRY(dev_alloc(&p->d_ny, slots));
-    HJM_TRY(dev_alloc(&p->d_ex, slots));
-    // exposure rows past the last date are never written by a run
-    HJM_HIP(hipMemset(p->d_ex, 0, slots * sizeof(double)), HJM_ERR_DEVICE);
     HJM_TRY(dev_alloc(&p->d_partials, (size_t)p->nblocks * kStatSlots));
     HJM_TRY(dev_alloc(&p->d_sums, kStatSlots + kTenors));
     p->d_pfe = p->d_sums + kStatSlots;
-    HJM_HIP(hipHostMalloc((void**)&p->h_res, sizeof(double) * (kStatSlots + kTenors),
-                          hipHostMallocDefault),
-            HJM_ERR_ALLOC);
     if (p->do_pfe) {
+        HJM_TRY(dev_alloc(&p->d_ex, slots));
         const size_t wsb = bracket_workspace_bytes(
             kTenors, bracket_plan(cfg->paths, p->pfe_rank, sizeof(double)), sizeof(double));
         if (wsb) HJM_TRY(dev_alloc(&p->d_selws, wsb));
@@ -236,8 +234,6 @@ int plan_init(hjm_plan p, const hjm_market* market, const hjm_swap* swap, const 
             mg.spot64[j] = market->spot_rates[j];
         }
     }
-    HJM_HIP(hipMemsetAsync(p->d_nx, 0, slots * sizeof(double), p->stream), HJM_ERR_DEVICE);
-    HJM_HIP(hipMemsetAsync(p->d_ny, 0, slots * sizeof(double), p->stream), HJM_ERR_DEVICE);
     if (p->host_rng) {
         const size_t n = (size_t)cfg->paths * S * 3;
         HJM_TRY(dev_alloc(&p->d_normals, n));
@@ -253,6 +249,7 @@ int plan_init(hjm_plan p, const hjm_market* market, const hjm_swap* swap, const 
 int plan_launch(hjm_plan p, bool keep_exposures, float* zs = nullptr)
 {
     hipStream_t st = p->stream;
+    if (keep_exposures && !p->d_ex) HJM_TRY(dev_alloc(&p->d_ex, (size_t)kTenors * p->paths));
     HJM_HIP(hipEventRecord(p->ev[0], st), HJM_ERR_DEVICE);
     const bool f64 = p->precision == HJM_FP64;
     hipError_t err;
@@ -311,18 +308,21 @@ int plan_collect(hjm_plan p, hjm_results* r)
         if (p->do_pfe) memcpy(r->pfe, p->h_res + kStatSlots, sizeof(double) * p->grid.ndates);
     }
     const int64_t P = p->paths;
-    auto transpose_back = [&](const double* dsrc, double* dst) -> int {
-        std::vector<double> tmp((size_t)kTenors * P);
-        if (hipMemcpy(tmp.data(), dsrc, tmp.size() * sizeof(double), hipMemcpyDeviceToHost) !=
-            hipSuccess)
+    // device rows [lo, hi) to the caller's [path][slot], the other slots 0
+    auto transpose_back = [&](const double* dsrc, double* dst, int lo, int hi) -> int {
+        std::vector<double> tmp((size_t)(hi - lo) * P);
+        if (hipMemcpy(tmp.data(), dsrc + (size_t)lo * P, tmp.size() * sizeof(double),
+                      hipMemcpyDeviceToHost) != hipSuccess)
             return HJM_ERR_DEVICE;
         for (int64_t i = 0; i < P; ++i)
-            for (int t = 0; t < kTenors; ++t) dst[i * kTenors + t] = tmp[(size_t)t * P + i];
+            for (int t = 0; t < kTenors; ++t)
+                dst[i * kTenors + t] = (t >= lo && t < hi) ? tmp[(size_t)(t - lo) * P + i] : 0.0;
         return HJM_OK;
     };
-    if (r->num_x) HJM_TRY(transpose_back(p->d_nx, r->num_x));
-    if (r->num_y) HJM_TRY(transpose_back(p->d_ny, r->num_y));
-    if (r->exposures) HJM_TRY(transpose_back(p->d_ex, r->exposures));
+    const int D = p->grid.ndates;
+    if (r->num_x) HJM_TRY(transpose_back(p->d_nx, r->num_x, 1, D + 1));
+    if (r->num_y) HJM_TRY(transpose_back(p->d_ny, r->num_y, 1, D + 1));
+    if (r->exposures) HJM_TRY(transpose_back(p->d_ex, r->exposures, 0, D));
     if (r->timings_ms) {
         float ms = 0.f;
         for (int i = 0; i < 4; ++i) {
@@ -447,25 +447,25 @@ int hjm_simulate_reference(const hjm_market* market, const hjm_swap* swap,
 int hjm_cva_greeks_reference(const hjm_market* market, const hjm_swap* swap,
                              const hjm_config* cfg, hjm_greeks* gr)
 {
-    if (!gr) return HJM_ERR_NULL;
+    if (!gr || !cfg) return HJM_ERR_NULL;
+    hjm_config config = *cfg;
+    if (config.pfe_quantile <= 1.0) config.pfe_quantile = 0.0;   // no PFE here (> 1: rejected)
     hjm_plan p = nullptr;
-    HJM_TRY(hjm_plan_create(&p, market, swap, cfg));
+    HJM_TRY(hjm_plan_create(&p, market, swap, &config));
     constexpr int kOut = 5 * kTenors;  // g0, g1, g2, sum of lambda_e, d spot
     struct Cleanup {
         hjm_plan p;
         float *gx = nullptr, *gA = nullptr, *zs = nullptr;
         double *part = nullptr, *sums = nullptr, *sap = nullptr;
-        hipEvent_t e0 = nullptr, e1 = nullptr;
         ~Cleanup()
         {
+            (void)p->ctx.quiesce();
             dev_free(gx);
             dev_free(zs);
             dev_free(gA);
             dev_free(part);
             dev_free(sums);
             dev_free(sap);
-            if (e0) (void)hipEventDestroy(e0);
-            if (e1) (void)hipEventDestroy(e1);
             hjm_plan_destroy(p);
         }
     } c{p};
@@ -479,8 +479,7 @@ int hjm_cva_greeks_reference(const hjm_market* market, const hjm_swap* swap,
     HJM_TRY(dev_alloc(&c.part, (size_t)nb * kOut));
     HJM_TRY(dev_alloc(&c.sums, kOut + kTenors));  // then the per-slot sums of gA
     HJM_TRY(dev_alloc(&c.sap, (size_t)p->nblocks * kTenors));
-    HJM_HIP(hipEventCreate(&c.e0), HJM_ERR_DEVICE);
-    HJM_HIP(hipEventCreate(&c.e1), HJM_ERR_DEVICE);
+    hipEvent_t e0 = p->ev[5], e1 = p->ev[6];
     // the matrix-core forward keeps its normals for the reverse sweep (one FP32 per factor
     // per evolved step and path); without the memory the sweep regenerates them
     if (p->use_mfma && cfg->adjoint_normals == HJM_ADJ_NORMALS_AUTO &&
@@ -488,7 +487,7 @@ int hjm_cva_greeks_reference(const hjm_market* market, const hjm_swap* swap,
         c.zs = nullptr;
     hipStream_t st = p->stream;
     HJM_TRY(plan_launch(p, false, c.zs));
-    HJM_HIP(hipEventRecord(c.e0, st), HJM_ERR_DEVICE);
+    HJM_HIP(hipEventRecord(e0, st), HJM_ERR_DEVICE);
     const double dt = p->grid.dt;
     const double cc = dt / swap->dtau;
     HJM_HIP(launch_ref_adjoint_seed(p->ep, dt, p->d_nx, p->d_ny, c.gx, c.gA, c.sap, st),
@@ -498,7 +497,7 @@ int hjm_cva_greeks_reference(const hjm_market* market, const hjm_swap* swap,
     HJM_HIP(launch_ref_adjoint(p->grid, cc, sqrt(dt), p->d_normals, c.zs, c.gx, c.gA, c.part, st),
             HJM_ERR_LAUNCH);
     HJM_HIP(launch_column_sum(c.part, nb, kOut, c.sums, st), HJM_ERR_LAUNCH);
-    HJM_HIP(hipEventRecord(c.e1, st), HJM_ERR_DEVICE);
+    HJM_HIP(hipEventRecord(e1, st), HJM_ERR_DEVICE);
     hjm_results r{};
     r.cva = gr->cva;
     r.cva_stderr = gr->cva_stderr;
@@ -537,7 +536,7 @@ int hjm_cva_greeks_reference(const hjm_market* market, const hjm_swap* swap,
     if (gr->timings_ms) {
         float fwd = 0.f, adj = 0.f;
         HJM_HIP(hipEventElapsedTime(&fwd, p->ev[0], p->ev[4]), HJM_ERR_DEVICE);
-        HJM_HIP(hipEventElapsedTime(&adj, c.e0, c.e1), HJM_ERR_DEVICE);
+        HJM_HIP(hipEventElapsedTime(&adj, e0, e1), HJM_ERR_DEVICE);
         gr->timings_ms[0] = fwd;
         gr->timings_ms[1] = adj;
         gr->timings_ms[2] = fwd + adj;
@@ -584,6 +583,7 @@ int hjm_simulate_reference_blockwise(const hjm_market* market, const hjm_swap* s
         hipEvent_t ev[5] = {};
         ~Bufs()
         {
+            if (st) (void)hipStreamSynchronize(st);
             dev_free(normals);
             dev_free(s0);
             dev_free(s1);
@@ -714,6 +714,7 @@ int hjm_generate_normals(uint64_t seed, int64_t path_offset, int64_t paths, int3
         rc = HJM_ERR_LAUNCH;
     else if (hipMemcpy(out, d, n * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess)
         rc = HJM_ERR_DEVICE;
+    (void)hipStreamSynchronize(nullptr);
     dev_free(d);
     return rc;
 }
@@ -740,6 +741,7 @@ int hjm_box_muller_parts(const uint32_t* words, int64_t n, int32_t device, float
                  hipMemcpy(cosine, d + n, b, hipMemcpyDeviceToHost) != hipSuccess ||
                  hipMemcpy(sine, d + 2 * n, b, hipMemcpyDeviceToHost) != hipSuccess)
             rc = HJM_ERR_DEVICE;
+        (void)hipStreamSynchronize(nullptr);
         dev_free(d);
     }
     dev_free(dw);
@@ -769,6 +771,7 @@ int hjm_select_kth(const double* values, int32_t rows, int64_t n, int64_t k, int
     if (rc == HJM_OK && hipDeviceSynchronize() != hipSuccess) rc = HJM_ERR_LAUNCH;
     if (rc == HJM_OK && hipMemcpy(out, d_out, rows * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess)
         rc = HJM_ERR_DEVICE;
+    (void)hipStreamSynchronize(nullptr);
     dev_free(d);
     dev_free(d_out);
     dev_free(ws);

@@ -16,8 +16,9 @@ using namespace hjm_host;
 
 struct hjm_pplan_s {
     int device = 0;
-    hipStream_t stream = nullptr;
-    hipEvent_t ev[5] = {};
+    ContextHolder ctx;
+    hipStream_t stream = nullptr;   // the context's, as are the events
+    hipEvent_t* ev = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     hjm_tuning tuning{256, 0, 0, 0, 0, 0, 0, 0, 0, 0};  // block size 256, the rest defaults
@@ -45,7 +46,7 @@ struct hjm_pplan_s {
     void* d_ex = nullptr;
     double* d_partials = nullptr;
     double* d_sums = nullptr;
-    double* d_pfe = nullptr;
+    double* d_pfe = nullptr;  // [date][set], after the sums
     char* d_selws = nullptr;  // bracket-selection workspace (PFE)
     uint32_t* d_loparts = nullptr;  // counts below the bracket per row and statistics workgroup
     void* d_coef = nullptr;
@@ -65,6 +66,7 @@ void pplan_release(hjm_portfolio_plan p)
     int prev = -1;
     (void)hipGetDevice(&prev);
     (void)hipSetDevice(p->device);
+    const bool clean = p->ctx.quiesce();
     if (p->exec) (void)hipGraphExecDestroy(p->exec);
     if (p->graph) (void)hipGraphDestroy(p->graph);
     dev_free(p->d_normals);
@@ -73,7 +75,6 @@ void pplan_release(hjm_portfolio_plan p)
     dev_free(p->d_ex);
     dev_free(p->d_partials);
     dev_free(p->d_sums);
-    dev_free(p->d_pfe);
     dev_free(p->d_selws);
     dev_free(p->d_loparts);
     dev_free(p->d_coef);
@@ -85,9 +86,8 @@ void pplan_release(hjm_portfolio_plan p)
     dev_free(p->d_w);
     dev_free(p->d_wfrag);
     dev_free(p->d_wfrag64);
-    for (auto& e : p->ev)
-        if (e) (void)hipEventDestroy(e);
-    if (p->stream) (void)hipStreamDestroy(p->stream);
+    p->ctx.give();
+    if (!clean) pool_release_all();
     if (prev >= 0) (void)hipSetDevice(prev);
     delete p;
 }
@@ -234,8 +234,10 @@ int pplan_init(hjm_portfolio_plan p, const hjm_market* market, const hjm_portfol
     HJM_HIP(hipDeviceGetAttribute(&p->cus, hipDeviceAttributeMultiprocessorCount, cfg->device),
             HJM_ERR_DEVICE);
     pplan_apply_tuning(p, p->tuning);
-    HJM_HIP(hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking), HJM_ERR_DEVICE);
-    for (auto& ev : p->ev) HJM_HIP(hipEventCreate(&ev), HJM_ERR_DEVICE);
+    // pinned: the column sums and the PFE rows of one run
+    HJM_TRY(p->ctx.take(cfg->device, sizeof(double) * (size_t)pf->nsets * (2 * nd + 2)));
+    p->stream = p->ctx.c->stream;
+    p->ev = p->ctx.c->ev;
     const size_t rsz = (p->precision == HJM_FP64) ? sizeof(double) : sizeof(float);
     const size_t P = (size_t)cfg->paths;
     // workgroups of the statistics: 256 paths (exposure pass) or the fused pass's blocks
@@ -248,8 +250,8 @@ int pplan_init(hjm_portfolio_plan p, const hjm_market* market, const hjm_portfol
     HJM_TRY(dev_alloc(&raw, (size_t)pf->nsets * nd * P * rsz));
     p->d_ex = raw;
     HJM_TRY(dev_alloc(&p->d_partials, (size_t)pf->nsets * nb * (nd + 2)));
-    HJM_TRY(dev_alloc(&p->d_sums, (size_t)pf->nsets * (nd + 2)));
-    HJM_TRY(dev_alloc(&p->d_pfe, (size_t)pf->nsets * nd));
+    HJM_TRY(dev_alloc(&p->d_sums, (size_t)pf->nsets * (2 * nd + 2)));
+    p->d_pfe = p->d_sums + (size_t)pf->nsets * (nd + 2);
     if (p->do_pfe) {
         const size_t wsb = bracket_workspace_bytes(pf->nsets * nd, bracket_plan(cfg->paths, p->pfe_rank, (int)rsz),
                                                    (int)rsz);
@@ -486,11 +488,14 @@ int pplan_run(hjm_portfolio_plan p)
 
 int pplan_collect(hjm_portfolio_plan p, hjm_portfolio_results* r)
 {
-    HJM_HIP(hipStreamSynchronize(p->stream), HJM_ERR_LAUNCH);
     const int G = p->nsets, nd = p->ndates, nc = nd + 2;
-    std::vector<double> sums((size_t)G * nc);
-    HJM_HIP(hipMemcpy(sums.data(), p->d_sums, sums.size() * sizeof(double), hipMemcpyDeviceToHost),
+    double* sums = static_cast<double*>(p->ctx.c->host);
+    const double* pf = sums + (size_t)G * nc;
+    HJM_HIP(hipMemcpyAsync(sums, p->d_sums,
+                           sizeof(double) * G * (nc + (r->pfe && p->do_pfe ? nd : 0)),
+                           hipMemcpyDeviceToHost, p->stream),
             HJM_ERR_DEVICE);
+    HJM_HIP(hipStreamSynchronize(p->stream), HJM_ERR_LAUNCH);
     const double P = (double)p->paths, inv = 1.0 / P;
     for (int g = 0; g < G; ++g) {
         const double* sg = &sums[(size_t)g * nc];
@@ -510,9 +515,6 @@ int pplan_collect(hjm_portfolio_plan p, hjm_portfolio_results* r)
     // device rows are [date][set]; the results are [set][date]
     if (r->pfe) {
         if (p->do_pfe) {
-            std::vector<double> pf((size_t)G * nd);
-            HJM_HIP(hipMemcpy(pf.data(), p->d_pfe, sizeof(double) * G * nd, hipMemcpyDeviceToHost),
-                    HJM_ERR_DEVICE);
             for (int e = 0; e < nd; ++e)
                 for (int g = 0; g < G; ++g) r->pfe[(size_t)g * nd + e] = pf[(size_t)e * G + g];
         } else {
@@ -615,9 +617,9 @@ int hjm_portfolio_cva_greeks(const hjm_market* market, const hjm_portfolio* port
         float *gbar = nullptr, *beta = nullptr, *zs = nullptr;
         double *part = nullptr, *sums = nullptr, *bp = nullptr;
         uint16_t* tfrag = nullptr;
-        hipEvent_t e0 = nullptr, e1 = nullptr;
         ~Cleanup()
         {
+            (void)p->ctx.quiesce();
             dev_free(zs);
             dev_free(gbar);
             dev_free(beta);
@@ -625,8 +627,6 @@ int hjm_portfolio_cva_greeks(const hjm_market* market, const hjm_portfolio* port
             dev_free(sums);
             dev_free(bp);
             dev_free(tfrag);
-            if (e0) (void)hipEventDestroy(e0);
-            if (e1) (void)hipEventDestroy(e1);
             hjm_portfolio_plan_destroy(p);
         }
     } c{p};
@@ -655,8 +655,7 @@ int hjm_portfolio_cva_greeks(const hjm_market* market, const hjm_portfolio* port
         HJM_HIP(hipMemcpy(c.tfrag, tf.data(), tf.size() * sizeof(uint16_t), hipMemcpyHostToDevice),
                 HJM_ERR_DEVICE);
     }
-    HJM_HIP(hipEventCreate(&c.e0), HJM_ERR_DEVICE);
-    HJM_HIP(hipEventCreate(&c.e1), HJM_ERR_DEVICE);
+    hipEvent_t e0 = p->ev[5], e1 = p->ev[6];
     // the matrix-core forward keeps its normals for the reverse sweep; without the memory
     // the sweep regenerates them
     if ((p->use_mfma || p->use_mfma64) && config->adjoint_normals == HJM_ADJ_NORMALS_AUTO &&
@@ -664,7 +663,7 @@ int hjm_portfolio_cva_greeks(const hjm_market* market, const hjm_portfolio* port
         c.zs = nullptr;
     hipStream_t st = p->stream;
     HJM_TRY(pplan_enqueue(p, true, c.zs));
-    HJM_HIP(hipEventRecord(c.e0, st), HJM_ERR_DEVICE);
+    HJM_HIP(hipEventRecord(e0, st), HJM_ERR_DEVICE);
     hipError_t err = f64 ? launch_pf_adjoint_seed_f64(p->vp, (const double*)p->d_curves, p->d_logb,
                                                       (const double*)p->d_coef, (const double*)p->d_a,
                                                       p->d_kmax, p->d_w, c.gbar, c.beta, c.bp, st)
@@ -678,7 +677,7 @@ int hjm_portfolio_cva_greeks(const hjm_market* market, const hjm_portfolio* port
     HJM_HIP(launch_pf_adjoint(p->grid, cc, p->d_normals, c.zs, c.gbar, c.beta, c.part, st),
             HJM_ERR_LAUNCH);
     HJM_HIP(launch_column_sum(c.part, nb, kOut, c.sums, st), HJM_ERR_LAUNCH);
-    HJM_HIP(hipEventRecord(c.e1, st), HJM_ERR_DEVICE);
+    HJM_HIP(hipEventRecord(e1, st), HJM_ERR_DEVICE);
     std::vector<double> cvas(p->nsets);
     hjm_portfolio_results r{};
     r.cva = cvas.data();
@@ -722,7 +721,7 @@ int hjm_portfolio_cva_greeks(const hjm_market* market, const hjm_portfolio* port
     if (gr->timings_ms) {
         float fwd = 0.f, adj = 0.f;
         HJM_HIP(hipEventElapsedTime(&fwd, p->ev[0], p->ev[4]), HJM_ERR_DEVICE);
-        HJM_HIP(hipEventElapsedTime(&adj, c.e0, c.e1), HJM_ERR_DEVICE);
+        HJM_HIP(hipEventElapsedTime(&adj, e0, e1), HJM_ERR_DEVICE);
         gr->timings_ms[0] = fwd;
         gr->timings_ms[1] = adj;
         gr->timings_ms[2] = fwd + adj;

@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include "hjm_common.h"
+#include "hjm_pool.h"
 
 #define HJM_TRY(expr)                            \
     do {                                         \
@@ -47,20 +48,37 @@ inline int dev_alloc(T** p, size_t count)
 {
     *p = nullptr;
     if (count == 0) return HJM_OK;
-    if (hipMalloc((void**)p, count * sizeof(T)) != hipSuccess) {
-        *p = nullptr;
-        (void)hipGetLastError();
-        return HJM_ERR_ALLOC;
-    }
+    void* raw = nullptr;
+    if (pool_alloc(&raw, count * sizeof(T)) != hipSuccess) return HJM_ERR_ALLOC;
+    *p = static_cast<T*>(raw);
     return HJM_OK;
 }
 
+// Only once the work that used the block is done (hjm_pool.h).
 template <typename T>
 inline void dev_free(T*& p)
 {
-    if (p) (void)hipFree(p);
+    pool_free((void*)p);
     p = nullptr;
 }
+
+// A plan's stream, events and pinned buffer, returned to the cache when the plan goes. Waits
+// for the stream first, so the plan's blocks may be freed after quiesce() or this.
+struct ContextHolder {
+    PlanContext* c = nullptr;
+    int take(int device, size_t host_bytes)
+    {
+        c = context_acquire(device, host_bytes);
+        return c ? HJM_OK : HJM_ERR_DEVICE;
+    }
+    // false: the stream is in error and nothing that it used may be handed out again
+    bool quiesce() { return !c || hipStreamSynchronize(c->stream) == hipSuccess; }
+    void give()
+    {
+        context_release(c);
+        c = nullptr;
+    }
+};
 
 
 inline int check_market(const hjm_market* m)

@@ -8,7 +8,7 @@
 // curve; 258 products per wave-block at 5 M-tiles against 408 with bf16 throughout, and 1.5
 // instead of 5.5 VALU instructions to split a shock: the 10y path kernel at 131072 paths went
 // from 0.51 to 0.42 ms, its results' error against FP64 unchanged). The split products
-// keeps FP32 accuracy while running on the matrix cores concurrently with the VALU
+// keep FP32 accuracy while running on the matrix cores concurrently with the VALU
 // (FP32 MFMA on gfx950 shares the vector pipeline and gains nothing over it). A wave owns
 // 32 paths = 2 N-tiles of 16 (the portfolio kernel's shape is a launch choice). The
 // accumulator layout of a 16x16 tile -- lane l holds rows

@@ -1,0 +1,231 @@
+// hjm_pool.hip -- the device-memory and plan-context cache of hjm_pool.h (host code).
+#include "hjm_pool.h"
+
+#include <deque>
+#include <mutex>
+#include <new>
+#include <unordered_map>
+#include <vector>
+
+#include "hjm_cva.h"
+
+namespace hjm_host {
+namespace {
+
+struct Block {
+    void* p;
+    size_t bytes;
+    int device;
+};
+
+struct Pool {
+    std::mutex m;
+    std::unordered_map<void*, Block> live;  // handed out
+    std::deque<Block> idle;                 // oldest first, all devices
+    std::vector<PlanContext*> contexts;     // idle
+};
+
+// never destroyed: the HIP runtime may be gone when static destructors run
+Pool& pool()
+{
+    static Pool* p = new Pool();
+    return *p;
+}
+
+// Sizes in steps of 1/8 of their power of two, at least 512 bytes: repeated calls of nearby
+// sizes share blocks, and a block is at most 1/8 larger than asked for.
+size_t rounded(size_t bytes)
+{
+    size_t step = 512;
+    while (step * 16 < bytes) step *= 2;
+    return (bytes + step - 1) / step * step;
+}
+
+void device_free(const Block& b)
+{
+    int prev = -1;
+    (void)hipGetDevice(&prev);
+    if (prev != b.device) (void)hipSetDevice(b.device);
+    (void)hipFree(b.p);
+    if (prev >= 0 && prev != b.device) (void)hipSetDevice(prev);
+}
+
+void context_destroy(PlanContext* c)
+{
+    int prev = -1;
+    (void)hipGetDevice(&prev);
+    if (prev != c->device) (void)hipSetDevice(c->device);
+    if (c->host) (void)hipHostFree(c->host);
+    for (auto& e : c->ev)
+        if (e) (void)hipEventDestroy(e);
+    if (c->stream) (void)hipStreamDestroy(c->stream);
+    if (prev >= 0 && prev != c->device) (void)hipSetDevice(prev);
+    delete c;
+}
+
+}  // namespace
+
+hipError_t pool_alloc(void** out, size_t bytes)
+{
+    *out = nullptr;
+    int device = -1;
+    hipError_t err = hipGetDevice(&device);
+    if (err != hipSuccess) return err;
+    const size_t want = rounded(bytes);
+    Pool& q = pool();
+    try {
+        {
+            std::lock_guard<std::mutex> lock(q.m);
+            auto best = q.idle.end();
+            for (auto it = q.idle.begin(); it != q.idle.end(); ++it)
+                if (it->device == device && it->bytes >= want && it->bytes <= want + want / 8 &&
+                    (best == q.idle.end() || it->bytes < best->bytes))
+                    best = it;
+            if (best != q.idle.end()) {
+                const Block b = *best;
+                q.live.emplace(b.p, b);
+                q.idle.erase(best);
+                *out = b.p;
+                return hipSuccess;
+            }
+        }
+        void* p = nullptr;
+        err = hipMalloc(&p, want);
+        if (err != hipSuccess) {
+            (void)hipGetLastError();
+            pool_release_all();
+            err = hipMalloc(&p, want);
+            if (err != hipSuccess) {
+                (void)hipGetLastError();
+                return err;
+            }
+        }
+        try {
+            std::lock_guard<std::mutex> lock(q.m);
+            q.live.emplace(p, Block{p, want, device});
+        } catch (...) {
+            (void)hipFree(p);
+            return hipErrorOutOfMemory;
+        }
+        *out = p;
+        return hipSuccess;
+    } catch (...) {
+        return hipErrorOutOfMemory;
+    }
+}
+
+void pool_free(void* p)
+{
+    if (!p) return;
+    Pool& q = pool();
+    std::vector<Block> drop;
+    Block b{p, 0, 0};
+    try {
+        std::lock_guard<std::mutex> lock(q.m);
+        const auto it = q.live.find(p);
+        if (it != q.live.end()) {
+            b = it->second;
+            q.live.erase(it);
+            if (b.bytes <= kPoolBytes) {
+                size_t held = b.bytes;
+                for (const Block& x : q.idle) held += x.device == b.device ? x.bytes : 0;
+                for (auto x = q.idle.begin(); held > kPoolBytes && x != q.idle.end();) {
+                    if (x->device != b.device) {
+                        ++x;
+                        continue;
+                    }
+                    drop.push_back(*x);
+                    held -= x->bytes;
+                    x = q.idle.erase(x);
+                }
+                q.idle.push_back(b);
+                b.p = nullptr;
+            }
+        }
+    } catch (...) {
+        // bookkeeping memory ran out: the block itself goes back to the device below
+    }
+    if (b.p) {
+        if (b.bytes) device_free(b);
+        else (void)hipFree(p);
+    }
+    for (const Block& x : drop) device_free(x);
+}
+
+void pool_release_all()
+{
+    Pool& q = pool();
+    std::deque<Block> idle;
+    std::vector<PlanContext*> contexts;
+    {
+        std::lock_guard<std::mutex> lock(q.m);
+        idle.swap(q.idle);
+        contexts.swap(q.contexts);
+    }
+    for (const Block& b : idle) device_free(b);
+    for (PlanContext* c : contexts) context_destroy(c);
+}
+
+PlanContext* context_acquire(int device, size_t host_bytes)
+{
+    Pool& q = pool();
+    PlanContext* c = nullptr;
+    {
+        std::lock_guard<std::mutex> lock(q.m);
+        for (size_t i = q.contexts.size(); i-- > 0;)
+            if (q.contexts[i]->device == device) {
+                c = q.contexts[i];
+                q.contexts.erase(q.contexts.begin() + (std::ptrdiff_t)i);
+                break;
+            }
+    }
+    if (!c) {
+        c = new (std::nothrow) PlanContext();
+        if (!c) return nullptr;
+        c->device = device;
+        bool ok = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) == hipSuccess;
+        for (auto& e : c->ev) ok = ok && hipEventCreate(&e) == hipSuccess;
+        if (!ok) {
+            (void)hipGetLastError();
+            context_destroy(c);
+            return nullptr;
+        }
+    }
+    if (c->host_bytes < host_bytes) {
+        if (c->host) (void)hipHostFree(c->host);
+        c->host = nullptr;
+        c->host_bytes = 0;
+        if (hipHostMalloc(&c->host, host_bytes, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            c->host = nullptr;
+            context_destroy(c);
+            return nullptr;
+        }
+        c->host_bytes = host_bytes;
+    }
+    return c;
+}
+
+void context_release(PlanContext* c)
+{
+    if (!c) return;
+    const bool idle = hipStreamSynchronize(c->stream) == hipSuccess;
+    if (idle) {
+        Pool& q = pool();
+        try {
+            std::lock_guard<std::mutex> lock(q.m);
+            int n = 0;
+            for (const PlanContext* x : q.contexts) n += x->device == c->device ? 1 : 0;
+            if (n < kPoolContexts) {
+                q.contexts.push_back(c);
+                return;
+            }
+        } catch (...) {
+        }
+    }
+    context_destroy(c);
+}
+
+}  // namespace hjm_host
+
+extern "C" void hjm_release_cached_memory(void) { hjm_host::pool_release_all(); }

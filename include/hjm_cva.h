@@ -118,6 +118,12 @@ typedef struct {
 const char* hjm_status_string(int status);
 int hjm_device_count(int* count);
 
+/* The library keeps up to 8 GB per device of the memory that destroyed plans and finished
+ * calls used, with a few streams, for those that follow (mapping fresh device memory costs
+ * more than most runs). This returns all of it to the device; plans in use are not touched.
+ * A failed allocation does the same by itself before it is reported. */
+void hjm_release_cached_memory(void);
+
 /* CVA weights w_j = (1-R) * trapezoid share of the default probability of
  * [t_{j-1}, t_j], S(t) = exp(-h t), t_j = j * date_dt, j = 0..ndates-1. */
 int hjm_cva_weights(int ndates, double date_dt, double hazard_rate, double recovery,
