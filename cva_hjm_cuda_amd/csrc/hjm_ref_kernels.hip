@@ -1,7 +1,8 @@
 // hjm_ref_kernels.hip -- reference-semantics HJM path generation and exposure, gfx950.
 //
-// Layout: one Monte Carlo path per lane (wave64, 256-lane workgroups). The 51-point
-// forward curve and its 51 discount integrals live in VGPRs for the whole horizon; the
+// Layout: FP64 with in-kernel normals, 4 to 32 lanes per path (ref_paths_lanes_kernel); host
+// normals and FP32, one Monte Carlo path per lane (wave64, 256-lane workgroups). There the
+// 51-point forward curve and its 51 discount integrals live in VGPRs for the whole horizon; the
 // tenor constants (drift*dt, 3 loadings) come from the kernarg segment through scalar
 // loads, identical for every lane. Normals are generated in-kernel (counter Philox) or
 // read from the caller's [path][step][3] array. HBM is touched only at exposure dates:
@@ -172,6 +173,146 @@ __global__ __launch_bounds__(kBlock, 2) void ref_paths_kernel(const RefStepConst
     }
 }
 
+// ---- FP64 paths, L lanes per path ---------------------------------------------------------
+// The same steps in the same operations and order as ref_paths_kernel<double> (bit-identical
+// numeraires), with a path's 51 tenors spread over L lanes (n = ceil(51 / L) consecutive
+// tenors each): the tenor constants then live in VGPRs instead of 408 dwords of scalar loads
+// per step, the generator's calls are shared by the path's lanes, and the serial chain of a
+// path shrinks by almost L. A workgroup is one wave. Bound by FP64 issue: 131072 paths x 10y
+// in 1.40 ms at L = 4 (85 instructions a step for 16 paths, 49.9 TFLOP/s of the 561 flops per
+// path-step, 0.63 of the 78.6 peak; one path per lane took 1.84 ms, waiting on its scalar
+// loads); a few waves are bound by the chain of a step, 24 FP64 instructions at L = 16.
+template <int L>
+struct RefLanes {
+    static constexpr int n = (kTenors + L - 1) / L;       // tenors per lane
+    // lane l holds tenors n l - pad + u, u = 0 .. n-1; pad puts tenor 50 past slot 0, so that
+    // its neighbour 49 is in the same lane
+    static constexpr int pad = (kTenors - 1) % n == 0 ? 1 : 0;
+    static constexpr int last = (kTenors - 1 + pad) / n;  // lane and slot of tenor 50
+    static constexpr int slot = (kTenors - 1 + pad) % n;
+    static constexpr int paths = kWave / L;               // per wave
+    static constexpr int chunk = 32;                      // steps staged in LDS at a time
+    static constexpr int cls = 3 * chunk / 4;             // shocks per class and chunk
+    static constexpr int ld = 4 * cls + 4;                // doubles per path (bank spread)
+    static_assert(last < L && slot >= 1, "tenor 49 shares the lane of tenor 50");
+};
+
+// lane i receives lane i + 1's value: within rows of 16 (L <= 16) or across the wave
+template <int L>
+__device__ __forceinline__ double from_next_lane(double v)
+{
+    constexpr int ctrl = L <= 16 ? 0x101 : 0x130;   // row_shl:1, wave_shl:1
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, ctrl, 0xf, 0xf, true);
+    const uint32_t hi =
+        (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), ctrl, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+template <int L>
+__global__ __launch_bounds__(kWave) void ref_paths_lanes_kernel(const RefStepConsts<double> k,
+                                                             const RefGrid g,
+                                                             double* __restrict__ num_x,
+                                                             double* __restrict__ num_y)
+{
+    using C = RefLanes<L>;
+    constexpr int n = C::n;
+    __shared__ double shocks[C::paths * C::ld];
+    const int lane = threadIdx.x, sub = lane % L;
+    const int64_t P = g.paths;
+    const int64_t i = (int64_t)blockIdx.x * C::paths + lane / L;
+    const bool live = i < P;
+    const uint32_t pid = (uint32_t)(g.path0 + (live ? i : 0));
+    double* col = shocks + (lane / L) * C::ld;
+    const bool is_last = sub == C::last;
+    const double sqdt = k.sqrt_dt;
+    // slots without a tenor start at 0 and take no constants; no tenor reads them
+    double f[n], A[n], m[n], v0[n], v1[n], v2[n];
+#pragma unroll
+    for (int u = 0; u < n; ++u) {
+        const int j = sub * n + u - C::pad;
+        const bool on = j >= 0 && j < kTenors;
+        const int jc = on ? j : 0;
+        f[u] = on ? k.spot[jc] : 0.0;
+        A[u] = on ? g.a0[jc] : 0.0;
+        m[u] = on ? k.ddt[jc] : 0.0;
+        v0[u] = on ? k.v0[jc] : 0.0;
+        v1[u] = on ? k.v1[jc] : 0.0;
+        v2[u] = on ? k.v2[jc] : 0.0;
+    }
+    double cv = k.c, omc = k.omc;
+    // the slot of tenor 50 (in the last lane the backward difference, elsewhere as any other)
+    double cs = is_last ? -k.c : k.c, os = is_last ? k.opc : k.omc;
+    asm volatile("" : "+v"(cv), "+v"(omc), "+v"(cs), "+v"(os));
+    if (live && sub == 0) {
+        num_x[P + i] = k.spot[1];
+        num_y[P + i] = exp(-g.a0[1] * g.dt);
+    }
+    // one Euler step with the shocks q[0..2] (times sqrt(dt))
+    auto step = [&](const double* q) {
+        const double y0 = q[0], y1 = q[1], y2 = q[2];
+        const double fn = from_next_lane<L>(f[0]);
+        constexpr int S = C::slot;
+        const double fs = is_last ? f[S - 1] : (S + 1 < n ? f[S + 1 < n ? S + 1 : 0] : fn);
+        constexpr int G = 4;
+#pragma unroll
+        for (int u0 = 0; u0 < n; u0 += G) {
+            double t[G];
+#pragma unroll
+            for (int u = u0; u < u0 + G && u < n; ++u)
+                op_fma_vvv(t[u - u0], u == S ? cs : cv, u == S ? fs : (u + 1 < n ? f[u + 1 < n ? u + 1 : 0] : fn),
+                           m[u]);
+#pragma unroll
+            for (int u = u0; u < u0 + G && u < n; ++u) op_fmac_vv(t[u - u0], v0[u], y0);
+#pragma unroll
+            for (int u = u0; u < u0 + G && u < n; ++u) op_fmac_vv(t[u - u0], v1[u], y1);
+#pragma unroll
+            for (int u = u0; u < u0 + G && u < n; ++u) op_fmac_vv(t[u - u0], v2[u], y2);
+#pragma unroll
+            for (int u = u0; u < u0 + G && u < n; ++u) op_fma_inplace(f[u], u == S ? os : omc, t[u - u0]);
+#pragma unroll
+            for (int u = u0; u < u0 + G && u < n; ++u) op_add_inplace(A[u], f[u]);
+        }
+    };
+    for (int b = 1; b < g.ndates; ++b) {
+        for (int s0 = 0; s0 < g.stride; s0 += C::chunk) {
+            const int steps = min(C::chunk, g.stride - s0);
+            // steps [s0, s0 + 32) are quads 8 k .. 8 k + 7 of every class: calls 6 k .. 6 k + 5
+            const int calls = (3 * ((steps + 3) / 4) + 3) / 4, c0 = 3 * s0 / 16;
+            __syncthreads();   // the chunk before is read
+            for (int it = sub; it < 4 * calls; it += L) {
+                const int cls = it & 3, c = it >> 2;
+                float z[4];
+                stream_call(g.seed_lo, g.seed_hi, pid, (uint32_t)b, (uint32_t)cls, (uint32_t)(c0 + c), z);
+                double* o = col + cls * C::cls + 4 * c;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = sqdt * (double)z[e];
+            }
+            __syncthreads();
+            // step 4 q + g: class g, shocks 3 q .. 3 q + 2 of it
+            const double* q = col;
+            int st = 0;
+            for (; st + 4 <= steps; st += 4, q += 3) {
+#pragma unroll
+                for (int cls = 0; cls < 4; ++cls) step(q + cls * C::cls);
+            }
+            for (int cls = 0; st < steps; ++st, ++cls) step(q + cls * C::cls);
+        }
+        const int at = b + 1 + C::pad, owner = at / n, slot = at % n;
+        double x = f[0], a = A[0];
+#pragma unroll
+        for (int u = 1; u < n; ++u)
+            if (u == slot) {
+                x = f[u];
+                a = A[u];
+            }
+        if (live && sub == owner) {
+            num_x[(int64_t)(b + 1) * P + i] = x;
+            num_y[(int64_t)(b + 1) * P + i] = exp(-a * g.dt);
+        }
+    }
+}
+
 // Exposure of simulation_cpu.h:269-296 (simulation_gpu.cu:803-858) for one path per
 // lane: CF_i = DF_i N acc_i (m (e^{x_i/m} - 1) - K), E_t = max(sum_{i>t} CF_i, 0),
 // plus the per-path CVA sample sum_t w_t E_t. Writes E [date][path] when asked and one
@@ -301,28 +442,45 @@ __global__ __launch_bounds__(kBlock) void normals_kernel(uint32_t seed_lo, uint3
 }
 
 // ---- launchers -------------------------------------------------------------------
-template <typename Real, bool kKahan>
-static hipError_t launch_paths(const RefStepConsts<Real>& k, const RefGrid& g,
-                               const double* normals, double* nx, double* ny, hipStream_t st)
+template <int L>
+static hipError_t launch_paths_lanes(const RefStepConsts<double>& k, const RefGrid& g, double* nx,
+                                     double* ny, hipStream_t st)
 {
-    const dim3 grid((unsigned)((g.paths + kBlock - 1) / kBlock));
-    if (normals)
-        ref_paths_kernel<Real, kKahan, true><<<grid, kBlock, 0, st>>>(k, g, normals, nx, ny);
-    else
-        ref_paths_kernel<Real, kKahan, false><<<grid, kBlock, 0, st>>>(k, g, normals, nx, ny);
+    constexpr int paths = RefLanes<L>::paths;
+    ref_paths_lanes_kernel<L><<<(unsigned)((g.paths + paths - 1) / paths), kWave, 0, st>>>(k, g, nx, ny);
     return hipGetLastError();
 }
 
 hipError_t launch_ref_paths_f64(const RefStepConsts<double>& k, const RefGrid& g,
                                 const double* normals, double* nx, double* ny, hipStream_t st)
 {
-    return launch_paths<double, false>(k, g, normals, nx, ny, st);
+    // In-kernel normals: L lanes per path. Fewer paths take more lanes each until the chip's
+    // 1024 SIMDs hold a wave: L = 32 up to 2048 paths, 16 up to 4096, 8 up to 24576 (three
+    // waves per SIMD), and 4 beyond, which wastes the fewest slots (52 for 51 tenors) but
+    // holds 246 VGPRs. Path kernel in us at L = 32 / 16 / 8 / 4, one path per lane in brackets:
+    //   1000 x 5y 38 / 49 / 63 / 101 [716]; 4096 x 10y 105 / 100 / 134 / 204 [1495];
+    //   5000 x 25y 344 / 365 / 333 / 520 [3958]; 20000 x 10y 404 / 354 / 335 / 383 [1513];
+    //   30000 x 10y 574 / 510 / 421 / 383 [1517]; 131072 x 10y 2207 / 1820 / 1538 / 1404 [1841].
+    if (!normals) {
+        if (g.paths <= 2048) return launch_paths_lanes<32>(k, g, nx, ny, st);
+        if (g.paths <= 4096) return launch_paths_lanes<16>(k, g, nx, ny, st);
+        if (g.paths <= 24576) return launch_paths_lanes<8>(k, g, nx, ny, st);
+        return launch_paths_lanes<4>(k, g, nx, ny, st);
+    }
+    ref_paths_kernel<double, false, true><<<(unsigned)((g.paths + kBlock - 1) / kBlock), kBlock, 0, st>>>(
+        k, g, normals, nx, ny);
+    return hipGetLastError();
 }
 
 hipError_t launch_ref_paths_f32k(const RefStepConsts<float>& k, const RefGrid& g,
                                  const double* normals, double* nx, double* ny, hipStream_t st)
 {
-    return launch_paths<float, true>(k, g, normals, nx, ny, st);
+    const dim3 grid((unsigned)((g.paths + kBlock - 1) / kBlock));
+    if (normals)
+        ref_paths_kernel<float, true, true><<<grid, kBlock, 0, st>>>(k, g, normals, nx, ny);
+    else
+        ref_paths_kernel<float, true, false><<<grid, kBlock, 0, st>>>(k, g, normals, nx, ny);
+    return hipGetLastError();
 }
 
 hipError_t launch_ref_exposure(const ExposureParams& e, const double* nx, const double* ny,

@@ -45,6 +45,16 @@ __device__ __forceinline__ void op_add_inplace(float& a, float x)
     asm("v_add_f32 %0, %0, %1" : "+v"(a) : "v"(x));
 }
 
+// the same with every operand in VGPRs (FP64 paths with several lanes per path)
+__device__ __forceinline__ void op_fma_vvv(double& d, double a, double b, double c)
+{
+    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
+}
+__device__ __forceinline__ void op_fmac_vv(double& d, double a, double b)
+{
+    asm("v_fmac_f64 %0, %1, %2" : "+v"(d) : "v"(a), "v"(b));
+}
+
 // ---- adjoint sweep forms ------------------------------------------------------------
 // d = a * b + c with all operands in VGPRs
 __device__ __forceinline__ void op_fma_vvv(float& d, float a, float b, float c)
