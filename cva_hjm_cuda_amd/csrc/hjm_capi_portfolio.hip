@@ -49,8 +49,10 @@ struct hjm_pplan_s {
     double* d_pfe = nullptr;  // [date][set], after the sums
     char* d_selws = nullptr;  // bracket-selection workspace (PFE)
     uint32_t* d_loparts = nullptr;  // counts below the bracket per row and statistics workgroup
-    void* d_coef = nullptr;
-    void* d_a = nullptr;
+    double* d_coef = nullptr;
+    double* d_a = nullptr;
+    int* d_book_ints = nullptr;      // the swap list: set offsets, periods
+    double* d_book_reals = nullptr;  // signed notionals, coupons
     int* d_kmax = nullptr;
     double* d_w = nullptr;
     uint16_t* d_vfrag = nullptr;  // FP32: bf16 parts of -gamma (matrix-core valuation)
@@ -78,6 +80,8 @@ void pplan_release(hjm_portfolio_plan p)
     dev_free(p->d_selws);
     dev_free(p->d_loparts);
     dev_free(p->d_coef);
+    dev_free(p->d_book_ints);
+    dev_free(p->d_book_reals);
     dev_free(p->d_vfrag);
     dev_free(p->d_apad);
     dev_free(p->d_tilek);
@@ -115,32 +119,6 @@ int check_portfolio(const hjm_portfolio* pf, int* ndates)
     return HJM_OK;
 }
 
-// V_g(t_e) = a_ge - sum_k gamma_gek P_k with, for every live swap (k_s = n_s - e > 0):
-// a += sN, gamma_{k_s} += sN (the -sN P_{n} term), gamma_j += sN K dtau for j <= k_s.
-void build_tables(const hjm_portfolio* pf, int ndates, std::vector<double>& coef,
-                  std::vector<double>& a, std::vector<int>& kmax)
-{
-    const int G = pf->nsets;
-    coef.assign((size_t)ndates * G * kMaxPeriods, 0.0);
-    a.assign((size_t)ndates * G, 0.0);
-    kmax.assign((size_t)ndates * G, 0);
-    for (int e = 0; e < ndates; ++e) {
-        for (int s = 0; s < pf->nswaps; ++s) {
-            const int k = pf->periods[s] - e;
-            if (k <= 0) continue;
-            const int g = pf->netting_set[s];
-            const size_t row = (size_t)e * G + g;
-            const double sn = pf->sign_notional[s];
-            a[row] += sn;
-            double* gam = &coef[row * kMaxPeriods];
-            gam[k - 1] += sn;
-            const double fx = sn * pf->fixed_rate[s] * pf->dtau;
-            for (int j = 1; j <= k; ++j) gam[j - 1] += fx;
-            kmax[row] = std::max(kmax[row], k);
-        }
-    }
-}
-
 int check_tuning(const hjm_tuning& t)
 {
     if (t.block_size != 64 && t.block_size != 128 && t.block_size != 256) return HJM_ERR_ARG;
@@ -168,8 +146,9 @@ void pplan_apply_tuning(hjm_portfolio_plan p, const hjm_tuning& t)
     p->value_shape = MfmaShape{t.value_tiles, t.value_waves, t.value_stage, 0};
 }
 
+// greeks: a plan of the Greeks call, whose seeds value the sets (no exposures, no statistics)
 int pplan_init(hjm_portfolio_plan p, const hjm_market* market, const hjm_portfolio* pf,
-               const hjm_config* cfg, const hjm_tuning* tuning)
+               const hjm_config* cfg, const hjm_tuning* tuning, bool greeks = false)
 {
     HJM_TRY(check_market(market));
     if (!cfg) return HJM_ERR_NULL;
@@ -225,17 +204,32 @@ int pplan_init(hjm_portfolio_plan p, const hjm_market* market, const hjm_portfol
     p->w.assign((size_t)pf->nsets * nd, 0.0);
     for (int s = 0; s < pf->nsets; ++s)
         cva_weights(nd, pf->dtau, pf->hazard_rate[s], pf->recovery, &p->w[(size_t)s * nd]);
-    std::vector<double> coef, a;
-    std::vector<int> kmax;
-    build_tables(pf, nd, coef, a, kmax);
+    // the swaps grouped by set, in the caller's order within a set
+    const int G = pf->nsets, N = pf->nswaps;
+    std::vector<int> order((size_t)N), ints((size_t)G + 1 + N, 0);
+    std::vector<double> reals(2 * (size_t)N);
+    int* first = ints.data();
+    for (int s = 0; s < N; ++s) ++first[pf->netting_set[s] + 1];
+    for (int g = 0; g < G; ++g) first[g + 1] += first[g];
+    {
+        std::vector<int> at(first, first + G);
+        for (int s = 0; s < N; ++s) order[(size_t)at[pf->netting_set[s]]++] = s;
+    }
+    for (int i = 0; i < N; ++i) {
+        const int s = order[(size_t)i];
+        first[G + 1 + i] = pf->periods[s];
+        reals[(size_t)i] = pf->sign_notional[s];
+        reals[(size_t)N + i] = pf->sign_notional[s] * pf->fixed_rate[s] * pf->dtau;
+    }
 
     DeviceGuard guard;
     HJM_TRY(guard.set(cfg->device));
     HJM_HIP(hipDeviceGetAttribute(&p->cus, hipDeviceAttributeMultiprocessorCount, cfg->device),
             HJM_ERR_DEVICE);
     pplan_apply_tuning(p, p->tuning);
-    // pinned: the column sums and the PFE rows of one run
-    HJM_TRY(p->ctx.take(cfg->device, sizeof(double) * (size_t)pf->nsets * (2 * nd + 2)));
+    // pinned: the column sums and the PFE rows of one run, or a Greeks call's sums
+    const size_t pinned = std::max<size_t>((size_t)pf->nsets * (2 * nd + 2), 5 * kTenors + 2 * (size_t)nd);
+    HJM_TRY(p->ctx.take(cfg->device, sizeof(double) * pinned));
     p->stream = p->ctx.c->stream;
     p->ev = p->ctx.c->ev;
     const size_t rsz = (p->precision == HJM_FP64) ? sizeof(double) : sizeof(float);
@@ -246,65 +240,54 @@ int pplan_init(hjm_portfolio_plan p, const hjm_market* market, const hjm_portfol
     HJM_TRY(dev_alloc(&raw, (size_t)nd * kTenors * P * rsz));
     p->d_curves = raw;
     HJM_TRY(dev_alloc(&p->d_logb, (size_t)nd * P));
-    raw = nullptr;
-    HJM_TRY(dev_alloc(&raw, (size_t)pf->nsets * nd * P * rsz));
-    p->d_ex = raw;
-    HJM_TRY(dev_alloc(&p->d_partials, (size_t)pf->nsets * nb * (nd + 2)));
-    HJM_TRY(dev_alloc(&p->d_sums, (size_t)pf->nsets * (2 * nd + 2)));
-    p->d_pfe = p->d_sums + (size_t)pf->nsets * (nd + 2);
+    hipStream_t st = p->stream;
+    const size_t rows = (size_t)G * nd;
+    if (!greeks) {
+        raw = nullptr;
+        HJM_TRY(dev_alloc(&raw, rows * P * rsz));
+        p->d_ex = raw;
+        HJM_TRY(dev_alloc(&p->d_partials, (size_t)G * nb * (nd + 2)));
+        HJM_TRY(dev_alloc(&p->d_sums, (size_t)G * (2 * nd + 2)));
+        p->d_pfe = p->d_sums + (size_t)G * (nd + 2);
+    }
     if (p->do_pfe) {
-        const size_t wsb = bracket_workspace_bytes(pf->nsets * nd, bracket_plan(cfg->paths, p->pfe_rank, (int)rsz),
+        const size_t wsb = bracket_workspace_bytes((int)rows, bracket_plan(cfg->paths, p->pfe_rank, (int)rsz),
                                                    (int)rsz);
         if (wsb) {
             HJM_TRY(dev_alloc(&p->d_selws, wsb));
             if (rsz == sizeof(float))
-                HJM_TRY(dev_alloc(&p->d_loparts, (size_t)pf->nsets * nd * pf_stats_blocks(cfg->paths)));
+                HJM_TRY(dev_alloc(&p->d_loparts, rows * pf_stats_blocks(cfg->paths)));
         }
     }
-    HJM_TRY(dev_alloc(&p->d_kmax, kmax.size()));
     HJM_TRY(dev_alloc(&p->d_w, p->w.size()));
-    HJM_HIP(hipMemcpy(p->d_kmax, kmax.data(), kmax.size() * sizeof(int), hipMemcpyHostToDevice),
+    HJM_HIP(hipMemcpyAsync(p->d_w, p->w.data(), p->w.size() * sizeof(double), hipMemcpyHostToDevice, st),
             HJM_ERR_DEVICE);
+    // coefficient tables from the swap list
+    HJM_TRY(dev_alloc(&p->d_book_ints, ints.size()));
+    HJM_TRY(dev_alloc(&p->d_book_reals, reals.size()));
+    HJM_HIP(hipMemcpyAsync(p->d_book_ints, ints.data(), ints.size() * sizeof(int), hipMemcpyHostToDevice, st),
+            HJM_ERR_DEVICE);
+    HJM_HIP(hipMemcpyAsync(p->d_book_reals, reals.data(), reals.size() * sizeof(double),
+                           hipMemcpyHostToDevice, st),
+            HJM_ERR_DEVICE);
+    HJM_TRY(dev_alloc(&p->d_coef, rows * kMaxPeriods));
+    HJM_TRY(dev_alloc(&p->d_a, rows));
+    HJM_TRY(dev_alloc(&p->d_kmax, rows));
     p->vp.kmax = p->d_kmax;
+    const BookSwaps book{p->d_book_ints, p->d_book_ints + G + 1, p->d_book_reals, p->d_book_reals + N};
+    HJM_HIP(launch_book_tables(book, G, nd, p->d_coef, p->d_a, p->d_kmax, st), HJM_ERR_LAUNCH);
     // rows of matured sets are never written (their exposures are 0) and never read by the
     // statistics pass; they hold zeros for the PFE selection and the per-path copy
-    HJM_HIP(hipMemset(p->d_ex, 0, (size_t)pf->nsets * nd * P * rsz), HJM_ERR_DEVICE);
-    HJM_HIP(hipMemcpy(p->d_w, p->w.data(), p->w.size() * sizeof(double), hipMemcpyHostToDevice),
-            HJM_ERR_DEVICE);
-    if (p->precision == HJM_FP64) {
-        double *c = nullptr, *aa = nullptr;
-        HJM_TRY(dev_alloc(&c, coef.size()));
-        p->d_coef = c;
-        HJM_TRY(dev_alloc(&aa, a.size()));
-        p->d_a = aa;
-        HJM_HIP(hipMemcpy(c, coef.data(), coef.size() * sizeof(double), hipMemcpyHostToDevice),
-                HJM_ERR_DEVICE);
-        HJM_HIP(hipMemcpy(aa, a.data(), a.size() * sizeof(double), hipMemcpyHostToDevice),
-                HJM_ERR_DEVICE);
-    } else {
-        std::vector<float> cf(coef.begin(), coef.end()), af(a.begin(), a.end());
-        float *c = nullptr, *aa = nullptr;
-        HJM_TRY(dev_alloc(&c, cf.size()));
-        p->d_coef = c;
-        HJM_TRY(dev_alloc(&aa, af.size()));
-        p->d_a = aa;
-        HJM_HIP(hipMemcpy(c, cf.data(), cf.size() * sizeof(float), hipMemcpyHostToDevice),
-                HJM_ERR_DEVICE);
-        HJM_HIP(hipMemcpy(aa, af.data(), af.size() * sizeof(float), hipMemcpyHostToDevice),
-                HJM_ERR_DEVICE);
-        std::vector<uint16_t> vf;
-        std::vector<float> ap;
-        std::vector<int> tk;
-        build_value_fragments(coef, a, kmax, nd, pf->nsets, kMaxPeriods, vf, ap, tk);
-        HJM_TRY(dev_alloc(&p->d_vfrag, vf.size()));
-        HJM_TRY(dev_alloc(&p->d_apad, ap.size()));
-        HJM_TRY(dev_alloc(&p->d_tilek, tk.size()));
-        HJM_HIP(hipMemcpy(p->d_vfrag, vf.data(), vf.size() * sizeof(uint16_t), hipMemcpyHostToDevice),
-                HJM_ERR_DEVICE);
-        HJM_HIP(hipMemcpy(p->d_apad, ap.data(), ap.size() * sizeof(float), hipMemcpyHostToDevice),
-                HJM_ERR_DEVICE);
-        HJM_HIP(hipMemcpy(p->d_tilek, tk.data(), tk.size() * sizeof(int), hipMemcpyHostToDevice),
-                HJM_ERR_DEVICE);
+    if (!greeks)
+        HJM_HIP(launch_clear_matured(p->d_kmax, (int)rows, (int64_t)P, p->d_ex, (int)rsz, st), HJM_ERR_LAUNCH);
+    if (p->precision != HJM_FP64) {
+        const size_t mt = (size_t)value_mtiles(G);
+        HJM_TRY(dev_alloc(&p->d_vfrag, nd * mt * kValueFragsPerTile * kWave * 8));
+        HJM_TRY(dev_alloc(&p->d_apad, nd * mt * 16));
+        HJM_TRY(dev_alloc(&p->d_tilek, nd * mt));
+        HJM_HIP(launch_value_fragments(p->d_coef, p->d_a, p->d_kmax, G, nd, p->d_vfrag, p->d_apad, p->d_tilek,
+                                       st),
+                HJM_ERR_LAUNCH);
     }
     if (cfg->rng == HJM_RNG_HOST) {
         const size_t n = P * (size_t)S * 3;
@@ -345,6 +328,8 @@ int pplan_init(hjm_portfolio_plan p, const hjm_market* market, const hjm_portfol
             mg.spot64[j] = market->spot_rates[j];
         }
     }
+    // the host copies above go with this call
+    HJM_HIP(hipStreamSynchronize(st), HJM_ERR_DEVICE);
     return HJM_OK;
 }
 
@@ -386,6 +371,7 @@ int pplan_enqueue(hjm_portfolio_plan p, bool events = true, float* zs = nullptr,
                                   p->tuning.block_size, p->grid_blocks, st);
     HJM_HIP(err, HJM_ERR_LAUNCH);
     HJM_HIP(mark(1), HJM_ERR_DEVICE);
+    if (!p->d_ex) return HJM_OK;   // a plan of the Greeks call
     if (pplan_fused(p, keep_exposures)) {
         const float* curves = (const float*)p->d_curves;
         float* ex = (float*)p->d_ex;
@@ -423,7 +409,7 @@ int pplan_enqueue(hjm_portfolio_plan p, bool events = true, float* zs = nullptr,
         return HJM_OK;
     }
     err = f64 ? launch_pf_value_f64(p->vp, (const double*)p->d_curves, p->d_logb,
-                                    (const double*)p->d_coef, (const double*)p->d_a, p->d_kmax,
+                                    p->d_coef, p->d_a, p->d_kmax,
                                     (double*)p->d_ex, st)
               : launch_pf_value_mfma(p->vp, (const float*)p->d_curves, p->d_logb, p->d_vfrag,
                                      p->d_apad, p->d_tilek, (float*)p->d_ex, p->value_shape, st);
@@ -556,6 +542,22 @@ int pplan_collect(hjm_portfolio_plan p, hjm_portfolio_results* r)
     return HJM_OK;
 }
 
+int pplan_create(hjm_portfolio_plan* out, const hjm_market* market, const hjm_portfolio* portfolio,
+                 const hjm_config* config, const hjm_tuning* tuning, bool greeks)
+{
+    if (!out) return HJM_ERR_NULL;
+    *out = nullptr;
+    hjm_portfolio_plan p = new (std::nothrow) hjm_pplan_s();
+    if (!p) return HJM_ERR_ALLOC;
+    const int rc = pplan_init(p, market, portfolio, config, tuning, greeks);
+    if (rc != HJM_OK) {
+        pplan_release(p);
+        return rc;
+    }
+    *out = p;
+    return HJM_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -564,17 +566,7 @@ int hjm_portfolio_plan_create(hjm_portfolio_plan* out, const hjm_market* market,
                               const hjm_portfolio* portfolio, const hjm_config* config,
                               const hjm_tuning* tuning)
 {
-    if (!out) return HJM_ERR_NULL;
-    *out = nullptr;
-    hjm_portfolio_plan p = new (std::nothrow) hjm_pplan_s();
-    if (!p) return HJM_ERR_ALLOC;
-    const int rc = pplan_init(p, market, portfolio, config, tuning);
-    if (rc != HJM_OK) {
-        pplan_release(p);
-        return rc;
-    }
-    *out = p;
-    return HJM_OK;
+    return pplan_create(out, market, portfolio, config, tuning, false);
 }
 
 int hjm_portfolio_plan_execute(hjm_portfolio_plan plan, hjm_portfolio_results* results)
@@ -610,7 +602,7 @@ int hjm_portfolio_cva_greeks(const hjm_market* market, const hjm_portfolio* port
     hjm_config cfg = *config;
     cfg.pfe_quantile = 0.0;
     hjm_portfolio_plan p = nullptr;
-    HJM_TRY(hjm_portfolio_plan_create(&p, market, portfolio, &cfg, tuning));
+    HJM_TRY(pplan_create(&p, market, portfolio, &cfg, tuning, true));
     constexpr int kOut = 5 * kTenors;  // g0, g1, g2, sum of lambda_e, d spot
     struct Cleanup {
         hjm_portfolio_plan p;
@@ -638,22 +630,20 @@ int hjm_portfolio_cva_greeks(const hjm_market* market, const hjm_portfolio* port
     HJM_TRY(dev_alloc(&c.gbar, (size_t)nd * kTenors * P));
     HJM_TRY(dev_alloc(&c.beta, (size_t)nd * P));
     HJM_TRY(dev_alloc(&c.part, (size_t)nb * kOut));
-    HJM_TRY(dev_alloc(&c.sums, (size_t)kOut + kMaxDates));  // then the per-date sums of beta
+    // the sweep's sums, then per date the sums of beta and of the CVA's terms
+    const size_t nsum = (size_t)kOut + 2 * nd;
+    HJM_TRY(dev_alloc(&c.sums, nsum));
     const bool f64 = p->precision == HJM_FP64;
-    // rows of the seeds' beta partials: blocks of 256 paths (FP64) or the matrix-core
-    // kernel's workgroups (FP32)
+    // rows of the seeds' partials: blocks of 256 paths (FP64) or the matrix-core kernel's
+    // workgroups (FP32)
     const int64_t tiles = f64 ? (P + kBlock - 1) / kBlock : pf_adjoint_seed_mfma_blocks(P);
-    HJM_TRY(dev_alloc(&c.bp, (size_t)tiles * nd));
+    HJM_TRY(dev_alloc(&c.bp, (size_t)tiles * 2 * nd));
+    hipStream_t st = p->stream;
     if (!f64) {
         // -Gamma^T in the order the seed's second product reads it
-        std::vector<double> coef, a;
-        std::vector<int> kmax;
-        build_tables(portfolio, nd, coef, a, kmax);
-        std::vector<uint16_t> tf;
-        build_adjoint_fragments(coef, nd, p->nsets, kMaxPeriods, tf);
-        HJM_TRY(dev_alloc(&c.tfrag, tf.size()));
-        HJM_HIP(hipMemcpy(c.tfrag, tf.data(), tf.size() * sizeof(uint16_t), hipMemcpyHostToDevice),
-                HJM_ERR_DEVICE);
+        const size_t nch = (size_t)(value_mtiles(p->nsets) + 1) / 2;
+        HJM_TRY(dev_alloc(&c.tfrag, (size_t)nd * 4 * nch * kMfmaParts * kWave * 8));
+        HJM_HIP(launch_adjoint_fragments(p->d_coef, p->nsets, nd, c.tfrag, st), HJM_ERR_LAUNCH);
     }
     hipEvent_t e0 = p->ev[5], e1 = p->ev[6];
     // the matrix-core forward keeps its normals for the reverse sweep; without the memory
@@ -661,33 +651,28 @@ int hjm_portfolio_cva_greeks(const hjm_market* market, const hjm_portfolio* port
     if ((p->use_mfma || p->use_mfma64) && config->adjoint_normals == HJM_ADJ_NORMALS_AUTO &&
         dev_alloc(&c.zs, (size_t)p->grid.nsteps * 3 * (size_t)P) != HJM_OK)
         c.zs = nullptr;
-    hipStream_t st = p->stream;
     HJM_TRY(pplan_enqueue(p, true, c.zs));
     HJM_HIP(hipEventRecord(e0, st), HJM_ERR_DEVICE);
     hipError_t err = f64 ? launch_pf_adjoint_seed_f64(p->vp, (const double*)p->d_curves, p->d_logb,
-                                                      (const double*)p->d_coef, (const double*)p->d_a,
+                                                      p->d_coef, p->d_a,
                                                       p->d_kmax, p->d_w, c.gbar, c.beta, c.bp, st)
                          : launch_pf_adjoint_seed_mfma(p->vp, (const float*)p->d_curves, p->d_logb,
                                                        p->d_vfrag, c.tfrag, p->d_apad, p->d_tilek,
                                                        p->d_w, c.gbar, c.beta, c.bp, st);
     HJM_HIP(err, HJM_ERR_LAUNCH);
     const double cc = p->grid.dt / portfolio->dtau;
-    // beta summed over the paths at every date (the drift gradient's bank-account terms)
-    HJM_HIP(launch_column_sum(c.bp, tiles, nd, c.sums + kOut, st), HJM_ERR_LAUNCH);
+    // over the paths at every date: beta (the drift gradient's bank-account terms), w E
+    HJM_HIP(launch_column_sum(c.bp, tiles, 2 * nd, c.sums + kOut, st), HJM_ERR_LAUNCH);
     HJM_HIP(launch_pf_adjoint(p->grid, cc, p->d_normals, c.zs, c.gbar, c.beta, c.part, st),
             HJM_ERR_LAUNCH);
     HJM_HIP(launch_column_sum(c.part, nb, kOut, c.sums, st), HJM_ERR_LAUNCH);
     HJM_HIP(hipEventRecord(e1, st), HJM_ERR_DEVICE);
-    std::vector<double> cvas(p->nsets);
-    hjm_portfolio_results r{};
-    r.cva = cvas.data();
-    HJM_TRY(pplan_collect(p, &r));
-    std::vector<double> sums((size_t)kOut + kMaxDates, 0.0);
-    HJM_HIP(hipMemcpy(sums.data(), c.sums, sizeof(double) * (kOut + nd), hipMemcpyDeviceToHost),
-            HJM_ERR_DEVICE);
+    double* sums = static_cast<double*>(p->ctx.c->host);
+    HJM_HIP(hipMemcpyAsync(sums, c.sums, sizeof(double) * nsum, hipMemcpyDeviceToHost, st), HJM_ERR_DEVICE);
+    HJM_HIP(hipStreamSynchronize(st), HJM_ERR_LAUNCH);
     double total = 0.0;
-    for (double v : cvas) total += v;
-    if (gr->cva) *gr->cva = total;
+    for (int e = 0; e < nd; ++e) total += sums[kOut + nd + e];
+    if (gr->cva) *gr->cva = total / (double)P;
     if (gr->cva_stderr) *gr->cva_stderr = NAN;
     const double inv = 1.0 / (double)P, dt = p->grid.dt;
     double dv[kFactors * kTenors], dm[kTenors];
@@ -701,7 +686,7 @@ int hjm_portfolio_cva_greeks(const hjm_market* market, const hjm_portfolio* port
         double musum = 0.0;
         for (int e = 1; e <= E; ++e) musum += (double)e * sums[kOut + e];
         musum *= dt;
-        const double* L = sums.data() + 3 * kTenors;
+        const double* L = sums + 3 * kTenors;
         for (int j = 0; j < kTenors; ++j) {
             double a = B[(size_t)j * kTenors] * musum;
             for (int m = 0; m < kTenors; ++m) a += A[(size_t)j * kTenors + m] * L[m];
@@ -720,7 +705,7 @@ int hjm_portfolio_cva_greeks(const hjm_market* market, const hjm_portfolio* port
         *gr->stored_normals_bytes = c.zs ? (int64_t)p->grid.nsteps * 3 * P * (int64_t)sizeof(float) : 0;
     if (gr->timings_ms) {
         float fwd = 0.f, adj = 0.f;
-        HJM_HIP(hipEventElapsedTime(&fwd, p->ev[0], p->ev[4]), HJM_ERR_DEVICE);
+        HJM_HIP(hipEventElapsedTime(&fwd, p->ev[0], p->ev[1]), HJM_ERR_DEVICE);
         HJM_HIP(hipEventElapsedTime(&adj, e0, e1), HJM_ERR_DEVICE);
         gr->timings_ms[0] = fwd;
         gr->timings_ms[1] = adj;

@@ -75,6 +75,24 @@ hipError_t launch_ref_adjoint(const RefGrid& rg, double c, double sqrt_dt, const
                               const float* zs, const float* gx, const float* gA, double* partials,
                               hipStream_t st);
 
+// A book's swaps on the device, grouped by netting set (the caller's order within a set):
+// maturity in periods, signed notional, notional x rate x dtau; set g owns [first[g], first[g + 1]).
+struct BookSwaps {
+    const int* first;
+    const int* periods;
+    const double* notional;
+    const double* coupon;
+};
+// Coefficient tables [ndates][nsets][60], [ndates][nsets] of the set values a - gamma P and the
+// sets' largest live period; from them the matrix-core tables of FP32 plans, and the adjoint's.
+hipError_t launch_book_tables(const BookSwaps& b, int nsets, int ndates, double* coef, double* a, int* kmax,
+                              hipStream_t st);
+hipError_t launch_value_fragments(const double* coef, const double* a, const int* kmax, int nsets, int ndates,
+                                  uint16_t* frag, float* apad, int* tilek, hipStream_t st);
+hipError_t launch_adjoint_fragments(const double* coef, int nsets, int ndates, uint16_t* frag, hipStream_t st);
+hipError_t launch_clear_matured(const int* kmax, int rows, int64_t paths, void* ex, int elem_bytes,
+                                hipStream_t st);
+
 // Portfolio semantics.
 hipError_t launch_pf_paths_f64(const RefStepConsts<double>& k, const PfGrid& g, const double* normals,
                                double* curves, double* logb, int block, int grid, hipStream_t st);
@@ -83,7 +101,7 @@ hipError_t launch_pf_paths_f32(const RefStepConsts<float>& k, const PfGrid& g, c
 hipError_t launch_pf_value_f64(const PfValueParams& v, const double* curves, const double* logb,
                                const double* coef, const double* a, const int* kmax, double* ex,
                                hipStream_t st);
-// FP32 plans: the matrix-core valuation over build_value_fragments' tables, of paths
+// FP32 plans: the matrix-core valuation over launch_value_fragments' tables, of paths
 // [0, count) (count < 0: all); filter (or null): only the rows (date, set) whose PFE
 // bracket selection is unresolved for rank fk with fcap candidate slots
 hipError_t launch_pf_value_mfma(const PfValueParams& v, const float* curves, const double* logb,
@@ -132,18 +150,19 @@ hipError_t launch_bracket_finish(const double* x, int rows, int64_t n, int64_t k
 hipError_t launch_bracket_finish_f32(const float* x, int rows, int64_t n, int64_t k, void* ws,
                                      double* out, hipStream_t st);
 
-// FP64 plans; beta_partials: [blocks of 256 paths][ndates] sums of beta over the block's paths
+// FP64 plans; partials: [blocks of 256 paths][2 ndates], the sums over the block's paths of
+// beta at every date, then of sum_g w_ge E_ge (the CVA's numerator)
 hipError_t launch_pf_adjoint_seed_f64(const PfValueParams& v, const double* curves,
                                       const double* logb, const double* coef, const double* a,
                                       const int* kmax, const double* w, float* gbar, float* beta,
-                                      double* beta_partials, hipStream_t st);
-// FP32 plans: both products on the matrix cores over build_value_fragments' and
-// build_adjoint_fragments' tables; beta_partials: [pf_adjoint_seed_mfma_blocks(paths)][ndates]
+                                      double* partials, hipStream_t st);
+// FP32 plans: both products on the matrix cores over launch_value_fragments' and
+// launch_adjoint_fragments' tables; partials: [pf_adjoint_seed_mfma_blocks(paths)][2 ndates]
 int64_t pf_adjoint_seed_mfma_blocks(int64_t paths);
 hipError_t launch_pf_adjoint_seed_mfma(const PfValueParams& v, const float* curves, const double* logb,
                                        const uint16_t* gfrag, const uint16_t* tfrag, const float* apad,
                                        const int* tilek, const double* w, float* gbar, float* beta,
-                                       double* beta_partials, hipStream_t st);
+                                       double* partials, hipStream_t st);
 // One-pass sweep, two lanes per path; partials [pf_adjoint_blocks(paths)][5 * 51] as the
 // reference sweep's.
 int64_t pf_adjoint_blocks(int64_t paths);

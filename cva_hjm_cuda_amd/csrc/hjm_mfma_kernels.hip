@@ -857,7 +857,7 @@ __device__ __forceinline__ T cross_row_sum(T x)
 // Both products run on the matrix cores (bf16x6 split products). The second takes u
 // straight from the first's accumulators: its K chunk c holds sets 16 (2c + i/4) + 4 g +
 // i % 4 in lane group g's slot i, which are the registers i % 4 of set tiles 2c and 2c + 1
-// (build_adjoint_fragments orders -Gamma^T the same way), and its output rows are the
+// (launch_adjoint_fragments orders -Gamma^T the same way), and its output rows are the
 // periods 16 pm + 4 g + r. A workgroup of 8 waves values 128 paths at one date
 // (blockIdx.y), then the next of its kSeedGroups groups; -Gamma and -Gamma^T of 128 sets
 // at a time are staged in LDS (once per workgroup up to 128 sets), the bond prices go
@@ -874,16 +874,16 @@ __global__ __launch_bounds__(kSeedBlock) void pf_adjoint_seed_mfma_kernel(
     const PfValueParams v, int mtiles, const float* __restrict__ curves,
     const double* __restrict__ logb, const u4_t* __restrict__ gfrag, const u4_t* __restrict__ tfrag,
     const float* __restrict__ apad, const int* __restrict__ tilek, const double* __restrict__ w,
-    float* __restrict__ gbar, float* __restrict__ beta, double* __restrict__ beta_partials)
+    float* __restrict__ gbar, float* __restrict__ beta, double* __restrict__ partials)
 {
     __shared__ u4_t s1[kSeedTiles * kValueFragsPerTile * kWave];
     __shared__ u4_t s2[kPeriodTiles * (kSeedTiles / 2) * kMfmaParts * kWave];
     // per path: bond prices, then iota; rows of 65 floats so the 16 paths of a wave fall
     // in distinct LDS banks
     __shared__ float scr[kSeedWaves][16][65];
-    __shared__ float s_w[16 * kSeedTiles];
+    __shared__ double s_w[16 * kSeedTiles];
     __shared__ int s_tk[kSeedTiles];
-    __shared__ double s_b[kSeedWaves];
+    __shared__ double s_b[2][kSeedWaves];
     const int e = blockIdx.y;
     const int64_t P = v.paths;
     const int G = v.nsets, nd = v.ndates;
@@ -903,7 +903,7 @@ __global__ __launch_bounds__(kSeedBlock) void pf_adjoint_seed_mfma_kernel(
         }
         for (int gl = threadIdx.x; gl < 16 * kSeedTiles; gl += kSeedBlock) {
             const int g = 16 * m0 + gl;
-            s_w[gl] = g < G ? (float)w[(int64_t)g * nd + e] : 0.f;
+            s_w[gl] = g < G ? w[(int64_t)g * nd + e] : 0.0;
         }
         if (threadIdx.x < kSeedTiles)
             s_tk[threadIdx.x] = (int)threadIdx.x < nt ? tilek[(int64_t)e * mtiles + m0 + threadIdx.x] : 0;
@@ -913,6 +913,7 @@ __global__ __launch_bounds__(kSeedBlock) void pf_adjoint_seed_mfma_kernel(
         __syncthreads();
     }
     double bsum = 0.0;   // the wave's sum of beta over its paths of all groups
+    double csum = 0.0;   // the lane's sum of w E, the exposures as the exposure pass makes them
     for (int pg = 0; pg < kSeedGroups; ++pg) {
         const int64_t p = ((int64_t)blockIdx.x * kSeedGroups + pg) * kSeedPaths + wave * 16 + col;
         const bool live = p < P;
@@ -943,8 +944,11 @@ __global__ __launch_bounds__(kSeedBlock) void pf_adjoint_seed_mfma_kernel(
                     value_tile<1>(s1 + (m * kValueFragsPerTile) * kWave, lane, s_tk[m], a4, bs, acc);
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        const float V = acc[0][r], wg = s_w[16 * m + 4 * grp + r];
+                        const double wd = s_w[16 * m + 4 * grp + r];
+                        const float V = acc[0][r], wg = (float)wd;
                         const bool pos = V > 0.f;
+                        const float E = exposure_of(V, D);
+                        csum = __builtin_fma(wd, live ? (double)E : 0.0, csum);
                         u[m][r] = pos ? wg * D : 0.f;
                         b -= pos ? wg * V * D : 0.f;
                     }
@@ -1017,13 +1021,17 @@ __global__ __launch_bounds__(kSeedBlock) void pf_adjoint_seed_mfma_kernel(
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         __builtin_amdgcn_wave_barrier();   // the next group's prices overwrite these rows
     }
-    if (lane == 0) s_b[wave] = bsum;
+    csum = wave_sum(csum);
+    if (lane == 0) {
+        s_b[0][wave] = bsum;
+        s_b[1][wave] = csum;
+    }
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (threadIdx.x < 2) {
         double t = 0.0;
 #pragma unroll
-        for (int ww = 0; ww < kSeedWaves; ++ww) t += s_b[ww];
-        beta_partials[(int64_t)blockIdx.x * nd + e] = t;
+        for (int ww = 0; ww < kSeedWaves; ++ww) t += s_b[threadIdx.x][ww];
+        partials[(int64_t)blockIdx.x * 2 * nd + threadIdx.x * nd + e] = t;
     }
 }
 
@@ -1035,14 +1043,14 @@ int64_t pf_adjoint_seed_mfma_blocks(int64_t paths)
 hipError_t launch_pf_adjoint_seed_mfma(const PfValueParams& v, const float* curves, const double* logb,
                                        const uint16_t* gfrag, const uint16_t* tfrag, const float* apad,
                                        const int* tilek, const double* w, float* gbar, float* beta,
-                                       double* beta_partials, hipStream_t st)
+                                       double* partials, hipStream_t st)
 {
     const int mtiles = value_mtiles(v.nsets);
     if (v.paths <= 0 || v.nsets <= 0 || v.ndates <= 0 || mtiles > kMaxPfMTiles) return hipErrorInvalidValue;
     const dim3 grid((unsigned)pf_adjoint_seed_mfma_blocks(v.paths), (unsigned)v.ndates);
     pf_adjoint_seed_mfma_kernel<<<grid, kSeedBlock, 0, st>>>(
         v, mtiles, curves, logb, reinterpret_cast<const u4_t*>(gfrag), reinterpret_cast<const u4_t*>(tfrag),
-        apad, tilek, w, gbar, beta, beta_partials);
+        apad, tilek, w, gbar, beta, partials);
     return hipGetLastError();
 }
 

@@ -360,71 +360,11 @@ constexpr int kValueFragsPerTile = 2 * kMfmaParts;  // u4 fragments per lane and
 inline int value_mtiles(int nsets) { return (nsets + 15) / 16; }
 constexpr int kMaxPfMTiles = (HJM_MAX_SETS + 15) / 16;
 
-inline void build_value_fragments(const std::vector<double>& coef, const std::vector<double>& a,
-                                  const std::vector<int>& kmax, int ndates, int nsets, int kpad,
-                                  std::vector<uint16_t>& frag, std::vector<float>& apad,
-                                  std::vector<int>& tilek)
-{
-    const int mt = value_mtiles(nsets);
-    frag.assign((size_t)ndates * mt * kValueFragsPerTile * kWave * 8, 0);
-    apad.assign((size_t)ndates * mt * 16, 0.f);
-    tilek.assign((size_t)ndates * mt, 0);
-    for (int e = 0; e < ndates; ++e)
-        for (int m = 0; m < mt; ++m) {
-            for (int j = 0; j < 16; ++j) {
-                const int g = 16 * m + j;
-                if (g >= nsets) continue;
-                apad[((size_t)e * mt + m) * 16 + j] = (float)a[(size_t)e * nsets + g];
-                tilek[(size_t)e * mt + m] = std::max(tilek[(size_t)e * mt + m], kmax[(size_t)e * nsets + g]);
-            }
-            for (int c = 0; c < 2; ++c)
-                for (int l = 0; l < kWave; ++l)
-                    for (int i = 0; i < 8; ++i) {
-                        const int g = 16 * m + l % 16, kk = 32 * c + 8 * (l / 16) + i;
-                        const double w = (g < nsets && kk < kpad)
-                                             ? -coef[((size_t)e * nsets + g) * kpad + kk]
-                                             : 0.0;
-                        const uint16_t h = bf16_rne(w);
-                        const double r1 = w - bf16_value(h);
-                        const uint16_t mm = bf16_rne(r1);
-                        const uint16_t lo = bf16_rne(r1 - bf16_value(mm));
-                        const uint16_t parts[3] = {h, mm, lo};
-                        for (int q = 0; q < kMfmaParts; ++q)
-                            frag[(((((size_t)e * mt + m) * 2 + c) * kMfmaParts + q) * kWave + l) * 8 + i] =
-                                parts[q];
-                    }
-        }
-}
-
 // The portfolio adjoint's second product dP = (-Gamma)^T u on the matrix cores
 // (pf_adjoint_seed_mfma_kernel): per date, 4 period tiles x ceil(mtiles / 2) K chunks of 32
 // sets x 3 bf16 parts, [date][pm][c][part][lane][i] = part of -gamma[date][set][16 pm +
 // lane % 16] with set = 16 (2c + i/4) + 4 (lane/16) + i%4, the order in which the first
-// product's accumulators hold u (0 past the last set or period).
-inline void build_adjoint_fragments(const std::vector<double>& coef, int ndates, int nsets, int kpad,
-                                    std::vector<uint16_t>& frag)
-{
-    const int nch = (value_mtiles(nsets) + 1) / 2;
-    frag.assign((size_t)ndates * 4 * nch * kMfmaParts * kWave * 8, 0);
-    for (int e = 0; e < ndates; ++e)
-        for (int pm = 0; pm < 4; ++pm)
-            for (int c = 0; c < nch; ++c)
-                for (int l = 0; l < kWave; ++l)
-                    for (int i = 0; i < 8; ++i) {
-                        const int set = 16 * (2 * c + i / 4) + 4 * (l / 16) + i % 4;
-                        const int kk = 16 * pm + l % 16;
-                        const double w = (set < nsets && kk < kpad)
-                                             ? -coef[((size_t)e * nsets + set) * kpad + kk]
-                                             : 0.0;
-                        const uint16_t h = bf16_rne(w);
-                        const double r1 = w - bf16_value(h);
-                        const uint16_t mm = bf16_rne(r1);
-                        const uint16_t lo = bf16_rne(r1 - bf16_value(mm));
-                        const uint16_t parts[3] = {h, mm, lo};
-                        for (int q = 0; q < kMfmaParts; ++q)
-                            frag[(((((size_t)e * 4 + pm) * nch + c) * kMfmaParts + q) * kWave + l) * 8 + i] =
-                                parts[q];
-                    }
-}
+// product's accumulators hold u (0 past the last set or period). Built on the device
+// (hjm_book_kernels.hip), as are the valuation's.
 
 }  // namespace hjm

@@ -644,7 +644,7 @@ __global__ __launch_bounds__(kBlock) void pf_adjoint_seed_kernel(const PfValuePa
                                                                  const double* __restrict__ w,
                                                                  float* __restrict__ gbar,
                                                                  float* __restrict__ beta,
-                                                                 double* __restrict__ beta_partials)
+                                                                 double* __restrict__ partials)
 {
     const int64_t P = v.paths;
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -723,17 +723,21 @@ __global__ __launch_bounds__(kBlock) void pf_adjoint_seed_kernel(const PfValuePa
         Sk[kk] = S;
         if (kk > kTenors - 1) ext += (Real)(kk - (kTenors - 1)) * iota;
     }
-    // the workgroup's sum of beta at this date (the drift gradient's bank-account terms)
+    // the workgroup's sums at this date: beta as stored (the drift gradient's bank-account
+    // terms) and -beta = sum_g w E in double (the CVA)
     {
-        __shared__ double bred[kBlock / kWave];
-        const double bs = wave_sum(live ? (double)(float)b : 0.0);
-        if (threadIdx.x % kWave == 0) bred[threadIdx.x / kWave] = bs;
+        __shared__ double bred[2][kBlock / kWave];
+        const double bs = wave_sum(live ? (double)(float)b : 0.0), cs = wave_sum(live ? -b : 0.0);
+        if (threadIdx.x % kWave == 0) {
+            bred[0][threadIdx.x / kWave] = bs;
+            bred[1][threadIdx.x / kWave] = cs;
+        }
         __syncthreads();
-        if (threadIdx.x == 0) {
+        if (threadIdx.x < 2) {
             double t = 0.0;
 #pragma unroll
-            for (int q = 0; q < kBlock / kWave; ++q) t += bred[q];
-            beta_partials[(int64_t)blockIdx.x * v.ndates + e] = t;
+            for (int q = 0; q < kBlock / kWave; ++q) t += bred[threadIdx.x][q];
+            partials[(int64_t)blockIdx.x * 2 * v.ndates + threadIdx.x * v.ndates + e] = t;
         }
     }
     if (!live) return;
@@ -926,20 +930,20 @@ template <typename Real>
 static hipError_t pf_adj_seed_launch(const PfValueParams& v, const Real* curves, const double* logb,
                                      const Real* coef, const Real* a, const int* kmax,
                                      const double* w, float* gbar, float* beta,
-                                     double* beta_partials, hipStream_t st)
+                                     double* partials, hipStream_t st)
 {
     const dim3 grid((unsigned)((v.paths + kBlock - 1) / kBlock), (unsigned)v.ndates);
     pf_adjoint_seed_kernel<Real><<<grid, kBlock, 0, st>>>(v, curves, logb, coef, a, kmax, w, gbar,
-                                                          beta, beta_partials);
+                                                          beta, partials);
     return hipGetLastError();
 }
 
 hipError_t launch_pf_adjoint_seed_f64(const PfValueParams& v, const double* curves,
                                       const double* logb, const double* coef, const double* a,
                                       const int* kmax, const double* w, float* gbar, float* beta,
-                                      double* beta_partials, hipStream_t st)
+                                      double* partials, hipStream_t st)
 {
-    return pf_adj_seed_launch<double>(v, curves, logb, coef, a, kmax, w, gbar, beta, beta_partials,
+    return pf_adj_seed_launch<double>(v, curves, logb, coef, a, kmax, w, gbar, beta, partials,
                                       st);
 }
 

@@ -259,9 +259,9 @@ int hjm_simulate_portfolio(const hjm_market* market, const hjm_portfolio* portfo
                            hjm_portfolio_results* results);
 /* Total portfolio CVA (sum over netting sets) and its pathwise-adjoint sensitivities to
  * the 51 initial forwards, 153 loadings and 51 drifts (hjm_greeks; cva_stderr = NaN:
- * per-set standard errors come from hjm_simulate_portfolio). Forward pass as
- * hjm_simulate_portfolio without PFE; the curve checkpoints at every date seed the
- * backward sweep. timings_ms: forward, adjoint, total. */
+ * per-set standard errors come from hjm_simulate_portfolio). The path kernel as in
+ * hjm_simulate_portfolio; the curve checkpoints at every date give the CVA and seed the
+ * backward sweep. timings_ms: forward (paths), adjoint (valuation, seeds, sweep), total. */
 int hjm_portfolio_cva_greeks(const hjm_market* market, const hjm_portfolio* portfolio,
                              const hjm_config* config, const hjm_tuning* tuning,
                              hjm_greeks* greeks);
