@@ -17,6 +17,7 @@
 #include "hjm_host.h"
 #include "hjm_mfma_plan.h"
 #include "hjm_select.h"
+#include "hjm_sweep.h"
 
 using namespace hjm;
 using namespace hjm_host;
@@ -158,7 +159,9 @@ void fill_ref_params(const hjm_market* market, const hjm_swap* swap, const hjm_c
     cva_weights(kTenors, swap->dtau, cfg->hazard_rate, cfg->recovery, e.w);
 }
 
-int plan_init(hjm_plan p, const hjm_market* market, const hjm_swap* swap, const hjm_config* cfg)
+// host_doubles: size of the pinned result buffer
+int plan_init(hjm_plan p, const hjm_market* market, const hjm_swap* swap, const hjm_config* cfg,
+              size_t host_doubles = kStatSlots + kTenors)
 {
     int stride, S, D;
     HJM_TRY(check_ref_config(market, swap, cfg, &stride, &S, &D));
@@ -181,7 +184,7 @@ int plan_init(hjm_plan p, const hjm_market* market, const hjm_swap* swap, const 
 
     DeviceGuard guard;
     HJM_TRY(guard.set(cfg->device));
-    HJM_TRY(p->ctx.take(cfg->device, sizeof(double) * (kStatSlots + kTenors)));
+    HJM_TRY(p->ctx.take(cfg->device, sizeof(double) * host_doubles));
     p->stream = p->ctx.c->stream;
     p->ev = p->ctx.c->ev;
     p->h_res = static_cast<double*>(p->ctx.c->host);
@@ -242,6 +245,22 @@ int plan_init(hjm_plan p, const hjm_market* market, const hjm_swap* swap, const 
                 HJM_ERR_DEVICE);
     }
     HJM_HIP(hipStreamSynchronize(p->stream), HJM_ERR_DEVICE);
+    return HJM_OK;
+}
+
+int plan_create(hjm_plan* out, const hjm_market* market, const hjm_swap* swap, const hjm_config* config,
+                size_t host_doubles)
+{
+    if (!out) return HJM_ERR_NULL;
+    *out = nullptr;
+    hjm_plan p = new (std::nothrow) hjm_plan_s();
+    if (!p) return HJM_ERR_ALLOC;
+    const int rc = plan_init(p, market, swap, config, host_doubles);
+    if (rc != HJM_OK) {
+        plan_release(p);
+        return rc;
+    }
+    *out = p;
     return HJM_OK;
 }
 
@@ -409,17 +428,7 @@ int hjm_hjm_drift(const double* vols, double dtau, double* drifts)
 int hjm_plan_create(hjm_plan* out, const hjm_market* market, const hjm_swap* swap,
                     const hjm_config* config)
 {
-    if (!out) return HJM_ERR_NULL;
-    *out = nullptr;
-    hjm_plan p = new (std::nothrow) hjm_plan_s();
-    if (!p) return HJM_ERR_ALLOC;
-    const int rc = plan_init(p, market, swap, config);
-    if (rc != HJM_OK) {
-        plan_release(p);
-        return rc;
-    }
-    *out = p;
-    return HJM_OK;
+    return plan_create(out, market, swap, config, kStatSlots + kTenors);
 }
 
 int hjm_plan_execute(hjm_plan plan, hjm_results* results)
@@ -451,12 +460,15 @@ int hjm_cva_greeks_reference(const hjm_market* market, const hjm_swap* swap,
     hjm_config config = *cfg;
     if (config.pfe_quantile <= 1.0) config.pfe_quantile = 0.0;   // no PFE here (> 1: rejected)
     hjm_plan p = nullptr;
-    HJM_TRY(hjm_plan_create(&p, market, swap, &config));
-    constexpr int kOut = 5 * kTenors;  // g0, g1, g2, sum of lambda_e, d spot
+    // pinned: the plan's results, then the sweep's sums (at most 8 row tiles)
+    constexpr size_t kPlan = kStatSlots + kTenors;
+    HJM_TRY(plan_create(&p, market, swap, &config, kPlan + 8 * 16 * 160));
+    constexpr int kOut = 5 * kTenors;  // VALU sweep: g0, g1, g2, sum of lambda_e, d spot
     struct Cleanup {
         hjm_plan p;
         float *gx = nullptr, *gA = nullptr, *zs = nullptr;
         double *part = nullptr, *sums = nullptr, *sap = nullptr;
+        SweepBuffers sweep;
         ~Cleanup()
         {
             (void)p->ctx.quiesce();
@@ -466,6 +478,7 @@ int hjm_cva_greeks_reference(const hjm_market* market, const hjm_swap* swap,
             dev_free(part);
             dev_free(sums);
             dev_free(sap);
+            sweep.free();
             hjm_plan_destroy(p);
         }
     } c{p};
@@ -476,8 +489,6 @@ int hjm_cva_greeks_reference(const hjm_market* market, const hjm_swap* swap,
     const size_t cells = (size_t)kTenors * P;
     HJM_TRY(dev_alloc(&c.gx, cells));
     HJM_TRY(dev_alloc(&c.gA, cells));
-    HJM_TRY(dev_alloc(&c.part, (size_t)nb * kOut));
-    HJM_TRY(dev_alloc(&c.sums, kOut + kTenors));  // then the per-slot sums of gA
     HJM_TRY(dev_alloc(&c.sap, (size_t)p->nblocks * kTenors));
     hipEvent_t e0 = p->ev[5], e1 = p->ev[6];
     // the matrix-core forward keeps its normals for the reverse sweep (one FP32 per factor
@@ -486,31 +497,48 @@ int hjm_cva_greeks_reference(const hjm_market* market, const hjm_swap* swap,
         dev_alloc(&c.zs, (size_t)p->grid.nsteps * 3 * (size_t)P) != HJM_OK)
         c.zs = nullptr;
     hipStream_t st = p->stream;
+    const double dt = p->grid.dt, cc = dt / swap->dtau;
+    SweepGrid sg{};
+    sg.hi = D - 1;
+    sg.lo = 1;
+    sg.paths = P;
+    // the matrix-core sweep for the path kernels' 50-step blocks with in-kernel normals; the
+    // VALU sweep for the others, and where the matrix sweep's buffers cannot be had
+    const bool matrix = S == kMfmaStride && !p->host_rng && D > 1 &&
+                        c.sweep.take(sg, false, cc, p->grid.nsteps, c.zs != nullptr, st) == HJM_OK;
     HJM_TRY(plan_launch(p, false, c.zs));
     HJM_HIP(hipEventRecord(e0, st), HJM_ERR_DEVICE);
-    const double dt = p->grid.dt;
-    const double cc = dt / swap->dtau;
     HJM_HIP(launch_ref_adjoint_seed(p->ep, dt, p->d_nx, p->d_ny, c.gx, c.gA, c.sap, st),
             HJM_ERR_LAUNCH);
-    // gA summed over the paths at every slot (the drift gradient's mu terms)
-    HJM_HIP(launch_column_sum(c.sap, p->nblocks, kTenors, c.sums + kOut, st), HJM_ERR_LAUNCH);
-    HJM_HIP(launch_ref_adjoint(p->grid, cc, sqrt(dt), p->d_normals, c.zs, c.gx, c.gA, c.part, st),
-            HJM_ERR_LAUNCH);
-    HJM_HIP(launch_column_sum(c.part, nb, kOut, c.sums, st), HJM_ERR_LAUNCH);
+    double* sums = p->h_res + kPlan;
+    if (matrix) {
+        HJM_TRY(c.sweep.run(sg, false, c.zs, cfg->seed, cfg->path_offset, c.gx, c.gA, sums, st));
+    } else {
+        HJM_TRY(dev_alloc(&c.part, (size_t)nb * kOut));
+        HJM_TRY(dev_alloc(&c.sums, kOut + kTenors));  // then the per-slot sums of gA
+        // gA summed over the paths at every slot (the drift gradient's mu terms)
+        HJM_HIP(launch_column_sum(c.sap, p->nblocks, kTenors, c.sums + kOut, st), HJM_ERR_LAUNCH);
+        HJM_HIP(launch_ref_adjoint(p->grid, cc, sqrt(dt), p->d_normals, c.gx, c.gA, c.part, st),
+                HJM_ERR_LAUNCH);
+        HJM_HIP(launch_column_sum(c.part, nb, kOut, c.sums, st), HJM_ERR_LAUNCH);
+        HJM_HIP(hipMemcpyAsync(sums, c.sums, sizeof(double) * (kOut + kTenors), hipMemcpyDeviceToHost, st),
+                HJM_ERR_DEVICE);
+    }
     HJM_HIP(hipEventRecord(e1, st), HJM_ERR_DEVICE);
     hjm_results r{};
     r.cva = gr->cva;
     r.cva_stderr = gr->cva_stderr;
     HJM_TRY(plan_collect(p, &r));
-    double sums[kOut + kTenors];
-    HJM_HIP(hipMemcpy(sums, c.sums, sizeof(sums), hipMemcpyDeviceToHost), HJM_ERR_DEVICE);
     const double inv = 1.0 / (double)P;
-    double dv[kFactors * kTenors], dm[kTenors];
-    for (int k = 0; k < kFactors * kTenors; ++k) dv[k] = sums[k] * inv;
-    // drift: dt (A Lambda + B M) / P, Lambda = sum over blocks and paths of lambda_e, M_s =
-    // (s - 1) x (sum over paths of gA at slot s): the injection at slot s is live in the
-    // s - 1 blocks 1 .. s - 1
-    {
+    double ds[kTenors], dv[kFactors * kTenors], dm[kTenors];
+    if (matrix) {
+        sweep_gradients(sums, false, D, cc, dt, S, inv, ds, dv, dm);
+    } else {
+        for (int k = 0; k < kFactors * kTenors; ++k) dv[k] = sums[k] * inv;
+        for (int j = 0; j < kTenors; ++j) ds[j] = sums[4 * kTenors + j] * inv;
+        // drift: dt (A Lambda + B M) / P, Lambda = sum over blocks and paths of lambda_e, M_s =
+        // (s - 1) x (sum over paths of gA at slot s): the injection at slot s is live in the
+        // s - 1 blocks 1 .. s - 1
         std::vector<double> A((size_t)kTenors * kTenors), B((size_t)kTenors * kTenors);
         adjoint_block_sums((double)step_ratio_f32(cc), S, A.data(), B.data());
         double M[kTenors] = {0.0};
@@ -523,8 +551,7 @@ int hjm_cva_greeks_reference(const hjm_market* market, const hjm_swap* swap,
             dm[j] = dt * a * inv;
         }
     }
-    if (gr->d_spot)
-        for (int j = 0; j < kTenors; ++j) gr->d_spot[j] = sums[4 * kTenors + j] * inv;
+    if (gr->d_spot) memcpy(gr->d_spot, ds, sizeof(ds));
     if (gr->d_vol) memcpy(gr->d_vol, dv, sizeof(dv));
     if (gr->d_drift) memcpy(gr->d_drift, dm, sizeof(dm));
     if (gr->d_vol_total) {

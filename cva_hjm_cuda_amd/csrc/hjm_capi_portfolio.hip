@@ -10,6 +10,7 @@
 #include "hjm_kernels.h"
 #include "hjm_mfma_plan.h"
 #include "hjm_select.h"
+#include "hjm_sweep.h"
 
 using namespace hjm;
 using namespace hjm_host;
@@ -228,7 +229,7 @@ int pplan_init(hjm_portfolio_plan p, const hjm_market* market, const hjm_portfol
             HJM_ERR_DEVICE);
     pplan_apply_tuning(p, p->tuning);
     // pinned: the column sums and the PFE rows of one run, or a Greeks call's sums
-    const size_t pinned = std::max<size_t>((size_t)pf->nsets * (2 * nd + 2), 5 * kTenors + 2 * (size_t)nd);
+    const size_t pinned = std::max<size_t>((size_t)pf->nsets * (2 * nd + 2), 64 * 160 + 5 * kTenors + 2 * (size_t)nd);
     HJM_TRY(p->ctx.take(cfg->device, sizeof(double) * pinned));
     p->stream = p->ctx.c->stream;
     p->ev = p->ctx.c->ev;
@@ -603,12 +604,13 @@ int hjm_portfolio_cva_greeks(const hjm_market* market, const hjm_portfolio* port
     cfg.pfe_quantile = 0.0;
     hjm_portfolio_plan p = nullptr;
     HJM_TRY(pplan_create(&p, market, portfolio, &cfg, tuning, true));
-    constexpr int kOut = 5 * kTenors;  // g0, g1, g2, sum of lambda_e, d spot
+    constexpr int kOut = 5 * kTenors;  // VALU sweep: g0, g1, g2, sum of lambda_e, d spot
     struct Cleanup {
         hjm_portfolio_plan p;
         float *gbar = nullptr, *beta = nullptr, *zs = nullptr;
         double *part = nullptr, *sums = nullptr, *bp = nullptr;
         uint16_t* tfrag = nullptr;
+        SweepBuffers sweep;
         ~Cleanup()
         {
             (void)p->ctx.quiesce();
@@ -619,6 +621,7 @@ int hjm_portfolio_cva_greeks(const hjm_market* market, const hjm_portfolio* port
             dev_free(sums);
             dev_free(bp);
             dev_free(tfrag);
+            sweep.free();
             hjm_portfolio_plan_destroy(p);
         }
     } c{p};
@@ -629,8 +632,7 @@ int hjm_portfolio_cva_greeks(const hjm_market* market, const hjm_portfolio* port
     const int64_t nb = pf_adjoint_blocks(P);
     HJM_TRY(dev_alloc(&c.gbar, (size_t)nd * kTenors * P));
     HJM_TRY(dev_alloc(&c.beta, (size_t)nd * P));
-    HJM_TRY(dev_alloc(&c.part, (size_t)nb * kOut));
-    // the sweep's sums, then per date the sums of beta and of the CVA's terms
+    // the VALU sweep's sums, then per date the sums of beta and of the CVA's terms
     const size_t nsum = (size_t)kOut + 2 * nd;
     HJM_TRY(dev_alloc(&c.sums, nsum));
     const bool f64 = p->precision == HJM_FP64;
@@ -651,36 +653,53 @@ int hjm_portfolio_cva_greeks(const hjm_market* market, const hjm_portfolio* port
     if ((p->use_mfma || p->use_mfma64) && config->adjoint_normals == HJM_ADJ_NORMALS_AUTO &&
         dev_alloc(&c.zs, (size_t)p->grid.nsteps * 3 * (size_t)P) != HJM_OK)
         c.zs = nullptr;
+    const double dt = p->grid.dt, cc = dt / portfolio->dtau;
+    SweepGrid sg{};
+    sg.hi = E - 1;
+    sg.lo = 0;
+    sg.dt = (float)dt;
+    sg.paths = P;
+    // the matrix-core sweep for the path kernels' 50-step blocks with in-kernel normals; the
+    // VALU sweep for the others, and where the matrix sweep's buffers cannot be had
+    const bool matrix = p->grid.stride == kMfmaStride && !p->d_normals &&
+                        c.sweep.take(sg, true, cc, p->grid.nsteps, c.zs != nullptr, st) == HJM_OK;
     HJM_TRY(pplan_enqueue(p, true, c.zs));
     HJM_HIP(hipEventRecord(e0, st), HJM_ERR_DEVICE);
     hipError_t err = f64 ? launch_pf_adjoint_seed_f64(p->vp, (const double*)p->d_curves, p->d_logb,
-                                                      p->d_coef, p->d_a,
-                                                      p->d_kmax, p->d_w, c.gbar, c.beta, c.bp, st)
+                                                      p->d_coef, p->d_a, p->d_kmax, p->d_w, c.gbar,
+                                                      c.beta, c.bp, st)
                          : launch_pf_adjoint_seed_mfma(p->vp, (const float*)p->d_curves, p->d_logb,
                                                        p->d_vfrag, c.tfrag, p->d_apad, p->d_tilek,
                                                        p->d_w, c.gbar, c.beta, c.bp, st);
     HJM_HIP(err, HJM_ERR_LAUNCH);
-    const double cc = p->grid.dt / portfolio->dtau;
     // over the paths at every date: beta (the drift gradient's bank-account terms), w E
     HJM_HIP(launch_column_sum(c.bp, tiles, 2 * nd, c.sums + kOut, st), HJM_ERR_LAUNCH);
-    HJM_HIP(launch_pf_adjoint(p->grid, cc, p->d_normals, c.zs, c.gbar, c.beta, c.part, st),
-            HJM_ERR_LAUNCH);
-    HJM_HIP(launch_column_sum(c.part, nb, kOut, c.sums, st), HJM_ERR_LAUNCH);
-    HJM_HIP(hipEventRecord(e1, st), HJM_ERR_DEVICE);
     double* sums = static_cast<double*>(p->ctx.c->host);
+    double* swept = sums + nsum;
+    if (matrix) {
+        HJM_TRY(c.sweep.run(sg, true, c.zs, cfg.seed, cfg.path_offset, c.gbar, c.beta, swept, st));
+    } else {
+        HJM_TRY(dev_alloc(&c.part, (size_t)nb * kOut));
+        HJM_HIP(launch_pf_adjoint(p->grid, cc, p->d_normals, c.gbar, c.beta, c.part, st), HJM_ERR_LAUNCH);
+        HJM_HIP(launch_column_sum(c.part, nb, kOut, c.sums, st), HJM_ERR_LAUNCH);
+    }
+    HJM_HIP(hipEventRecord(e1, st), HJM_ERR_DEVICE);
     HJM_HIP(hipMemcpyAsync(sums, c.sums, sizeof(double) * nsum, hipMemcpyDeviceToHost, st), HJM_ERR_DEVICE);
     HJM_HIP(hipStreamSynchronize(st), HJM_ERR_LAUNCH);
     double total = 0.0;
     for (int e = 0; e < nd; ++e) total += sums[kOut + nd + e];
     if (gr->cva) *gr->cva = total / (double)P;
     if (gr->cva_stderr) *gr->cva_stderr = NAN;
-    const double inv = 1.0 / (double)P, dt = p->grid.dt;
-    double dv[kFactors * kTenors], dm[kTenors];
-    for (int k = 0; k < kFactors * kTenors; ++k) dv[k] = sums[k] * inv;
-    // drift: dt (A Lambda + B mu_sum e_0) / P with Lambda the sum over dates and paths of
-    // the date-end adjoints and mu_sum = dt sum_e e (sum over paths of beta_e): beta_e
-    // feeds mu in the e intervals before date e
-    {
+    const double inv = 1.0 / (double)P;
+    double ds[kTenors], dv[kFactors * kTenors], dm[kTenors];
+    if (matrix) {
+        sweep_gradients(swept, true, nd, cc, dt, p->grid.stride, inv, ds, dv, dm);
+    } else {
+        for (int k = 0; k < kFactors * kTenors; ++k) dv[k] = sums[k] * inv;
+        for (int j = 0; j < kTenors; ++j) ds[j] = sums[4 * kTenors + j] * inv;
+        // drift: dt (A Lambda + B mu_sum e_0) / P with Lambda the sum over dates and paths of
+        // the date-end adjoints and mu_sum = dt sum_e e (sum over paths of beta_e): beta_e
+        // feeds mu in the e intervals before date e
         std::vector<double> A((size_t)kTenors * kTenors), B((size_t)kTenors * kTenors);
         adjoint_block_sums((double)step_ratio_f32(cc), p->grid.stride, A.data(), B.data());
         double musum = 0.0;
@@ -693,8 +712,7 @@ int hjm_portfolio_cva_greeks(const hjm_market* market, const hjm_portfolio* port
             dm[j] = dt * a * inv;
         }
     }
-    if (gr->d_spot)
-        for (int j = 0; j < kTenors; ++j) gr->d_spot[j] = sums[4 * kTenors + j] * inv;
+    if (gr->d_spot) memcpy(gr->d_spot, ds, sizeof(ds));
     if (gr->d_vol) memcpy(gr->d_vol, dv, sizeof(dv));
     if (gr->d_drift) memcpy(gr->d_drift, dm, sizeof(dm));
     if (gr->d_vol_total) {

@@ -154,8 +154,6 @@ inline void cumulative_simpson(const double* y, double h, double* out)
     }
 }
 
-// out += (d m / d sigma)^T g for m_j = sum_k sigma_kj I_kj, I_k = W sigma_k:
-// d m_j / d sigma_kl = delta_jl I_kj + sigma_kj W_jl.
 // Sums over the S steps of a date block of the adjoint's reverse recursion
 // lambda(k + 1) = T^T lambda(k) + mu, lambda(0) = lambda_e (T = I + c Dfwd with the
 // backward difference on the last tenor, c as the FP32 step takes it):
@@ -186,6 +184,55 @@ inline void adjoint_block_sums(double c, int S, double* A, double* B)
     }
 }
 
+// The gradients from the matrix-core sweep's sums M [rows][160] (hjm_adjoint_mfma.hip), each
+// times `scale`: with lambda(s) = (T^T)^{S-1-s} lambda_e + sum_{q < S-1-s} (T^T)^q mu at the
+// block's step s,
+//   loading k: sqrt(dt) ( sum_s (T^T)^{S-1-s} Lambda_ks + sum_{q <= S-2} (T^T)^q sum_{s <= S-2-q} Mu_ks ),
+//   drift:     dt ( sum_{q < S} (T^T)^q Lambda + sum_{q <= S-2} (S-1-q) (T^T)^q Mu ),
+// all by Horner in T^T (c: dt / dtau). mu: rows 64 + j of the reference sweep (to the last
+// slot), row 51 (tenor 0) of the portfolio's.
+inline void sweep_gradients(const double* M, bool pf, int ndates, double c, double dt, int S, double scale,
+                            double* d_spot, double* d_vol, double* d_drift)
+{
+    constexpr int n = kTenors, cols = 160;
+    auto step = [c](double* x) {   // x <- T^T x
+        const double last = x[n - 1];
+        x[n - 1] = (1.0 + c) * last + c * x[n - 2];
+        x[n - 2] = (1.0 - c) * x[n - 2] + c * x[n - 3] - c * last;
+        for (int j = n - 3; j > 0; --j) x[j] = (1.0 - c) * x[j] + c * x[j - 1];
+        x[0] *= 1.0 - c;
+    };
+    auto lambda = [&](int j, int col) { return M[(size_t)j * cols + col]; };
+    auto mu = [&](int j, int col) {
+        if (pf) return j == 0 ? M[(size_t)n * cols + col] : 0.0;
+        return j <= ndates ? M[(size_t)(64 + j) * cols + col] : 0.0;
+    };
+    for (int k = 0; k < kFactors; ++k) {
+        double x[n] = {0.0}, y[n] = {0.0}, pre[n] = {0.0};
+        for (int s = 0; s < S; ++s) {
+            step(x);
+            if (s < S - 1) step(y);
+            for (int j = 0; j < n; ++j) {
+                x[j] += lambda(j, 3 * s + k);
+                pre[j] += mu(j, 3 * s + k);
+                if (s < S - 1) y[j] += pre[j];
+            }
+        }
+        for (int j = 0; j < n; ++j) d_vol[k * n + j] = scale * sqrt(dt) * (x[j] + y[j]);
+    }
+    double x[n] = {0.0};
+    for (int q = S - 1; q >= 0; --q) {
+        step(x);
+        for (int j = 0; j < n; ++j) x[j] += lambda(j, 3 * S) + (double)(S - 1 - q) * mu(j, 3 * S);
+    }
+    for (int j = 0; j < n; ++j) {
+        d_drift[j] = scale * dt * x[j];
+        d_spot[j] = scale * (lambda(j, 3 * S + 1) + (pf ? 0.0 : (double)(S - 1) * mu(j, 3 * S + 1)));
+    }
+}
+
+// out += (d m / d sigma)^T g for m_j = sum_k sigma_kj I_kj, I_k = W sigma_k:
+// d m_j / d sigma_kl = delta_jl I_kj + sigma_kj W_jl.
 inline void drift_vjp(const double* vols, double h, const double* g, double* out)
 {
     double W[kTenors][kTenors];  // W[l][j] = weight of y_l in the integral to node j

@@ -67,13 +67,29 @@ hipError_t launch_pf_paths_mfma(const MfmaGrid& g, const uint16_t* wfrag, float*
 hipError_t launch_ref_adjoint_seed(const ExposureParams& e, double dt, const double* nx,
                                    const double* ny, float* gx, float* gA, double* sa_partials,
                                    hipStream_t st);
-// One-pass sweep, two lanes per path. normals: host FP64 [path][step][3]; else zs: stored
-// FP32 [step][3][path]; else regenerate. partials: [ref_adjoint_blocks(paths)][5 * 51]
+// One-pass VALU sweep, two lanes per path. normals: host FP64 [path][step][3], or null:
+// regenerate. partials: [ref_adjoint_blocks(paths)][5 * 51]
 // (loading gradients of factors 0, 1, 2, sum of the block-end adjoints, d J / d spot).
 int64_t ref_adjoint_blocks(int64_t paths);
 hipError_t launch_ref_adjoint(const RefGrid& rg, double c, double sqrt_dt, const double* normals,
-                              const float* zs, const float* gx, const float* gA, double* partials,
-                              hipStream_t st);
+                              const float* gx, const float* gA, double* partials, hipStream_t st);
+
+// The reverse sweep on the matrix cores (50 steps per date, in-kernel normals; hjm_adjoint_mfma.hip).
+struct SweepGrid {
+    int hi, lo;               // blocks hi .. lo, swept downwards
+    int units;                // units of 32 paths per wave (sweep_units of the whole run)
+    float dt;                 // portfolio: the bank account's step
+    int64_t paths;            // row stride of the seeds
+    int64_t begin, end;       // paths of this launch; begin a multiple of sweep_group
+    int64_t zld;              // row stride of zs, whose column 0 is path begin
+};
+int sweep_row_tiles(bool pf, int ndates);    // rows of a partial: 16 x this, 160 columns
+int sweep_units(int64_t paths);
+int64_t sweep_group(int64_t paths);          // paths of a workgroup: one partial each
+hipError_t launch_adjoint_mfma(const SweepGrid& g, bool pf, const uint16_t* maps, const float* zs,
+                               const float* seed_a, const float* seed_b, float* partials, hipStream_t st);
+hipError_t launch_sweep_sum(const float* partials, int64_t rows, int cols, double* out, hipStream_t st);
+hipError_t launch_sweep_shocks(uint64_t seed, int64_t path0, const SweepGrid& g, float* zs, hipStream_t st);
 
 // A book's swaps on the device, grouped by netting set (the caller's order within a set):
 // maturity in periods, signed notional, notional x rate x dtau; set g owns [first[g], first[g + 1]).
@@ -166,8 +182,8 @@ hipError_t launch_pf_adjoint_seed_mfma(const PfValueParams& v, const float* curv
 // One-pass sweep, two lanes per path; partials [pf_adjoint_blocks(paths)][5 * 51] as the
 // reference sweep's.
 int64_t pf_adjoint_blocks(int64_t paths);
-hipError_t launch_pf_adjoint(const PfGrid& g, double c, const double* normals, const float* zs,
-                             const float* gbar, const float* beta, double* partials, hipStream_t st);
+hipError_t launch_pf_adjoint(const PfGrid& g, double c, const double* normals, const float* gbar,
+                             const float* beta, double* partials, hipStream_t st);
 
 // The reference's own GPU design (baseline form).
 hipError_t launch_blockwise_paths(const RefStepConsts<double>& k, const RefGrid& g, int block_index,

@@ -1,0 +1,80 @@
+// hjm_sweep.h -- buffers and launches of the matrix-core reverse sweep (host side, shared by
+// the reference and portfolio Greeks).
+#pragma once
+#include <vector>
+
+#include "hjm_host.h"
+#include "hjm_kernels.h"
+#include "hjm_mfma_plan.h"
+
+namespace hjm_host {
+
+// Shocks regenerated for the sweep pass through a buffer of at most this many bytes, a whole
+// number of workgroups' paths at a time (the sums do not depend on it: every workgroup writes
+// its own partial).
+constexpr size_t kSweepChunkBytes = (size_t)1 << 30;
+
+struct SweepBuffers {
+    uint16_t* maps = nullptr;
+    float* partials = nullptr;
+    double* out = nullptr;
+    float* chunk = nullptr;
+    int64_t chunk_paths = 0;
+    int rows = 0;             // 16 x row tiles
+
+    // Allocates for g.paths paths and uploads the maps; stored: the forward keeps the shocks.
+    int take(SweepGrid& g, bool pf, double c, int nsteps, bool stored, hipStream_t st)
+    {
+        g.units = sweep_units(g.paths);
+        const int64_t group = sweep_group(g.paths), groups = (g.paths + group - 1) / group;
+        rows = 16 * sweep_row_tiles(pf, g.hi + 1);
+        std::vector<uint16_t> frag;
+        build_sweep_maps(c, pf, frag);
+        HJM_TRY(dev_alloc(&maps, frag.size()));
+        HJM_TRY(dev_alloc(&partials, (size_t)groups * rows * 160));
+        HJM_TRY(dev_alloc(&out, (size_t)rows * 160));
+        if (!stored) {
+            const size_t per = (size_t)group * nsteps * 3 * sizeof(float);
+            int64_t n = std::min<int64_t>(groups, std::max<int64_t>(1, (int64_t)(kSweepChunkBytes / per)));
+            while (n > 1 && dev_alloc(&chunk, (size_t)n * per / sizeof(float)) != HJM_OK) n /= 2;
+            if (!chunk) HJM_TRY(dev_alloc(&chunk, (size_t)n * per / sizeof(float)));
+            chunk_paths = n * group;
+        }
+        // synchronous: the host copy goes with this call
+        HJM_HIP(hipMemcpyAsync(maps, frag.data(), frag.size() * sizeof(uint16_t), hipMemcpyHostToDevice, st),
+                HJM_ERR_DEVICE);
+        HJM_HIP(hipStreamSynchronize(st), HJM_ERR_DEVICE);
+        return HJM_OK;
+    }
+
+    // The sweep and its sums, copied to the (pinned) host array sums[rows * 160].
+    int run(SweepGrid g, bool pf, const float* zs, uint64_t seed, int64_t path0, const float* seed_a,
+            const float* seed_b, double* sums, hipStream_t st)
+    {
+        const int64_t group = sweep_group(g.paths), groups = (g.paths + group - 1) / group;
+        const int cols = rows * 160;
+        const int64_t step = zs ? g.paths : chunk_paths;
+        for (int64_t p = 0; p < g.paths; p += step) {
+            g.begin = p;
+            g.end = std::min(g.paths, p + step);
+            g.zld = zs ? g.paths : g.end - g.begin;
+            if (!zs) HJM_HIP(launch_sweep_shocks(seed, path0, g, chunk, st), HJM_ERR_LAUNCH);
+            HJM_HIP(launch_adjoint_mfma(g, pf, maps, zs ? zs : chunk, seed_a, seed_b,
+                                        partials + (size_t)(p / group) * cols, st),
+                    HJM_ERR_LAUNCH);
+        }
+        HJM_HIP(launch_sweep_sum(partials, groups, cols, out, st), HJM_ERR_LAUNCH);
+        HJM_HIP(hipMemcpyAsync(sums, out, sizeof(double) * cols, hipMemcpyDeviceToHost, st), HJM_ERR_DEVICE);
+        return HJM_OK;
+    }
+
+    void free()
+    {
+        dev_free(maps);
+        dev_free(partials);
+        dev_free(out);
+        dev_free(chunk);
+    }
+};
+
+}  // namespace hjm_host
