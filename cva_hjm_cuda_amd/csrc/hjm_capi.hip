@@ -460,9 +460,9 @@ int hjm_cva_greeks_reference(const hjm_market* market, const hjm_swap* swap,
     hjm_config config = *cfg;
     if (config.pfe_quantile <= 1.0) config.pfe_quantile = 0.0;   // no PFE here (> 1: rejected)
     hjm_plan p = nullptr;
-    // pinned: the plan's results, then the sweep's sums (at most 8 row tiles)
+    // pinned: the plan's results, then the sweep's sums (at most 7 row tiles)
     constexpr size_t kPlan = kStatSlots + kTenors;
-    HJM_TRY(plan_create(&p, market, swap, &config, kPlan + 8 * 16 * 160));
+    HJM_TRY(plan_create(&p, market, swap, &config, kPlan + 7 * 16 * 160));
     constexpr int kOut = 5 * kTenors;  // VALU sweep: g0, g1, g2, sum of lambda_e, d spot
     struct Cleanup {
         hjm_plan p;
@@ -494,7 +494,7 @@ int hjm_cva_greeks_reference(const hjm_market* market, const hjm_swap* swap,
     // the matrix-core forward keeps its normals for the reverse sweep (one FP32 per factor
     // per evolved step and path); without the memory the sweep regenerates them
     if (p->use_mfma && cfg->adjoint_normals == HJM_ADJ_NORMALS_AUTO &&
-        dev_alloc(&c.zs, (size_t)p->grid.nsteps * 3 * (size_t)P) != HJM_OK)
+        dev_alloc(&c.zs, (size_t)p->grid.nsteps * 3 * (size_t)P + kSweepSlack) != HJM_OK)
         c.zs = nullptr;
     hipStream_t st = p->stream;
     const double dt = p->grid.dt, cc = dt / swap->dtau;
@@ -512,7 +512,7 @@ int hjm_cva_greeks_reference(const hjm_market* market, const hjm_swap* swap,
             HJM_ERR_LAUNCH);
     double* sums = p->h_res + kPlan;
     if (matrix) {
-        HJM_TRY(c.sweep.run(sg, false, c.zs, cfg->seed, cfg->path_offset, c.gx, c.gA, sums, st));
+        HJM_TRY(c.sweep.run(sg, false, c.zs, p->grid.nsteps, cfg->seed, cfg->path_offset, c.gx, c.gA, sums, st));
     } else {
         HJM_TRY(dev_alloc(&c.part, (size_t)nb * kOut));
         HJM_TRY(dev_alloc(&c.sums, kOut + kTenors));  // then the per-slot sums of gA

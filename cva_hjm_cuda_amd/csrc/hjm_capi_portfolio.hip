@@ -651,7 +651,7 @@ int hjm_portfolio_cva_greeks(const hjm_market* market, const hjm_portfolio* port
     // the matrix-core forward keeps its normals for the reverse sweep; without the memory
     // the sweep regenerates them
     if ((p->use_mfma || p->use_mfma64) && config->adjoint_normals == HJM_ADJ_NORMALS_AUTO &&
-        dev_alloc(&c.zs, (size_t)p->grid.nsteps * 3 * (size_t)P) != HJM_OK)
+        dev_alloc(&c.zs, (size_t)p->grid.nsteps * 3 * (size_t)P + kSweepSlack) != HJM_OK)
         c.zs = nullptr;
     const double dt = p->grid.dt, cc = dt / portfolio->dtau;
     SweepGrid sg{};
@@ -677,7 +677,7 @@ int hjm_portfolio_cva_greeks(const hjm_market* market, const hjm_portfolio* port
     double* sums = static_cast<double*>(p->ctx.c->host);
     double* swept = sums + nsum;
     if (matrix) {
-        HJM_TRY(c.sweep.run(sg, true, c.zs, cfg.seed, cfg.path_offset, c.gbar, c.beta, swept, st));
+        HJM_TRY(c.sweep.run(sg, true, c.zs, p->grid.nsteps, cfg.seed, cfg.path_offset, c.gbar, c.beta, swept, st));
     } else {
         HJM_TRY(dev_alloc(&c.part, (size_t)nb * kOut));
         HJM_HIP(launch_pf_adjoint(p->grid, cc, p->d_normals, c.gbar, c.beta, c.part, st), HJM_ERR_LAUNCH);

@@ -189,8 +189,8 @@ inline void adjoint_block_sums(double c, int S, double* A, double* B)
 // block's step s,
 //   loading k: sqrt(dt) ( sum_s (T^T)^{S-1-s} Lambda_ks + sum_{q <= S-2} (T^T)^q sum_{s <= S-2-q} Mu_ks ),
 //   drift:     dt ( sum_{q < S} (T^T)^q Lambda + sum_{q <= S-2} (S-1-q) (T^T)^q Mu ),
-// all by Horner in T^T (c: dt / dtau). mu: rows 64 + j of the reference sweep (to the last
-// slot), row 51 (tenor 0) of the portfolio's.
+// all by Horner in T^T (c: dt / dtau). mu: rows 49 + j of the reference sweep (slots 2
+// to the last), row 51 (tenor 0) of the portfolio's.
 inline void sweep_gradients(const double* M, bool pf, int ndates, double c, double dt, int S, double scale,
                             double* d_spot, double* d_vol, double* d_drift)
 {
@@ -205,7 +205,7 @@ inline void sweep_gradients(const double* M, bool pf, int ndates, double c, doub
     auto lambda = [&](int j, int col) { return M[(size_t)j * cols + col]; };
     auto mu = [&](int j, int col) {
         if (pf) return j == 0 ? M[(size_t)n * cols + col] : 0.0;
-        return j <= ndates ? M[(size_t)(64 + j) * cols + col] : 0.0;
+        return j >= 2 && j <= ndates ? M[(size_t)(49 + j) * cols + col] : 0.0;
     };
     for (int k = 0; k < kFactors; ++k) {
         double x[n] = {0.0}, y[n] = {0.0}, pre[n] = {0.0};

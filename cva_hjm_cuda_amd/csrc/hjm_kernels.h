@@ -77,17 +77,20 @@ hipError_t launch_ref_adjoint(const RefGrid& rg, double c, double sqrt_dt, const
 // The reverse sweep on the matrix cores (50 steps per date, in-kernel normals; hjm_adjoint_mfma.hip).
 struct SweepGrid {
     int hi, lo;               // blocks hi .. lo, swept downwards
-    int units;                // units of 32 paths per wave (sweep_units of the whole run)
+    int units;                // units of 32 paths per pair of waves (sweep_units of the whole run)
     float dt;                 // portfolio: the bank account's step
     int64_t paths;            // row stride of the seeds
     int64_t begin, end;       // paths of this launch; begin a multiple of sweep_group
     int64_t zld;              // row stride of zs, whose column 0 is path begin
 };
+constexpr int64_t kSweepMaxPaths = (int64_t)1 << 26;   // 32-bit lane offsets: 48 B x paths
+constexpr int kSweepSlack = 32;              // floats of zeros the sweep needs past zs
 int sweep_row_tiles(bool pf, int ndates);    // rows of a partial: 16 x this, 160 columns
 int sweep_units(int64_t paths);
 int64_t sweep_group(int64_t paths);          // paths of a workgroup: one partial each
-hipError_t launch_adjoint_mfma(const SweepGrid& g, bool pf, const uint16_t* maps, const float* zs,
-                               const float* seed_a, const float* seed_b, float* partials, hipStream_t st);
+hipError_t launch_adjoint_mfma(const SweepGrid& g, bool pf, const uint16_t* map, const float* ptab,
+                               const float* zs, const float* seed_a, const float* seed_b, float* partials,
+                               hipStream_t st);
 hipError_t launch_sweep_sum(const float* partials, int64_t rows, int cols, double* out, hipStream_t st);
 hipError_t launch_sweep_shocks(uint64_t seed, int64_t path0, const SweepGrid& g, float* zs, hipStream_t st);
 

@@ -367,11 +367,10 @@ constexpr int kMaxPfMTiles = (HJM_MAX_SETS + 15) / 16;
 // product's accumulators hold u (0 past the last set or period). Built on the device
 // (hjm_book_kernels.hip), as are the valuation's.
 
-// Maps of the matrix-core reverse sweep (hjm_adjoint_mfma.hip), each 64 x 64 as [m][c][part]
-// [lane][8] bf16 parts of row 16 m + lane % 16 and the curve column of K slot (c, lane / 16,
-// i): (T^T)^S, then for the reference semantics sum_{q < S} (T^T)^q. The portfolio's single
-// map carries that sum's column of tenor 0 in the K slot of row 51 (the scalar mu).
-inline void build_sweep_maps(double c, bool pf, std::vector<uint16_t>& frag)
+// Tables of the matrix-core reverse sweep (hjm_adjoint_mfma.hip): the 64 x 64 map (T^T)^S as
+// [m][c][part][lane][8] bf16 parts of row 16 m + lane % 16 and the curve column of K slot (c,
+// lane / 16, i); and ptab[j][64], column j of sum_{q < S} (T^T)^q (portfolio: j = 0 only).
+inline void build_sweep_maps(double c, bool pf, std::vector<uint16_t>& frag, std::vector<float>& ptab)
 {
     const int n = kTenors, S = kMfmaStride;
     // rows of T^T: y_j = (1 - c) x_j + c x_{j-1}, y_49 also - c x_50, y_50 = (1 + c) x_50 + c x_49
@@ -388,24 +387,23 @@ inline void build_sweep_maps(double c, bool pf, std::vector<uint16_t>& frag)
             }
         A.swap(next);
     }
-    const int maps = pf ? 1 : 2;
-    frag.assign((size_t)maps * 8 * kMfmaParts * kWave * 8, 0);
-    for (int map = 0; map < maps; ++map)
-        for (int m = 0; m < 4; ++m)
-            for (int ch = 0; ch < 2; ++ch)
-                for (int l = 0; l < kWave; ++l)
-                    for (int i = 0; i < 8; ++i) {
-                        const int row = 16 * m + l % 16, k = 16 * (2 * ch + i / 4) + 4 * (l / 16) + i % 4;
-                        if (row >= n) continue;
-                        double w = 0.0;
-                        if (k < n) w = (map ? B : A)[(size_t)row * n + k];
-                        else if (pf && k == n) w = B[(size_t)row * n];
-                        for (int p = 0; p < kMfmaParts; ++p) {
-                            const uint16_t h = bf16_rne(w);
-                            frag[(((((size_t)map * 4 + m) * 2 + ch) * kMfmaParts + p) * kWave + l) * 8 + i] = h;
-                            w -= bf16_value(h);
-                        }
+    ptab.assign((size_t)(pf ? 1 : n) * 64, 0.f);
+    for (int j = 0; j < (pf ? 1 : n); ++j)
+        for (int row = 0; row < n; ++row) ptab[(size_t)j * 64 + row] = (float)B[(size_t)row * n + j];
+    frag.assign((size_t)8 * kMfmaParts * kWave * 8, 0);
+    for (int m = 0; m < 4; ++m)
+        for (int ch = 0; ch < 2; ++ch)
+            for (int l = 0; l < kWave; ++l)
+                for (int i = 0; i < 8; ++i) {
+                    const int row = 16 * m + l % 16, k = 16 * (2 * ch + i / 4) + 4 * (l / 16) + i % 4;
+                    if (row >= n || k >= n) continue;
+                    double w = A[(size_t)row * n + k];
+                    for (int p = 0; p < kMfmaParts; ++p) {
+                        const uint16_t h = bf16_rne(w);
+                        frag[((((size_t)m * 2 + ch) * kMfmaParts + p) * kWave + l) * 8 + i] = h;
+                        w -= bf16_value(h);
                     }
+                }
 }
 
 }  // namespace hjm

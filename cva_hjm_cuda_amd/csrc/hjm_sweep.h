@@ -15,7 +15,8 @@ namespace hjm_host {
 constexpr size_t kSweepChunkBytes = (size_t)1 << 30;
 
 struct SweepBuffers {
-    uint16_t* maps = nullptr;
+    uint16_t* map = nullptr;
+    float* ptab = nullptr;
     float* partials = nullptr;
     double* out = nullptr;
     float* chunk = nullptr;
@@ -25,30 +26,42 @@ struct SweepBuffers {
     // Allocates for g.paths paths and uploads the maps; stored: the forward keeps the shocks.
     int take(SweepGrid& g, bool pf, double c, int nsteps, bool stored, hipStream_t st)
     {
+        if (g.paths > kSweepMaxPaths) return HJM_ERR_UNSUPPORTED;
         g.units = sweep_units(g.paths);
         const int64_t group = sweep_group(g.paths), groups = (g.paths + group - 1) / group;
         rows = 16 * sweep_row_tiles(pf, g.hi + 1);
         std::vector<uint16_t> frag;
-        build_sweep_maps(c, pf, frag);
-        HJM_TRY(dev_alloc(&maps, frag.size()));
+        std::vector<float> table;
+        build_sweep_maps(c, pf, frag, table);
+        HJM_TRY(dev_alloc(&map, frag.size()));
+        HJM_TRY(dev_alloc(&ptab, table.size()));
         HJM_TRY(dev_alloc(&partials, (size_t)groups * rows * 160));
         HJM_TRY(dev_alloc(&out, (size_t)rows * 160));
         if (!stored) {
             const size_t per = (size_t)group * nsteps * 3 * sizeof(float);
             int64_t n = std::min<int64_t>(groups, std::max<int64_t>(1, (int64_t)(kSweepChunkBytes / per)));
-            while (n > 1 && dev_alloc(&chunk, (size_t)n * per / sizeof(float)) != HJM_OK) n /= 2;
-            if (!chunk) HJM_TRY(dev_alloc(&chunk, (size_t)n * per / sizeof(float)));
+            while (n > 1 && dev_alloc(&chunk, (size_t)n * per / sizeof(float) + kSweepSlack) != HJM_OK) n /= 2;
+            if (!chunk) HJM_TRY(dev_alloc(&chunk, (size_t)n * per / sizeof(float) + kSweepSlack));
             chunk_paths = n * group;
         }
-        // synchronous: the host copy goes with this call
-        HJM_HIP(hipMemcpyAsync(maps, frag.data(), frag.size() * sizeof(uint16_t), hipMemcpyHostToDevice, st),
+        // the host copies go with this call
+        HJM_HIP(hipMemcpyAsync(map, frag.data(), frag.size() * sizeof(uint16_t), hipMemcpyHostToDevice, st),
+                HJM_ERR_DEVICE);
+        HJM_HIP(hipMemcpyAsync(ptab, table.data(), table.size() * sizeof(float), hipMemcpyHostToDevice, st),
                 HJM_ERR_DEVICE);
         HJM_HIP(hipStreamSynchronize(st), HJM_ERR_DEVICE);
         return HJM_OK;
     }
 
+    // zs[n]: a buffer of n shocks with its slack cleared.
+    static int clear_slack(float* zs, size_t n, hipStream_t st)
+    {
+        HJM_HIP(hipMemsetAsync(zs + n, 0, kSweepSlack * sizeof(float), st), HJM_ERR_DEVICE);
+        return HJM_OK;
+    }
+
     // The sweep and its sums, copied to the (pinned) host array sums[rows * 160].
-    int run(SweepGrid g, bool pf, const float* zs, uint64_t seed, int64_t path0, const float* seed_a,
+    int run(SweepGrid g, bool pf, float* zs, int nsteps, uint64_t seed, int64_t path0, const float* seed_a,
             const float* seed_b, double* sums, hipStream_t st)
     {
         const int64_t group = sweep_group(g.paths), groups = (g.paths + group - 1) / group;
@@ -58,8 +71,9 @@ struct SweepBuffers {
             g.begin = p;
             g.end = std::min(g.paths, p + step);
             g.zld = zs ? g.paths : g.end - g.begin;
+            HJM_TRY(clear_slack(zs ? zs : chunk, (size_t)g.zld * nsteps * 3, st));
             if (!zs) HJM_HIP(launch_sweep_shocks(seed, path0, g, chunk, st), HJM_ERR_LAUNCH);
-            HJM_HIP(launch_adjoint_mfma(g, pf, maps, zs ? zs : chunk, seed_a, seed_b,
+            HJM_HIP(launch_adjoint_mfma(g, pf, map, ptab, zs ? zs : chunk, seed_a, seed_b,
                                         partials + (size_t)(p / group) * cols, st),
                     HJM_ERR_LAUNCH);
         }
@@ -70,7 +84,8 @@ struct SweepBuffers {
 
     void free()
     {
-        dev_free(maps);
+        dev_free(map);
+        dev_free(ptab);
         dev_free(partials);
         dev_free(out);
         dev_free(chunk);
