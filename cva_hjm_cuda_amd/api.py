@@ -519,9 +519,9 @@ class Tuning:
     pfe_stage_slots: int = 0       # fused pass: 0 = 32
     path_tiles: int = 0            # matrix-core path kernel: N-tiles per wave (0 = 2)
     path_waves: int = 0            # ... waves per workgroup (0 = 8)
-    value_tiles: int = 0           # matrix-core valuation: N-tiles per wave (0 = 4)
-    value_waves: int = 0           # ... waves per workgroup (0 = 4)
-    value_stage: int = 0           # ... M-tiles staged in LDS at a time (0 = 8)
+    value_tiles: int = 0           # matrix-core valuation: N-tiles per wave (0 = 2)
+    value_waves: int = 0           # ... waves per workgroup (0 = 8)
+    value_stage: int = 0           # ... M-tiles staged in LDS at a time (0 = 2)
 
     def _c(self):
         return _Tuning(self.block_size, self.blocks_per_cu, int(self.use_graph),

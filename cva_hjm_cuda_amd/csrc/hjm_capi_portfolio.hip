@@ -129,7 +129,7 @@ int check_tuning(const hjm_tuning& t)
     if (t.pfe_stage_slots < 0 || t.pfe_stage_slots > 32) return HJM_ERR_ARG;
     if (!pf_path_shape_ok(t.path_tiles ? t.path_tiles : 2, t.path_waves ? t.path_waves : 8))
         return HJM_ERR_ARG;
-    if (!pf_value_shape_ok(t.value_tiles ? t.value_tiles : 4, t.value_waves ? t.value_waves : 4))
+    if (!pf_value_shape_ok(t.value_tiles ? t.value_tiles : 2, t.value_waves ? t.value_waves : 8))
         return HJM_ERR_ARG;
     if (t.value_stage < 0 || t.value_stage > 8) return HJM_ERR_ARG;
     return HJM_OK;

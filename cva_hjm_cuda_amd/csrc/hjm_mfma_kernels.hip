@@ -551,17 +551,20 @@ __device__ __forceinline__ void value_bonds(const PfValueParams& v, int e, int64
     // in VGPRs nor their addresses
     asm volatile("" : "+s"(P));
     const float hw = (float)(0.5 * v.dtau), dtf = (float)v.dtau;
-    const float* fc = curves + (int64_t)e * kTenors * P + p;
-    asm volatile("" : "+v"(fc));
+    // (the lane's offset opaque, not a pointer: a pointer through asm loses its address space
+    // and the reads become flat loads, which also hold up the LDS counter)
+    const float* fc = curves + (int64_t)e * kTenors * P;
+    int64_t at = p;
+    asm volatile("" : "+v"(at));
     // segment 0: periods k = 8 grp + 1 .. 8 grp + 8 (tenors 8 grp .. 8 grp + 8 <= 32);
     // segment 1: k = 33 + 8 grp .. 40 + 8 grp (tenors capped at the last, 50)
     float fa[9], fb[9];
 #pragma unroll
-    for (int i = 0; i < 9; ++i) fa[i] = fc[(int64_t)(8 * grp + i) * P];
+    for (int i = 0; i < 9; ++i) fa[i] = fc[at + (int64_t)(8 * grp + i) * P];
 #pragma unroll
     for (int i = 0; i < 9; ++i) {
         const int j = 32 + 8 * grp + i;
-        fb[i] = fc[(int64_t)(j < kTenors - 1 ? j : kTenors - 1) * P];
+        fb[i] = fc[at + (int64_t)(j < kTenors - 1 ? j : kTenors - 1) * P];
     }
     float ca[8], cb[8];
     float s = 0.f;
@@ -621,17 +624,19 @@ __device__ __forceinline__ void value_tile(const u4_t* __restrict__ fr0, int lan
         if (tk > 32 * c) {
             const u4_t* fr = fr0 + (c * kMfmaParts) * kWave + lane;
             const u4_t ah = fr[0], am = fr[kWave], al = fr[2 * kWave];
+            // one product for the N-tiles in turn: no product waits for the one before
 #pragma unroll
-            for (int n = 0; n < NT; ++n) {
-                f4_t x = acc[n];
-                x = mfma_bf16(ah, bs[n][c].h, x);
-                x = mfma_bf16(ah, bs[n][c].m, x);
-                x = mfma_bf16(am, bs[n][c].h, x);
-                x = mfma_bf16(ah, bs[n][c].l, x);
-                x = mfma_bf16(al, bs[n][c].h, x);
-                x = mfma_bf16(am, bs[n][c].m, x);
-                acc[n] = x;
-            }
+            for (int n = 0; n < NT; ++n) acc[n] = mfma_bf16(ah, bs[n][c].h, acc[n]);
+#pragma unroll
+            for (int n = 0; n < NT; ++n) acc[n] = mfma_bf16(ah, bs[n][c].m, acc[n]);
+#pragma unroll
+            for (int n = 0; n < NT; ++n) acc[n] = mfma_bf16(am, bs[n][c].h, acc[n]);
+#pragma unroll
+            for (int n = 0; n < NT; ++n) acc[n] = mfma_bf16(ah, bs[n][c].l, acc[n]);
+#pragma unroll
+            for (int n = 0; n < NT; ++n) acc[n] = mfma_bf16(al, bs[n][c].h, acc[n]);
+#pragma unroll
+            for (int n = 0; n < NT; ++n) acc[n] = mfma_bf16(am, bs[n][c].m, acc[n]);
         }
     }
 }
@@ -645,6 +650,15 @@ __device__ __forceinline__ float exposure_of(float V, float disc) { return V > 0
 // filter (or null): value only the M-tiles holding a set whose PFE row at this date the
 // counting pass left unresolved (bracket_row_resolved false for rank fk and fcap
 // candidate slots); a workgroup with none returns at once.
+//
+// Bound by the exposure stores and the matrix products about equally (128 sets x 61 dates x
+// 1048576 paths are up to 33 GB and 12 products a bond chunk) once nothing in the M-tile loop
+// waits for the stores: a global load there would, since loads and stores share one counter,
+// so the tile constants and live sets are read once into LDS. Products go round the N-tiles,
+// so none waits for the one before. {2 N-tiles, 8 waves, stage 2} by measurement: at that
+// size 9.86 ms against 10.62 for {4, 4, 8}, at 32 sets x 262144 paths 1.20 against 1.23, at
+// 11 x 10007 0.042 against 0.048 (all {4, 4, 8} with the constants in global memory: 12.2,
+// 1.31 and 0.048).
 constexpr int kValMaxStage = 8;  // M-tiles staged at a time, at most
 
 template <int NT, int WAVES>
@@ -662,7 +676,12 @@ __global__ __launch_bounds__(WAVES * kWave) void pf_value_mfma_kernel(const PfVa
     constexpr int kThreads = WAVES * kWave, kPaths = WAVES * NT * 16;
     extern __shared__ u4_t sfrag[];
     __shared__ uint32_t s_need[kMaxPfMTiles];
-    __shared__ uint8_t s_live[HJM_MAX_SETS];
+    // per M-tile and lane group: bit r set where set 16 m + 4 grp + r has a live swap; the
+    // tile's constants and its largest live period (kept out of the loop's global loads, whose
+    // waits would also wait for the exposure stores in flight)
+    __shared__ uint32_t s_live[4 * kMaxPfMTiles];
+    __shared__ f4_t s_a[4 * kMaxPfMTiles];
+    __shared__ int s_tk[kMaxPfMTiles];
     __shared__ int s_any;
     const int e = blockIdx.y;
     const int64_t P = v.paths;
@@ -697,7 +716,17 @@ __global__ __launch_bounds__(WAVES * kWave) void pf_value_mfma_kernel(const PfVa
         const int64_t p = pbase + 16 * n + col;
         value_bonds(v, e, p < count ? p : 0, curves, grp, col, bs[n]);
     }
-    for (int g = threadIdx.x; g < G; g += kThreads) s_live[g] = v.kmax[(int64_t)e * G + g] > 0;
+    for (int t = threadIdx.x; t < 4 * mtiles; t += kThreads) {
+        uint32_t bits = 0;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (4 * t + r < G && v.kmax[(int64_t)e * G + 4 * t + r] > 0) bits |= 1u << r;
+        s_live[t] = bits;
+        s_a[t] = *reinterpret_cast<const f4_t*>(apad + ((int64_t)e * mtiles * 4 + t) * 4);
+        if (t < mtiles) s_tk[t] = tilek[(int64_t)e * mtiles + t];
+    }
+    const bool whole = pbase + NT * 16 <= count;   // wave-uniform
+    const int64_t lane_at = (int64_t)(4 * grp) * P + pbase + col;
     for (int m0 = 0; m0 < mtiles; m0 += stage) {
         const int mt = mtiles - m0 < stage ? mtiles - m0 : stage;
         __syncthreads();
@@ -707,21 +736,23 @@ __global__ __launch_bounds__(WAVES * kWave) void pf_value_mfma_kernel(const PfVa
         for (int mm = 0; mm < mt; ++mm) {
             const int m = m0 + mm;
             if (filter && !s_need[m]) continue;
-            const int tk = tilek[(int64_t)e * mtiles + m];
+            const int tk = __builtin_amdgcn_readfirstlane(s_tk[m]);
             if (tk == 0) continue;   // every set of the tile has matured
-            const f4_t a4 = *reinterpret_cast<const f4_t*>(apad + ((int64_t)e * mtiles + m) * 16 + 4 * grp);
             f4_t acc[NT];
-            value_tile<NT>(sfrag + (mm * kValueFragsPerTile) * kWave, lane, tk, a4, bs, acc);
+            value_tile<NT>(sfrag + (mm * kValueFragsPerTile) * kWave, lane, tk, s_a[4 * m + grp], bs, acc);
+            const uint32_t on = s_live[4 * m + grp];
+            float* rows = exposures + ((int64_t)e * G + 16 * m) * P + lane_at;
 #pragma unroll
-            for (int n = 0; n < NT; ++n) {
-                const int64_t p = pbase + 16 * n + col;
-                if (p < count) {
+            for (int r = 0; r < 4; ++r) {
+                if (!(on >> r & 1u)) continue;
+                float* q = rows + r * P;
+                if (whole) {
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int g = 16 * m + 4 * grp + r;
-                        if (g < G && s_live[g])
-                            exposures[((int64_t)e * G + g) * P + p] = exposure_of(acc[n][r], disc[n]);
-                    }
+                    for (int n = 0; n < NT; ++n) q[16 * n] = exposure_of(acc[n][r], disc[n]);
+                } else {
+#pragma unroll
+                    for (int n = 0; n < NT; ++n)
+                        if (pbase + 16 * n + col < count) q[16 * n] = exposure_of(acc[n][r], disc[n]);
                 }
             }
         }
@@ -741,10 +772,10 @@ hipError_t launch_pf_value_mfma(const PfValueParams& v, const float* curves, con
     if (v.paths <= 0 || v.nsets <= 0 || v.ndates <= 0) return hipErrorInvalidValue;
     const int mtiles = value_mtiles(v.nsets);
     if (mtiles > kMaxPfMTiles) return hipErrorInvalidValue;
-    const int tiles = shape.tiles ? shape.tiles : 4, waves = shape.waves ? shape.waves : 4;
+    const int tiles = shape.tiles ? shape.tiles : 2, waves = shape.waves ? shape.waves : 8;
     if (!pf_value_shape_ok(tiles, waves) || shape.stage < 0 || shape.stage > kValMaxStage)
         return hipErrorInvalidValue;
-    const int stage = std::min(shape.stage ? shape.stage : kValMaxStage, mtiles);
+    const int stage = std::min(shape.stage ? shape.stage : 2, mtiles);
     if (count < 0 || count > v.paths) count = v.paths;
     if (count == 0) return hipSuccess;
     const int64_t paths_per_block = (int64_t)waves * tiles * 16;
@@ -805,6 +836,7 @@ __global__ __launch_bounds__(kSeedBlock) void pf_adjoint_seed_mfma_kernel(
     // in distinct LDS banks
     __shared__ float scr[kSeedWaves][16][65];
     __shared__ double s_w[16 * kSeedTiles];
+    __shared__ f4_t s_a[4 * kSeedTiles];
     __shared__ int s_tk[kSeedTiles];
     __shared__ double s_b[2][kSeedWaves];
     const int e = blockIdx.y;
@@ -828,6 +860,8 @@ __global__ __launch_bounds__(kSeedBlock) void pf_adjoint_seed_mfma_kernel(
             const int g = 16 * m0 + gl;
             s_w[gl] = g < G ? w[(int64_t)g * nd + e] : 0.0;
         }
+        if ((int)threadIdx.x < 4 * nt)
+            s_a[threadIdx.x] = *reinterpret_cast<const f4_t*>(apad + (((int64_t)e * mtiles + m0) * 4 + threadIdx.x) * 4);
         if (threadIdx.x < kSeedTiles)
             s_tk[threadIdx.x] = (int)threadIdx.x < nt ? tilek[(int64_t)e * mtiles + m0 + threadIdx.x] : 0;
     };
@@ -861,10 +895,8 @@ __global__ __launch_bounds__(kSeedBlock) void pf_adjoint_seed_mfma_kernel(
 #pragma unroll
             for (int m = 0; m < kSeedTiles; ++m) {
                 if (m < nt) {
-                    const f4_t a4 =
-                        *reinterpret_cast<const f4_t*>(apad + ((int64_t)e * mtiles + m0 + m) * 16 + 4 * grp);
                     f4_t acc[1];
-                    value_tile<1>(s1 + (m * kValueFragsPerTile) * kWave, lane, s_tk[m], a4, bs, acc);
+                    value_tile<1>(s1 + (m * kValueFragsPerTile) * kWave, lane, s_tk[m], s_a[4 * m + grp], bs, acc);
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const double wd = s_w[16 * m + 4 * grp + r];
@@ -889,17 +921,27 @@ __global__ __launch_bounds__(kSeedBlock) void pf_adjoint_seed_mfma_kernel(
                     for (int i = 0; i < 8; ++i) x[i] = u[2 * cc + i / 4][i % 4];
                     const Split8 bu = split8(x);
 #pragma unroll
-                    for (int q = 0; q < kPeriodTiles; ++q) {
-                        const u4_t* fr = s2 + ((q * (kSeedTiles / 2) + cc) * kMfmaParts) * kWave + lane;
-                        const u4_t ah = fr[0], am = fr[kWave], al = fr[2 * kWave];
-                        f4_t y = dp[q];
-                        y = mfma_bf16(ah, bu.h, y);
-                        y = mfma_bf16(ah, bu.m, y);
-                        y = mfma_bf16(am, bu.h, y);
-                        y = mfma_bf16(ah, bu.l, y);
-                        y = mfma_bf16(al, bu.h, y);
-                        y = mfma_bf16(am, bu.m, y);
-                        dp[q] = y;
+                    for (int q = 0; q < kPeriodTiles; q += 2) {
+                        // two period tiles in turn: no product waits for the one before
+                        const u4_t* f0 = s2 + ((q * (kSeedTiles / 2) + cc) * kMfmaParts) * kWave + lane;
+                        const u4_t* f1 = f0 + (kSeedTiles / 2) * kMfmaParts * kWave;
+                        const u4_t h0 = f0[0], m0_ = f0[kWave], l0 = f0[2 * kWave];
+                        const u4_t h1 = f1[0], m1_ = f1[kWave], l1 = f1[2 * kWave];
+                        f4_t y0 = dp[q], y1 = dp[q + 1];
+                        y0 = mfma_bf16(h0, bu.h, y0);
+                        y1 = mfma_bf16(h1, bu.h, y1);
+                        y0 = mfma_bf16(h0, bu.m, y0);
+                        y1 = mfma_bf16(h1, bu.m, y1);
+                        y0 = mfma_bf16(m0_, bu.h, y0);
+                        y1 = mfma_bf16(m1_, bu.h, y1);
+                        y0 = mfma_bf16(h0, bu.l, y0);
+                        y1 = mfma_bf16(h1, bu.l, y1);
+                        y0 = mfma_bf16(l0, bu.h, y0);
+                        y1 = mfma_bf16(l1, bu.h, y1);
+                        y0 = mfma_bf16(m0_, bu.m, y0);
+                        y1 = mfma_bf16(m1_, bu.m, y1);
+                        dp[q] = y0;
+                        dp[q + 1] = y1;
                     }
                 }
             }

@@ -233,10 +233,10 @@ typedef struct {
                                 whole, for its selection (exact either way) */
     int32_t path_tiles;     /* matrix-core path kernel: N-tiles of 16 paths per wave, and */
     int32_t path_waves;     /* waves per workgroup: {2, 8} (default), {2, 12}, {1, 12}, {1, 16} */
-    int32_t value_tiles;    /* matrix-core valuation: N-tiles per wave, 2 or 4 (default) */
-    int32_t value_waves;    /* waves per workgroup, 4 (default) or 8 */
+    int32_t value_tiles;    /* matrix-core valuation: N-tiles per wave, 2 (default) or 4 */
+    int32_t value_waves;    /* waves per workgroup, 4 or 8 (default) */
     int32_t value_stage;    /* M-tiles (16 sets) of -gamma staged in LDS at a time, 1..8
-                               (default 8) */
+                               (default 2) */
 } hjm_tuning;
 
 typedef struct {
