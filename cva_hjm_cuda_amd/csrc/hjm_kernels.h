@@ -55,8 +55,8 @@ struct MfmaShape {
     int tiles = 0, waves = 0, stage = 0;
     int64_t max_blocks = 0;
 };
-// path kernel: {tiles, waves} in {2, 8} (default), {2, 12}, {1, 12}, {1, 16};
-// valuation: tiles 2 or 4 (default), waves 4 (default) or 8, stage 1..8 (default 8)
+// path kernel: {tiles, waves} in {2, 8} (default: by path count), {2, 12}, {1, 12}, {1, 16};
+// valuation: tiles 2 (default) or 4, waves 4 or 8 (default), stage 1..8 (default 2)
 bool pf_path_shape_ok(int tiles, int waves);
 bool pf_value_shape_ok(int tiles, int waves);
 hipError_t launch_pf_paths_mfma(const MfmaGrid& g, const uint16_t* wfrag, float* curves,

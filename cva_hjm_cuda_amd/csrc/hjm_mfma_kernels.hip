@@ -39,11 +39,6 @@
 
 namespace hjm {
 
-// reference kernel: 8 waves of 2 N-tiles (16 paths each); the portfolio kernel's shape
-// is a template choice (MfmaShape)
-constexpr int kNT = 2;
-constexpr int kMfmaBlock = 512;
-constexpr int kMfmaPathsPerBlock = kMfmaBlock / kWave * kNT * 16;
 
 // last quad whose values complete shock chunk s (values 8 s .. 8 s + 7, three per quad)
 __host__ __device__ constexpr int shock_chunk_last_quad(int s)
@@ -232,26 +227,35 @@ __device__ __forceinline__ void mfma_block(const u4_t* __restrict__ lds_w, const
     }
 }
 
+// Waves per SIMD (registers) and per workgroup, at most, of the path kernels with nt N-tiles
+// per wave. A wave makes all shocks of its paths and all rows: it is bound by the VALU work
+// of the shocks, which the matrix products run beside. More waves per SIMD hide more of its
+// latencies, and two N-tiles per wave share each fragment read.
+__host__ __device__ constexpr int path_waves_per_simd(int nt) { return nt == 1 ? 3 : 2; }
+__host__ __device__ constexpr int max_waves(int nt) { return 4 * path_waves_per_simd(nt); }
+
 // Reference semantics. MT = the live M-tiles of the block map: the curve (tiles 0..3,
 // rows 0..50) and the integral rows 51 + j up to the last recorded slot j = ndates (a
-// tile past it holds tenors whose numeraire is never recorded: ref_mfma_tiles).
-template <bool kStore, int MT>
-__global__ __launch_bounds__(kMfmaBlock) void ref_paths_mfma_kernel(const MfmaGrid g,
+// tile past it holds tenors whose numeraire is never recorded: ref_mfma_tiles). Paths from
+// `begin` on, 16 kNT per wave.
+template <bool kStore, int MT, int kNT>
+__global__ __launch_bounds__(max_waves(kNT) * kWave)
+__attribute__((amdgpu_waves_per_eu(path_waves_per_simd(kNT), path_waves_per_simd(kNT)))) void ref_paths_mfma_kernel(const MfmaGrid g,
                                                                 const u4_t* __restrict__ wfrag,
                                                                 double* __restrict__ num_x,
                                                                 double* __restrict__ num_y,
-                                                                float* __restrict__ zs)
+                                                                float* __restrict__ zs, int64_t begin)
 {
     constexpr int kInt = MT - 3;  // M-tiles holding integral rows (tile 3 holds both kinds)
     extern __shared__ u4_t lds_w[];
-    for (int t = threadIdx.x; t < MT * kMfmaTileFrags * kWave; t += kMfmaBlock)
+    for (int t = threadIdx.x; t < MT * kMfmaTileFrags * kWave; t += blockDim.x)
         lds_w[t] = wfrag[t];
     __syncthreads();
 
     const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
     const int grp = lane >> 4, col = lane & 15;
     const int64_t P = g.paths;
-    const int64_t base = (int64_t)blockIdx.x * kMfmaPathsPerBlock + (int64_t)wv * kNT * 16;
+    const int64_t base = begin + ((int64_t)blockIdx.x * (blockDim.x / kWave) + wv) * kNT * 16;
     int64_t path[kNT];
     bool live[kNT];
 #pragma unroll
@@ -345,19 +349,19 @@ __global__ __launch_bounds__(kMfmaBlock) void ref_paths_mfma_kernel(const MfmaGr
 // Portfolio semantics: dates e = 0 .. ndates-1 every 50 steps from t = 0. At each date the
 // curve goes to curves[e][tenor][path] and the log bank account dt sum_{n < 50 e} f_n(0)
 // to logb[e][path]; the block's row 51 (left-point sum of the short rate) extends it.
-// A workgroup of WAVES waves of NT N-tiles simulates path group blockIdx.x of WAVES x NT x
-// 16 paths; kPersist: then every gridDim.x-th group after it, with a grid smaller than the
+// A workgroup of WAVES waves (0: as launched) of NT N-tiles simulates path group blockIdx.x of
+// WAVES x NT x 16 paths from `begin` on; kPersist: then every gridDim.x-th group after it, with a grid smaller than the
 // number of groups (the block map is staged in LDS once per workgroup). The group loop is
 // a separate instantiation: around the date loop it costs the compiler's allocation
 // about 50 VGPRs.
 template <bool kStore, int NT, int WAVES, bool kPersist>
-__global__ __launch_bounds__(WAVES * kWave) void pf_paths_mfma_kernel(const MfmaGrid g,
+__global__ __launch_bounds__((WAVES ? WAVES : max_waves(NT)) * kWave) void pf_paths_mfma_kernel(const MfmaGrid g,
                                                                   const u4_t* __restrict__ wfrag,
                                                                   float* __restrict__ curves,
                                                                   double* __restrict__ logb,
-                                                                  float* __restrict__ zs)
+                                                                  float* __restrict__ zs, int64_t begin)
 {
-    constexpr int kThreads = WAVES * kWave, kGroup = WAVES * NT * 16;
+    const int kThreads = WAVES ? WAVES * kWave : blockDim.x, kGroup = kThreads / kWave * NT * 16;
     extern __shared__ u4_t lds_w[];
     for (int t = threadIdx.x; t < kMfmaPfFragElems / 8; t += kThreads) lds_w[t] = wfrag[t];
     __syncthreads();
@@ -365,12 +369,12 @@ __global__ __launch_bounds__(WAVES * kWave) void pf_paths_mfma_kernel(const Mfma
     const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
     const int grp = lane >> 4, col = lane & 15;
     const int64_t P = g.paths;
-    const int64_t groups = (P + kGroup - 1) / kGroup;
+    const int64_t groups = (P - begin + kGroup - 1) / kGroup;
     // row 51 (the short-rate sum) is register 4 * 3 + 3 of lane group 0
     constexpr int kSumReg = 4 * (kTenors / 16) + kTenors % 4;
     const bool sum_lane = grp == (kTenors % 16) / 4;
     for (int64_t gi = blockIdx.x; gi < groups; gi += kPersist ? gridDim.x : groups) {
-        const int64_t base = gi * kGroup + (int64_t)wv * NT * 16;
+        const int64_t base = begin + gi * kGroup + (int64_t)wv * NT * 16;
         int64_t path[NT];
         bool live[NT];
         float fin[NT][16];
@@ -422,41 +426,224 @@ __global__ __launch_bounds__(WAVES * kWave) void pf_paths_mfma_kernel(const Mfma
     }
 }
 
-// The portfolio path kernel's instantiated launch shapes {N-tiles per wave, waves}: {2, 8},
-// {2, 12}, {1, 12}, {1, 16} (64 KB of block map in LDS;
-// 2 N-tiles take about 164 VGPRs, at most 3 waves per SIMD).
-constexpr int kPathShapes = 4;
-template <bool kStore, bool kPersist>
-struct PfPathsKernels {
-    template <int NT, int W>
-    static const void* fn() { return (const void*)pf_paths_mfma_kernel<kStore, NT, W, kPersist>; }
-};
+// One N-tile over the waves of a workgroup, for path counts that leave the chip idle with a
+// wave per N-tile: wave m holds the fragments of M-tile m in registers and computes its rows,
+// waves 0 .. 4 make one shock chunk (two calls) each for the block to come, and the split
+// operands pass through LDS, double-buffered (one barrier per block). Products are added in
+// the order of mfma_block, so the results are bit-identical. Bound by the block's chain (two
+// calls, then 27 products of which 20 follow one another, then the barrier): 1.3 us a block
+// against 3.8 where a wave has the tile to itself and 9 with two tiles to a wave. Four waves
+// per SIMD, so that three workgroups share a CU (12288 paths on the chip).
+constexpr int kShockChunks = kMfmaChunks - 2;
+__host__ __device__ constexpr int tile_waves(int mt) { return mt < kShockChunks ? kShockChunks : mt; }
 
+template <bool kPf, bool kStore, int MT>
+__global__ __launch_bounds__(tile_waves(MT) * kWave, kStore && MT > 4 ? 3 : 4) void tile_paths_mfma_kernel(
+    const MfmaGrid g, const u4_t* __restrict__ wfrag, double* __restrict__ num_x,
+    double* __restrict__ num_y, float* __restrict__ curves, double* __restrict__ logb,
+    float* __restrict__ zs, int64_t begin)
+{
+    constexpr bool kTwoAcc = kPf || MT <= 5;   // as the kernels above
+    __shared__ u4_t s_z[2][kShockChunks][2][kWave];
+    __shared__ u4_t s_c[2][2][kMfmaParts][kWave];
+    const int lane = threadIdx.x & (kWave - 1), wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int grp = lane >> 4, col = lane & 15;
+    const int64_t P = g.paths;
+    const int64_t path = begin + (int64_t)blockIdx.x * 16 + col;
+    const bool live = path < P;
+    const bool mine = wv < MT;   // the wave has an M-tile
+
+    u4_t w[kMfmaTileFrags];
+#pragma unroll
+    for (int f = 0; f < kMfmaTileFrags; ++f)
+        w[f] = wfrag[((mine ? wv : 0) * kMfmaTileFrags + f) * kWave + lane];
+    // rows 16 wv + 4 grp + r: the curve (tiles 0..3), Kahan (A, C) of the integrals (3 ..)
+    float fin[4], Ak[4], Ck[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int R = 16 * wv + 4 * grp + r, j = R - kTenors;
+        fin[r] = R < kTenors ? g.spot[R < kTenors ? R : 0] : 0.f;
+        const double a0 = (j >= 0 && j < kTenors) ? g.a0[j >= 0 && j < kTenors ? j : 0] : 0.0;
+        Ak[r] = (float)a0;
+        Ck[r] = (float)((double)Ak[r] - a0);
+    }
+    double lnB = 0.0;
+
+    // shock chunk wv of block b: values 8 wv .. 8 wv + 7 of the lane group's stream
+    auto shocks = [&](int b, int buf) {
+        if (wv >= kShockChunks) return;
+        float z[8];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            float v[4];
+            stream_call(g.seed_lo, g.seed_hi, (uint32_t)(g.path0 + path), (uint32_t)b, (uint32_t)grp,
+                        (uint32_t)(2 * wv + c), v);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) z[4 * c + e] = v[e];
+        }
+        if (wv == kShockChunks - 1) {
+            // the last quad: steps 48 and 49, then the drift's 1 in factor 0
+            constexpr int q0 = 3 * (kMfmaQuads - 1) - 8 * (kShockChunks - 1);
+            const int t = 4 * (kMfmaQuads - 1) + grp;
+            const bool in = t < kMfmaStride;
+            z[q0] = in ? z[q0] : (t == kMfmaStride ? 1.f : 0.f);
+            z[q0 + 1] = in ? z[q0 + 1] : 0.f;
+            z[q0 + 2] = in ? z[q0 + 2] : 0.f;
+            z[q0 + 3] = 0.f;
+        }
+        if constexpr (kStore) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int v = 8 * wv + i, t = 4 * (v / 3) + grp;
+                if (v < 3 * kMfmaQuads && t < kMfmaStride && live)
+                    zs[((int64_t)(b * kMfmaStride + t) * 3 + v % 3) * P + path] = z[i];
+            }
+        }
+        const SplitH8 sp = split8h(z);
+        s_z[buf][wv][0][lane] = sp.h;
+        s_z[buf][wv][1][lane] = sp.l;
+    };
+    auto pass_curve = [&](int buf) {
+        if (wv >= 4) return;
+        const float x[8] = {fin[0], fin[1], fin[2], fin[3], 0.f, 0.f, 0.f, 0.f};
+        const Split8 sp = split8(x);
+        const u4_t part[3] = {sp.h, sp.m, sp.l};
+#pragma unroll
+        for (int q = 0; q < kMfmaParts; ++q) {
+            u2_t* o = reinterpret_cast<u2_t*>(&s_c[buf][wv / 2][q][lane]) + (wv & 1);
+            *o = u2_t{part[q][0], part[q][1]};
+        }
+    };
+    auto record_date = [&](int e) {   // portfolio
+        if (live && wv < 4) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int R = 16 * wv + 4 * grp + r;
+                if (R < kTenors) curves[((int64_t)e * kTenors + R) * P + path] = fin[r] * g.down;
+            }
+            if (wv == kTenors / 16 && grp == (kTenors % 16) / 4) logb[(int64_t)e * P + path] = lnB;
+        }
+    };
+
+    const int b0 = kPf ? 0 : 1, nb = g.ndates - 1;   // blocks b0 .. b0 + nb - 1
+    if constexpr (kPf) record_date(0);
+    else if (wv == 0 && grp == 0 && live) {
+        num_x[P + path] = (double)(g.spot[1] * g.down);
+        num_y[P + path] = exp(-g.a0[1] * g.dt);
+    }
+    if (nb > 0) {
+        shocks(b0, 0);
+        pass_curve(0);
+    }
+    __syncthreads();
+    for (int i = 0; i < nb; ++i) {
+        const int buf = i & 1;
+        if (i + 1 < nb) shocks(b0 + i + 1, buf ^ 1);
+        if (mine) {
+            f4_t acc = {0.f, 0.f, 0.f, 0.f}, acc2 = acc;
+            auto small = [&](auto fn, u4_t a, u4_t x) {
+                if constexpr (kTwoAcc) acc2 = fn(a, x, acc2);
+                else acc = fn(a, x, acc);
+            };
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                if (c < 1 || !mfma_chunk_zero(wv, c, false)) {
+                    const u4_t h = s_c[buf][c][0][lane], m = s_c[buf][c][1][lane], l = s_c[buf][c][2][lane];
+                    const u4_t* a = w + 3 * c;
+                    acc = mfma_bf16(a[0], h, acc);
+                    small(mfma_bf16, a[0], m);
+                    small(mfma_bf16, a[1], h);
+                    small(mfma_bf16, a[0], l);
+                    small(mfma_bf16, a[2], h);
+                    small(mfma_bf16, a[1], m);
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < kShockChunks; ++c) {
+                const u4_t h = s_z[buf][c][0][lane], l = s_z[buf][c][1][lane];
+                const u4_t* a = w + 6 + 2 * c;
+                acc = mfma_f16(a[0], h, acc);
+                small(mfma_f16, a[0], l);
+                small(mfma_f16, a[1], h);
+            }
+            if constexpr (kTwoAcc) acc += acc2;
+            if constexpr (!kPf) {
+                if (wv >= 3) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float y = acc[r] - Ck[r];
+                        const float tt = Ak[r] + y;
+                        Ck[r] = (tt - Ak[r]) - y;
+                        Ak[r] = tt;
+                    }
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) fin[r] = acc[r];
+            if constexpr (kPf) {
+                lnB += (double)fin[kTenors % 4] * g.dt;
+                record_date(i + 1);
+            } else {
+                // slot b + 1: x = curve row b + 1, integral = row 51 + b + 1
+                const int slot = b0 + i + 1, Ra = kTenors + slot;
+                if (wv == slot / 16 && grp == (slot % 16) / 4 && live) {
+                    float xv = fin[0];
+#pragma unroll
+                    for (int r = 1; r < 4; ++r) xv = r == slot % 4 ? fin[r] : xv;
+                    num_x[(int64_t)slot * P + path] = (double)(xv * g.down);
+                }
+                if (wv == Ra / 16 && grp == (Ra % 16) / 4 && live) {
+                    float av = Ak[0], cv = Ck[0];
+#pragma unroll
+                    for (int r = 1; r < 4; ++r) {
+                        av = r == Ra % 4 ? Ak[r] : av;
+                        cv = r == Ra % 4 ? Ck[r] : cv;
+                    }
+                    num_y[(int64_t)slot * P + path] = exp(-((double)av - (double)cv) * g.dt);
+                }
+            }
+            if (i + 1 < nb) pass_curve(buf ^ 1);
+        }
+        __syncthreads();
+    }
+}
+
+// Launch shapes {N-tiles per wave, waves per workgroup}: {1, up to 12} and {2, up to 8} by path
+// count (next_path_launch); a tuned portfolio plan's {2, 12}, {1, 12}, {1, 16} and persistent
+// {2, 8} (64 KB of block map in LDS).
+constexpr int kPathKernels = 16 + 11;
 hipError_t mfma_kernels_prepare()
 {
-    const void* fns[8 + 4 * kPathShapes] = {
-        (const void*)ref_paths_mfma_kernel<false, 4>, (const void*)ref_paths_mfma_kernel<false, 5>,
-        (const void*)ref_paths_mfma_kernel<false, 6>, (const void*)ref_paths_mfma_kernel<false, 7>,
-        (const void*)ref_paths_mfma_kernel<true, 4>,  (const void*)ref_paths_mfma_kernel<true, 5>,
-        (const void*)ref_paths_mfma_kernel<true, 6>,  (const void*)ref_paths_mfma_kernel<true, 7>};
-    int lds[8 + 4 * kPathShapes];
-    for (int i = 0; i < 8; ++i) lds[i] = ref_mfma_lds_bytes(4 + i % 4);
-    int k = 8;
-    auto add = [&](const void* f) {
+    const void* fns[kPathKernels];
+    int lds[kPathKernels];
+    int k = 0;
+    auto add = [&](const void* f, int bytes) {
         fns[k] = f;
-        lds[k++] = 2 * kMfmaPfFragElems;
+        lds[k++] = bytes;
     };
-    auto add_shapes = [&](auto kernels) {
-        using K = decltype(kernels);
-        add(K::template fn<2, 8>());
-        add(K::template fn<2, 12>());
-        add(K::template fn<1, 12>());
-        add(K::template fn<1, 16>());
+    auto add_ref = [&](auto mt) {
+        constexpr int MT = decltype(mt)::value;
+        add((const void*)ref_paths_mfma_kernel<false, MT, 1>, ref_mfma_lds_bytes(MT));
+        add((const void*)ref_paths_mfma_kernel<true, MT, 1>, ref_mfma_lds_bytes(MT));
+        add((const void*)ref_paths_mfma_kernel<false, MT, 2>, ref_mfma_lds_bytes(MT));
+        add((const void*)ref_paths_mfma_kernel<true, MT, 2>, ref_mfma_lds_bytes(MT));
     };
-    add_shapes(PfPathsKernels<false, false>{});
-    add_shapes(PfPathsKernels<true, false>{});
-    add_shapes(PfPathsKernels<false, true>{});
-    add_shapes(PfPathsKernels<true, true>{});
+    add_ref(std::integral_constant<int, 4>{});
+    add_ref(std::integral_constant<int, 5>{});
+    add_ref(std::integral_constant<int, 6>{});
+    add_ref(std::integral_constant<int, 7>{});
+    auto add_pf = [&](const void* f) { add(f, 2 * kMfmaPfFragElems); };
+    add_pf((const void*)pf_paths_mfma_kernel<false, 1, 0, false>);
+    add_pf((const void*)pf_paths_mfma_kernel<true, 1, 0, false>);
+    add_pf((const void*)pf_paths_mfma_kernel<false, 2, 0, false>);
+    add_pf((const void*)pf_paths_mfma_kernel<true, 2, 0, false>);
+    add_pf((const void*)pf_paths_mfma_kernel<false, 2, 12, false>);
+    add_pf((const void*)pf_paths_mfma_kernel<false, 1, 12, false>);
+    add_pf((const void*)pf_paths_mfma_kernel<false, 1, 16, false>);
+    add_pf((const void*)pf_paths_mfma_kernel<false, 2, 8, true>);
+    add_pf((const void*)pf_paths_mfma_kernel<false, 2, 12, true>);
+    add_pf((const void*)pf_paths_mfma_kernel<false, 1, 12, true>);
+    add_pf((const void*)pf_paths_mfma_kernel<false, 1, 16, true>);
     for (int i = 0; i < k; ++i) {
         const hipError_t e = hipFuncSetAttribute(fns[i], hipFuncAttributeMaxDynamicSharedMemorySize, lds[i]);
         if (e != hipSuccess) return e;
@@ -464,18 +651,86 @@ hipError_t mfma_kernels_prepare()
     return hipSuccess;
 }
 
+// The launch that takes the paths from `begin` on (one after another to the last path; every
+// path's result is the same whichever takes it): N-tiles per wave (0: a workgroup per
+// N-tile), waves per workgroup, workgroups. t = N-tiles per CU of the paths left. Path kernel
+// times in us by t, {workgroup per N-tile / 1 per wave / 2 per wave}, 10y reference (4
+// M-tiles) | 25y (7) | portfolio over 30y:
+//   t = 1   33 / 79 / 181  |  74 / 233 / 550 |  77 / 183 / 506
+//   t = 3   64 / 79 / 181  | 152 / 237 / 557 | 152 / 185 / 510
+//   t = 4   99 / 82 / 123  | 192 / 242 / 380 | 245 / 190 / 340
+//   t = 5  104 / 114 / 126 | 235 / 330 / 389 | 252 / 295 / 343
+//   t = 8  172 / 113 / 126 | 402 / 333 / 387 | 422 / 300 / 345
+//   t = 12 237 / 152 / 190 | 580 / 436 / 566 | 613 / 402 / 518
+//   t = 16 312 / 282 / 193 | 746 / 832 / 567 | 806 / 745 / 530
+// so: a workgroup per N-tile where its three to a CU (or a fuller second turn) serve, then a
+// wave each, then two to a wave. Past 16, whole turns of the chip go to {2, 8} and the rest
+// by the same rule (100000 paths: 368 -> 337 us, 25y 1114 -> 977; 80000: 366 -> 268).
+struct PathLaunch {
+    int tiles, waves;
+    int64_t blocks;
+    int64_t paths() const { return blocks * (tiles ? 16 * tiles * waves : 16); }
+};
+constexpr int kCus = 256;
+
+static PathLaunch next_path_launch(int64_t left, int mt)
+{
+    const int64_t n = (left + 15) / 16, t = (n + kCus - 1) / kCus;
+    if (t > 16) return {2, 8, left / (256 * kCus) * kCus};
+    if (t > 12) {
+        const int w = (int)(t + 1) / 2;
+        return {2, w, (n + 2 * w - 1) / (2 * w)};
+    }
+    if (t > 3 && t != 5 && (t != 4 || mt < 7)) return {1, (int)t, (n + t - 1) / t};
+    return {0, tile_waves(mt), n};
+}
+
+template <bool kStore, int MT>
+static void launch_ref_tiles(const MfmaGrid& g, const u4_t* w, double* nx, double* ny, float* zs,
+                             hipStream_t st)
+{
+    const size_t lds = (size_t)ref_mfma_lds_bytes(MT);
+    for (int64_t begin = 0; begin < g.paths;) {
+        const PathLaunch l = next_path_launch(g.paths - begin, MT);
+        const dim3 grid((unsigned)l.blocks), block((unsigned)(l.waves * kWave));
+        if (l.tiles == 2)
+            ref_paths_mfma_kernel<kStore, MT, 2><<<grid, block, lds, st>>>(g, w, nx, ny, zs, begin);
+        else if (l.tiles == 1)
+            ref_paths_mfma_kernel<kStore, MT, 1><<<grid, block, lds, st>>>(g, w, nx, ny, zs, begin);
+        else
+            tile_paths_mfma_kernel<false, kStore, MT>
+                <<<grid, block, 0, st>>>(g, w, nx, ny, nullptr, nullptr, zs, begin);
+        begin += l.paths();
+    }
+}
+
+template <bool kStore>
+static void launch_pf_tiles(const MfmaGrid& g, const u4_t* w, float* curves, double* logb, float* zs,
+                            hipStream_t st)
+{
+    const size_t lds = 2 * kMfmaPfFragElems;
+    for (int64_t begin = 0; begin < g.paths;) {
+        const PathLaunch l = next_path_launch(g.paths - begin, kMfmaPfMTiles);
+        const dim3 grid((unsigned)l.blocks), block((unsigned)(l.waves * kWave));
+        if (l.tiles == 2)
+            pf_paths_mfma_kernel<kStore, 2, 0, false><<<grid, block, lds, st>>>(g, w, curves, logb, zs, begin);
+        else if (l.tiles == 1)
+            pf_paths_mfma_kernel<kStore, 1, 0, false><<<grid, block, lds, st>>>(g, w, curves, logb, zs, begin);
+        else
+            tile_paths_mfma_kernel<true, kStore, kMfmaPfMTiles>
+                <<<grid, block, 0, st>>>(g, w, nullptr, nullptr, curves, logb, zs, begin);
+        begin += l.paths();
+    }
+}
+
 hipError_t launch_ref_paths_mfma(const MfmaGrid& g, const uint16_t* wfrag, double* nx, double* ny,
                                  float* zs, hipStream_t st)
 {
     if (g.ndates < 1 || g.ndates > kTenors - 1) return hipErrorInvalidValue;
-    const dim3 grid((unsigned)((g.paths + kMfmaPathsPerBlock - 1) / kMfmaPathsPerBlock));
     const u4_t* w = reinterpret_cast<const u4_t*>(wfrag);
-    const int mt = ref_mfma_tiles(g.ndates);
-    const size_t lds = (size_t)ref_mfma_lds_bytes(mt);
 #define HJM_REF_LAUNCH(MT)                                                                      \
-    (zs ? ref_paths_mfma_kernel<true, MT><<<grid, kMfmaBlock, lds, st>>>(g, w, nx, ny, zs)      \
-        : ref_paths_mfma_kernel<false, MT><<<grid, kMfmaBlock, lds, st>>>(g, w, nx, ny, zs))
-    switch (mt) {
+    (zs ? launch_ref_tiles<true, MT>(g, w, nx, ny, zs, st) : launch_ref_tiles<false, MT>(g, w, nx, ny, zs, st))
+    switch (ref_mfma_tiles(g.ndates)) {
     case 4: HJM_REF_LAUNCH(4); break;
     case 5: HJM_REF_LAUNCH(5); break;
     case 6: HJM_REF_LAUNCH(6); break;
@@ -490,20 +745,21 @@ bool pf_path_shape_ok(int tiles, int waves)
     return (tiles == 2 && (waves == 8 || waves == 12)) || (tiles == 1 && (waves == 12 || waves == 16));
 }
 
-template <bool kStore, bool kPersist>
+// a tuned plan's shape (no stored shocks: those plans have the default one)
+template <bool kPersist>
 static hipError_t launch_pf_paths_shape(const MfmaGrid& g, const u4_t* w, float* curves, double* logb,
-                                        float* zs, int tiles, int waves, int64_t blocks, hipStream_t st)
+                                        int tiles, int waves, int64_t blocks, hipStream_t st)
 {
     const dim3 grid((unsigned)blocks), block((unsigned)(waves * kWave));
     const size_t lds = 2 * kMfmaPfFragElems;
-    if (tiles == 2 && waves == 8)
-        pf_paths_mfma_kernel<kStore, 2, 8, kPersist><<<grid, block, lds, st>>>(g, w, curves, logb, zs);
-    else if (tiles == 2 && waves == 12)
-        pf_paths_mfma_kernel<kStore, 2, 12, kPersist><<<grid, block, lds, st>>>(g, w, curves, logb, zs);
+    if (tiles == 2 && waves == 12)
+        pf_paths_mfma_kernel<false, 2, 12, kPersist><<<grid, block, lds, st>>>(g, w, curves, logb, nullptr, 0);
     else if (tiles == 1 && waves == 12)
-        pf_paths_mfma_kernel<kStore, 1, 12, kPersist><<<grid, block, lds, st>>>(g, w, curves, logb, zs);
+        pf_paths_mfma_kernel<false, 1, 12, kPersist><<<grid, block, lds, st>>>(g, w, curves, logb, nullptr, 0);
     else if (tiles == 1 && waves == 16)
-        pf_paths_mfma_kernel<kStore, 1, 16, kPersist><<<grid, block, lds, st>>>(g, w, curves, logb, zs);
+        pf_paths_mfma_kernel<false, 1, 16, kPersist><<<grid, block, lds, st>>>(g, w, curves, logb, nullptr, 0);
+    else if (tiles == 2 && waves == 8 && kPersist)   // otherwise by path count
+        pf_paths_mfma_kernel<false, 2, 8, true><<<grid, block, lds, st>>>(g, w, curves, logb, nullptr, 0);
     else
         return hipErrorInvalidValue;
     return hipGetLastError();
@@ -517,13 +773,14 @@ hipError_t launch_pf_paths_mfma(const MfmaGrid& g, const uint16_t* wfrag, float*
     const u4_t* w = reinterpret_cast<const u4_t*>(wfrag);
     const int64_t group = (int64_t)waves * tiles * 16;
     const int64_t groups = (g.paths + group - 1) / group;
-    if (shape.max_blocks > 0 && shape.max_blocks < groups) {
-        const int64_t b = shape.max_blocks;
-        return zs ? launch_pf_paths_shape<true, true>(g, w, curves, logb, zs, tiles, waves, b, st)
-                  : launch_pf_paths_shape<false, true>(g, w, curves, logb, zs, tiles, waves, b, st);
+    const bool persist = shape.max_blocks > 0 && shape.max_blocks < groups;
+    if (zs || (tiles == 2 && waves == 8 && !persist)) {
+        if (zs) launch_pf_tiles<true>(g, w, curves, logb, zs, st);
+        else launch_pf_tiles<false>(g, w, curves, logb, zs, st);
+        return hipGetLastError();
     }
-    return zs ? launch_pf_paths_shape<true, false>(g, w, curves, logb, zs, tiles, waves, groups, st)
-              : launch_pf_paths_shape<false, false>(g, w, curves, logb, zs, tiles, waves, groups, st);
+    return persist ? launch_pf_paths_shape<true>(g, w, curves, logb, tiles, waves, shape.max_blocks, st)
+                   : launch_pf_paths_shape<false>(g, w, curves, logb, tiles, waves, groups, st);
 }
 
 // Netting-set exposures of one date on the matrix cores (FP32 plans):
@@ -650,7 +907,6 @@ __device__ __forceinline__ float exposure_of(float V, float disc) { return V > 0
 // filter (or null): value only the M-tiles holding a set whose PFE row at this date the
 // counting pass left unresolved (bracket_row_resolved false for rank fk and fcap
 // candidate slots); a workgroup with none returns at once.
-//
 // Bound by the exposure stores and the matrix products about equally (128 sets x 61 dates x
 // 1048576 paths are up to 33 GB and 12 products a bond chunk) once nothing in the M-tile loop
 // waits for the stores: a global load there would, since loads and stores share one counter,

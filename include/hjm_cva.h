@@ -232,7 +232,8 @@ typedef struct {
                                 set and date (1..32; 0: 32); a row with more is valued again,
                                 whole, for its selection (exact either way) */
     int32_t path_tiles;     /* matrix-core path kernel: N-tiles of 16 paths per wave, and */
-    int32_t path_waves;     /* waves per workgroup: {2, 8} (default), {2, 12}, {1, 12}, {1, 16} */
+    int32_t path_waves;     /* waves per workgroup: {2, 8} (default; fewer paths than
+                               fill the chip take smaller shapes), {2, 12}, {1, 12}, {1, 16} */
     int32_t value_tiles;    /* matrix-core valuation: N-tiles per wave, 2 (default) or 4 */
     int32_t value_waves;    /* waves per workgroup, 4 or 8 (default) */
     int32_t value_stage;    /* M-tiles (16 sets) of -gamma staged in LDS at a time, 1..8
