@@ -112,7 +112,10 @@ hipError_t launch_adjoint_fragments(const double* coef, int nsets, int ndates, u
 hipError_t launch_clear_matured(const int* kmax, int rows, int64_t paths, void* ex, int elem_bytes,
                                 hipStream_t st);
 
-// Portfolio semantics.
+// Portfolio semantics. FP64 with in-kernel normals: several lanes per path, the same for every
+// block and grid.
+hipError_t launch_pf_paths_lanes(const RefStepConsts<double>& k, const PfGrid& g, double* curves,
+                                 double* logb, hipStream_t st);
 hipError_t launch_pf_paths_f64(const RefStepConsts<double>& k, const PfGrid& g, const double* normals,
                                double* curves, double* logb, int block, int grid, hipStream_t st);
 hipError_t launch_pf_paths_f32(const RefStepConsts<float>& k, const PfGrid& g, const double* normals,

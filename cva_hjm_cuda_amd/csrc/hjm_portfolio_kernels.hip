@@ -282,10 +282,12 @@ __device__ __forceinline__ void pf_stats_rows(const PfValueParams v,
             for (int k = 0; k < kStatPerThread; ++k)
                 dst[k] = __builtin_nontemporal_load(row + i0 + (int64_t)k * kBlock);
         } else {
+            // without branches, which would wait for each load before the next
 #pragma unroll
             for (int k = 0; k < kStatPerThread; ++k) {
                 const int64_t i = i0 + (int64_t)k * kBlock;
-                dst[k] = i < P ? __builtin_nontemporal_load(row + i) : (Real)0;
+                const Real x = __builtin_nontemporal_load(row + (i < P ? i : P - 1));
+                dst[k] = i < P ? x : (Real)0;
             }
         }
     };
@@ -442,6 +444,71 @@ __global__ __launch_bounds__(kBlock) void pf_stats_kernel(const PfValueParams v,
     pf_stats_rows<Real, kCount>(v, exposures, w, partials, sel, cand, cap, stage, flush, lo_parts);
 }
 
+// The same without the counting for little work, which is bound by a workgroup's chain of
+// dates: one path per thread, kPlainDates dates' exposures loaded and reduced side by side.
+// By paths x sets up to 3 x 2^17; us here / with 8 paths per thread, FP32 | FP64 rows:
+//   11 x 1000 17 / 48 | 18 / 54; 11 x 10007 19 / 50 | 21 / 69; 32 x 10007 32 / 51 | 42 / 77;
+//   32 x 16384 44 / 38 | 60 / 50; 128 x 10007 97 / 78 | 141 / 132
+// (8 paths per thread took 76 | 69 at 11 x 10007 while loads past the last path were branched
+// around, each waiting for the one before).
+constexpr int64_t kPlainWork = 3 << 17;
+constexpr int kPlainDates = 8;
+
+template <typename Real>
+__global__ __launch_bounds__(kBlock) void pf_stats_plain_kernel(const PfValueParams v,
+                                                                const Real* __restrict__ exposures,
+                                                                const double* __restrict__ w,
+                                                                double* __restrict__ partials)
+{
+    constexpr int kWaves = kBlock / kWave;
+    __shared__ double red[kWaves][kMaxDates + 2];
+    __shared__ double s_w[kMaxDates];
+    const int gset = blockIdx.y, nd = v.ndates;
+    const int64_t P = v.paths, i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    for (int e = threadIdx.x; e < nd; e += kBlock) {
+        s_w[e] = w[(int64_t)gset * nd + e];
+    }
+    __syncthreads();
+    const bool live = i < P;
+    const Real* col = exposures + (int64_t)gset * P + (live ? i : 0);
+    double cva = 0.0;
+    for (int e0 = 0; e0 < nd; e0 += kPlainDates) {
+        Real x[kPlainDates];
+        double s[kPlainDates];
+        // without branches, which would wait for one date before the next is asked for; a
+        // matured set's row holds zeros
+#pragma unroll
+        for (int k = 0; k < kPlainDates; ++k) {
+            const int e = e0 + k < nd ? e0 + k : nd - 1;
+            x[k] = __builtin_nontemporal_load(col + (int64_t)e * v.nsets * P);
+        }
+#pragma unroll
+        for (int k = 0; k < kPlainDates; ++k) {
+            s[k] = live ? (double)x[k] : 0.0;
+            cva += (e0 + k < nd ? s_w[e0 + k] : 0.0) * s[k];
+        }
+#pragma unroll
+        for (int k = 0; k < kPlainDates; ++k) s[k] = wave_sum(s[k]);
+#pragma unroll
+        for (int k = 0; k < kPlainDates; ++k)
+            if (lane == 0 && e0 + k < nd) red[wave][e0 + k] = s[k];
+    }
+    const double c1 = wave_sum(cva), c2 = wave_sum(cva * cva);
+    if (lane == 0) {
+        red[wave][nd] = c1;
+        red[wave][nd + 1] = c2;
+    }
+    __syncthreads();
+    const int ncol = nd + 2;
+    for (int c = threadIdx.x; c < ncol; c += kBlock) {
+        double t = 0.0;
+#pragma unroll
+        for (int ww = 0; ww < kWaves; ++ww) t += red[ww][c];
+        partials[((int64_t)gset * gridDim.x + blockIdx.x) * ncol + c] = t;
+    }
+}
+
 // FP32 rows with the PFE counting: held to 80 VGPRs for 6 waves per SIMD, which it fits
 // without spills (it first spilled 20 bytes per lane there and was still faster: 7.87 ->
 // 7.63 ms at 1048576 paths x 61 dates x 128 sets). More waves have not paid: with FP32
@@ -508,9 +575,11 @@ static hipError_t pf_paths_launch(const RefStepConsts<Real>& k, const PfGrid& g,
 {
     if (block != 64 && block != 128 && block != 256) return hipErrorInvalidValue;
     if (grid <= 0) return hipErrorInvalidValue;
+    if constexpr (sizeof(Real) == sizeof(double))
+        if (!normals) return launch_pf_paths_lanes(k, g, curves, logb, st);
     if (normals)
         pf_paths_kernel<Real, true><<<grid, block, 0, st>>>(k, g, normals, curves, logb);
-    else
+    else if constexpr (sizeof(Real) == sizeof(float))
         pf_paths_kernel<Real, false><<<grid, block, (size_t)kGroupShocks * block * sizeof(float), st>>>(
             k, g, normals, curves, logb);
     return hipGetLastError();
@@ -569,7 +638,8 @@ static hipError_t pf_stats_launch(const PfValueParams& v, const Real* ex, const 
                                   double* partials, double* sums, void* selws, int64_t pfe_rank,
                                   uint32_t* lo_parts, hipStream_t st)
 {
-    const unsigned nb = (unsigned)((v.paths + kStatPaths - 1) / kStatPaths);
+    const int per = selws || v.paths * v.nsets > kPlainWork ? kStatPaths : kBlock;
+    const unsigned nb = (unsigned)((v.paths + per - 1) / per);
     const dim3 grid(nb, (unsigned)v.nsets);
     if (selws) {
         const BracketPlan bp = bracket_plan(v.paths, pfe_rank, (int)sizeof(Real));
@@ -591,9 +661,11 @@ static hipError_t pf_stats_launch(const PfValueParams& v, const Real* ex, const 
             const unsigned wgs = (unsigned)((rows + kBlock / kWave - 1) / (kBlock / kWave));
             sel_add_row_counts_kernel<<<wgs, kBlock, 0, st>>>(state, lo_parts, rows, (int)nb);
         }
-    } else {
+    } else if (per == kStatPaths) {
         pf_stats_kernel<Real, false><<<grid, kBlock, 0, st>>>(v, ex, w, partials, nullptr, nullptr, 0,
                                                              0, 0, nullptr);
+    } else {
+        pf_stats_plain_kernel<Real><<<grid, kBlock, 0, st>>>(v, ex, w, partials);
     }
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;

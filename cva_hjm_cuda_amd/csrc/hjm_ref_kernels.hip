@@ -209,11 +209,16 @@ __device__ __forceinline__ double from_next_lane(double v)
     return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
-template <int L>
-__global__ __launch_bounds__(kWave) void ref_paths_lanes_kernel(const RefStepConsts<double> k,
-                                                             const RefGrid g,
-                                                             double* __restrict__ num_x,
-                                                             double* __restrict__ num_y)
+// kPf: the portfolio's paths (pf_paths_kernel<double>, bit-identical): from t = 0, no discount
+// integrals, the curve and the log bank account at every date (g.a0 unused). Over 30 years in us,
+// one path per lane in brackets: 1000 paths 197 [3914], 10007 694 [3965], 65536 2199 [4006].
+template <int L, bool kPf>
+__global__ __launch_bounds__(kWave) void paths_lanes_kernel(const RefStepConsts<double> k,
+                                                         const RefGrid g,
+                                                         double* __restrict__ num_x,
+                                                         double* __restrict__ num_y,
+                                                         double* __restrict__ curves,
+                                                         double* __restrict__ logb)
 {
     using C = RefLanes<L>;
     constexpr int n = C::n;
@@ -234,7 +239,7 @@ __global__ __launch_bounds__(kWave) void ref_paths_lanes_kernel(const RefStepCon
         const bool on = j >= 0 && j < kTenors;
         const int jc = on ? j : 0;
         f[u] = on ? k.spot[jc] : 0.0;
-        A[u] = on ? g.a0[jc] : 0.0;
+        A[u] = on && !kPf ? g.a0[jc] : 0.0;
         m[u] = on ? k.ddt[jc] : 0.0;
         v0[u] = on ? k.v0[jc] : 0.0;
         v1[u] = on ? k.v1[jc] : 0.0;
@@ -244,13 +249,17 @@ __global__ __launch_bounds__(kWave) void ref_paths_lanes_kernel(const RefStepCon
     // the slot of tenor 50 (in the last lane the backward difference, elsewhere as any other)
     double cs = is_last ? -k.c : k.c, os = is_last ? k.opc : k.omc;
     asm volatile("" : "+v"(cv), "+v"(omc), "+v"(cs), "+v"(os));
-    if (live && sub == 0) {
-        num_x[P + i] = k.spot[1];
-        num_y[P + i] = exp(-g.a0[1] * g.dt);
+    double lnB = 0.0;   // tenor 0 is slot `pad` of a path's first lane
+    if constexpr (!kPf) {
+        if (live && sub == 0) {
+            num_x[P + i] = k.spot[1];
+            num_y[P + i] = exp(-g.a0[1] * g.dt);
+        }
     }
     // one Euler step with the shocks q[0..2] (times sqrt(dt))
     auto step = [&](const double* q) {
         const double y0 = q[0], y1 = q[1], y2 = q[2];
+        if constexpr (kPf) lnB += f[C::pad] * g.dt;
         const double fn = from_next_lane<L>(f[0]);
         constexpr int S = C::slot;
         const double fs = is_last ? f[S - 1] : (S + 1 < n ? f[S + 1 < n ? S + 1 : 0] : fn);
@@ -271,10 +280,22 @@ __global__ __launch_bounds__(kWave) void ref_paths_lanes_kernel(const RefStepCon
 #pragma unroll
             for (int u = u0; u < u0 + G && u < n; ++u) op_fma_inplace(f[u], u == S ? os : omc, t[u - u0]);
 #pragma unroll
-            for (int u = u0; u < u0 + G && u < n; ++u) op_add_inplace(A[u], f[u]);
+            for (int u = u0; u < u0 + G && u < n; ++u)
+                if constexpr (!kPf) op_add_inplace(A[u], f[u]);
         }
     };
-    for (int b = 1; b < g.ndates; ++b) {
+    for (int b = kPf ? 0 : 1; b < g.ndates; ++b) {
+        if constexpr (kPf) {
+            if (live) {
+#pragma unroll
+                for (int u = 0; u < n; ++u) {
+                    const int j = sub * n + u - C::pad;
+                    if (j >= 0 && j < kTenors) curves[((int64_t)b * kTenors + j) * P + i] = f[u];
+                }
+                if (sub == 0) logb[(int64_t)b * P + i] = lnB;
+            }
+            if (b + 1 == g.ndates) break;
+        }
         for (int s0 = 0; s0 < g.stride; s0 += C::chunk) {
             const int steps = min(C::chunk, g.stride - s0);
             // steps [s0, s0 + 32) are quads 8 k .. 8 k + 7 of every class: calls 6 k .. 6 k + 5
@@ -298,17 +319,19 @@ __global__ __launch_bounds__(kWave) void ref_paths_lanes_kernel(const RefStepCon
             }
             for (int cls = 0; st < steps; ++st, ++cls) step(q + cls * C::cls);
         }
-        const int at = b + 1 + C::pad, owner = at / n, slot = at % n;
-        double x = f[0], a = A[0];
+        if constexpr (!kPf) {
+            const int at = b + 1 + C::pad, owner = at / n, slot = at % n;
+            double x = f[0], a = A[0];
 #pragma unroll
-        for (int u = 1; u < n; ++u)
-            if (u == slot) {
-                x = f[u];
-                a = A[u];
+            for (int u = 1; u < n; ++u)
+                if (u == slot) {
+                    x = f[u];
+                    a = A[u];
+                }
+            if (live && sub == owner) {
+                num_x[(int64_t)(b + 1) * P + i] = x;
+                num_y[(int64_t)(b + 1) * P + i] = exp(-a * g.dt);
             }
-        if (live && sub == owner) {
-            num_x[(int64_t)(b + 1) * P + i] = x;
-            num_y[(int64_t)(b + 1) * P + i] = exp(-a * g.dt);
         }
     }
 }
@@ -442,31 +465,52 @@ __global__ __launch_bounds__(kBlock) void normals_kernel(uint32_t seed_lo, uint3
 }
 
 // ---- launchers -------------------------------------------------------------------
-template <int L>
-static hipError_t launch_paths_lanes(const RefStepConsts<double>& k, const RefGrid& g, double* nx,
-                                     double* ny, hipStream_t st)
+template <int L, bool kPf>
+static hipError_t launch_lanes(const RefStepConsts<double>& k, const RefGrid& g, double* nx, double* ny,
+                               double* curves, double* logb, hipStream_t st)
 {
     constexpr int paths = RefLanes<L>::paths;
-    ref_paths_lanes_kernel<L><<<(unsigned)((g.paths + paths - 1) / paths), kWave, 0, st>>>(k, g, nx, ny);
+    paths_lanes_kernel<L, kPf><<<(unsigned)((g.paths + paths - 1) / paths), kWave, 0, st>>>(
+        k, g, nx, ny, curves, logb);
     return hipGetLastError();
+}
+
+// In-kernel normals: L lanes per path. Fewer paths take more lanes each until the chip's
+// 1024 SIMDs hold a wave: L = 32 up to 2048 paths, 16 up to 4096, 8 up to 24576 (three
+// waves per SIMD), and 4 beyond, which wastes the fewest slots (52 for 51 tenors) but
+// holds 246 VGPRs. Path kernel in us at L = 32 / 16 / 8 / 4, one path per lane in brackets:
+//   1000 x 5y 38 / 49 / 63 / 101 [716]; 4096 x 10y 105 / 100 / 134 / 204 [1495];
+//   5000 x 25y 344 / 365 / 333 / 520 [3958]; 20000 x 10y 404 / 354 / 335 / 383 [1513];
+//   30000 x 10y 574 / 510 / 421 / 383 [1517]; 131072 x 10y 2207 / 1820 / 1538 / 1404 [1841].
+template <bool kPf>
+static hipError_t launch_paths_lanes(const RefStepConsts<double>& k, const RefGrid& g, double* nx,
+                                     double* ny, double* curves, double* logb, hipStream_t st)
+{
+    if (g.paths <= 2048) return launch_lanes<32, kPf>(k, g, nx, ny, curves, logb, st);
+    if (g.paths <= 4096) return launch_lanes<16, kPf>(k, g, nx, ny, curves, logb, st);
+    if (g.paths <= 24576) return launch_lanes<8, kPf>(k, g, nx, ny, curves, logb, st);
+    return launch_lanes<4, kPf>(k, g, nx, ny, curves, logb, st);
+}
+
+hipError_t launch_pf_paths_lanes(const RefStepConsts<double>& k, const PfGrid& g, double* curves,
+                                 double* logb, hipStream_t st)
+{
+    RefGrid r{};
+    r.stride = g.stride;
+    r.nsteps = g.nsteps;
+    r.ndates = g.ndates_m1 + 1;
+    r.paths = g.paths;
+    r.path0 = g.path0;
+    r.seed_lo = g.seed_lo;
+    r.seed_hi = g.seed_hi;
+    r.dt = g.dt;
+    return launch_paths_lanes<true>(k, r, nullptr, nullptr, curves, logb, st);
 }
 
 hipError_t launch_ref_paths_f64(const RefStepConsts<double>& k, const RefGrid& g,
                                 const double* normals, double* nx, double* ny, hipStream_t st)
 {
-    // In-kernel normals: L lanes per path. Fewer paths take more lanes each until the chip's
-    // 1024 SIMDs hold a wave: L = 32 up to 2048 paths, 16 up to 4096, 8 up to 24576 (three
-    // waves per SIMD), and 4 beyond, which wastes the fewest slots (52 for 51 tenors) but
-    // holds 246 VGPRs. Path kernel in us at L = 32 / 16 / 8 / 4, one path per lane in brackets:
-    //   1000 x 5y 38 / 49 / 63 / 101 [716]; 4096 x 10y 105 / 100 / 134 / 204 [1495];
-    //   5000 x 25y 344 / 365 / 333 / 520 [3958]; 20000 x 10y 404 / 354 / 335 / 383 [1513];
-    //   30000 x 10y 574 / 510 / 421 / 383 [1517]; 131072 x 10y 2207 / 1820 / 1538 / 1404 [1841].
-    if (!normals) {
-        if (g.paths <= 2048) return launch_paths_lanes<32>(k, g, nx, ny, st);
-        if (g.paths <= 4096) return launch_paths_lanes<16>(k, g, nx, ny, st);
-        if (g.paths <= 24576) return launch_paths_lanes<8>(k, g, nx, ny, st);
-        return launch_paths_lanes<4>(k, g, nx, ny, st);
-    }
+    if (!normals) return launch_paths_lanes<false>(k, g, nx, ny, nullptr, nullptr, st);
     ref_paths_kernel<double, false, true><<<(unsigned)((g.paths + kBlock - 1) / kBlock), kBlock, 0, st>>>(
         k, g, normals, nx, ny);
     return hipGetLastError();
