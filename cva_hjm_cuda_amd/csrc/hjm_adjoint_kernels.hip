@@ -90,14 +90,15 @@ struct AdjGrid {
     float c, omc, opc, sqrt_dt;
 };
 
-// Runs whose dates are not 50 steps apart, host normals, and the fallback of the matrix-core
-// sweep (hjm_adjoint_mfma.hip). kSrc: 0 regenerate the in-kernel normals, 1 host-supplied
-// FP64 [path][step][3].
+// FP64 runs, dates not 50 steps apart, host normals, and the fallback of the matrix-core sweep
+// (hjm_adjoint_mfma.hip). kSrc: 0 regenerate the in-kernel normals, 1 host-supplied FP64
+// [path][step][3], 2 the forward pass's stored FP32 normals [step][3][path].
 // partials[workgroup][5 * 51]: loading gradients g0, g1, g2 (tenor-major within each),
 // sum over blocks of lambda_e, and d J / d spot, each summed over the workgroup's paths.
 template <int kSrc>
 __global__ __launch_bounds__(kBlock) void ref_adjoint_kernel(const AdjGrid g,
                                                              const double* __restrict__ normals,
+                                                             const float* __restrict__ zs,
                                                              const float* __restrict__ gx,
                                                              const float* __restrict__ gA,
                                                              double* __restrict__ partials)
@@ -180,6 +181,18 @@ __global__ __launch_bounds__(kBlock) void ref_adjoint_kernel(const AdjGrid g,
     };
 
     const int S = g.stride;
+    constexpr int kPre = 5;   // stored normals: steps read ahead (the stride is a multiple)
+    float zq[kPre][3];
+    auto loadz = [&](int n, float (&d)[3]) {
+        const float* q = zs + (int64_t)n * 3 * P + ic;
+        d[0] = q[0];
+        d[1] = q[P];
+        d[2] = q[2 * P];
+    };
+    if constexpr (kSrc == 2) {
+#pragma unroll
+        for (int u = 0; u < kPre; ++u) loadz((g.ndates - 1) * S + S - 1 - u, zq[u]);
+    }
     const int whole = S / kGroupSteps * kGroupSteps;
     for (int b = g.ndates - 1; b >= 1; --b) {
         // exposure date n = b * stride records slot b + 1 (tenor b + 1 >= 2)
@@ -195,26 +208,38 @@ __global__ __launch_bounds__(kBlock) void ref_adjoint_kernel(const AdjGrid g,
         }
 #pragma unroll
         for (int k = 0; k < kHalfSlots; ++k) lacc[k][threadIdx.x] += lam[k];
-        for (int s = S - 1; s >= 0; --s) {
-            const int n = b * S + s;  // global step index of this Euler step
-            if constexpr (kSrc == 1) {
-                const double* q = normals + (ic * g.nsteps + n) * 3;
-                step((float)q[0], (float)q[1], (float)q[2]);
-            } else {
-                // groups of 16 steps staged in LDS, entered from their last step
-                Normals3 z;
-                if (s < whole) {
-                    if ((s & (kGroupSteps - 1)) == kGroupSteps - 1) {
-                        __syncthreads();   // the previous group's reads are done
-                        fill_group_half(g.seed_lo, g.seed_hi, pid, (uint32_t)b, s / kGroupSteps,
-                                        half, col, kAdjPaths);
-                        __syncthreads();   // both lanes' calls are in the column
-                    }
-                    z = group_step(col, kAdjPaths, s);
-                } else {
-                    z = step_normals(g.seed_lo, g.seed_hi, pid, (uint32_t)n, (uint32_t)S);
+        if constexpr (kSrc == 2) {
+            for (int s0 = S - 1; s0 >= 0; s0 -= kPre) {
+#pragma unroll
+                for (int u = 0; u < kPre; ++u) {
+                    const float a0 = zq[u][0], a1 = zq[u][1], a2 = zq[u][2];
+                    const int nn = b * S + s0 - kPre - u;   // same slot of the next chunk
+                    if (nn >= S) loadz(nn, zq[u]);
+                    step(a0, a1, a2);
                 }
-                step(z.z0, z.z1, z.z2);
+            }
+        } else {
+            for (int s = S - 1; s >= 0; --s) {
+                const int n = b * S + s;  // global step index of this Euler step
+                if constexpr (kSrc == 1) {
+                    const double* q = normals + (ic * g.nsteps + n) * 3;
+                    step((float)q[0], (float)q[1], (float)q[2]);
+                } else {
+                    // groups of 16 steps staged in LDS, entered from their last step
+                    Normals3 z;
+                    if (s < whole) {
+                        if ((s & (kGroupSteps - 1)) == kGroupSteps - 1) {
+                            __syncthreads();   // the previous group's reads are done
+                            fill_group_half(g.seed_lo, g.seed_hi, pid, (uint32_t)b, s / kGroupSteps,
+                                            half, col, kAdjPaths);
+                            __syncthreads();   // both lanes' calls are in the column
+                        }
+                        z = group_step(col, kAdjPaths, s);
+                    } else {
+                        z = step_normals(g.seed_lo, g.seed_hi, pid, (uint32_t)n, (uint32_t)S);
+                    }
+                    step(z.z0, z.z1, z.z2);
+                }
             }
         }
         // FP32 partials cover at most two blocks, then go to the FP64 accumulators
@@ -263,7 +288,8 @@ hipError_t launch_ref_adjoint_seed(const ExposureParams& e, double dt, const dou
 int64_t ref_adjoint_blocks(int64_t paths) { return (paths + kAdjPaths - 1) / kAdjPaths; }
 
 hipError_t launch_ref_adjoint(const RefGrid& rg, double c, double sqrt_dt, const double* normals,
-                              const float* gx, const float* gA, double* partials, hipStream_t st)
+                              const float* zs, const float* gx, const float* gA, double* partials,
+                              hipStream_t st)
 {
     AdjGrid g{};
     g.stride = rg.stride;
@@ -278,10 +304,13 @@ hipError_t launch_ref_adjoint(const RefGrid& rg, double c, double sqrt_dt, const
     g.opc = 1.0f + g.c;
     g.sqrt_dt = (float)sqrt_dt;
     const dim3 grid((unsigned)ref_adjoint_blocks(rg.paths));
+    if (zs && rg.stride % 5 != 0) return hipErrorInvalidValue;  // stored-normal read-ahead
     if (normals)
-        ref_adjoint_kernel<1><<<grid, kBlock, 0, st>>>(g, normals, gx, gA, partials);
+        ref_adjoint_kernel<1><<<grid, kBlock, 0, st>>>(g, normals, zs, gx, gA, partials);
+    else if (zs)
+        ref_adjoint_kernel<2><<<grid, kBlock, 0, st>>>(g, normals, zs, gx, gA, partials);
     else
-        ref_adjoint_kernel<0><<<grid, kBlock, 0, st>>>(g, normals, gx, gA, partials);
+        ref_adjoint_kernel<0><<<grid, kBlock, 0, st>>>(g, normals, zs, gx, gA, partials);
     return hipGetLastError();
 }
 

@@ -502,9 +502,11 @@ int hjm_cva_greeks_reference(const hjm_market* market, const hjm_swap* swap,
     sg.hi = D - 1;
     sg.lo = 1;
     sg.paths = P;
-    // the matrix-core sweep for the path kernels' 50-step blocks with in-kernel normals; the
-    // VALU sweep for the others, and where the matrix sweep's buffers cannot be had
-    const bool matrix = S == kMfmaStride && !p->host_rng && D > 1 &&
+    // the matrix-core sweep for FP32 runs of the path kernels' 50-step blocks with in-kernel
+    // normals; the VALU sweep for the others, and where the matrix sweep's buffers cannot be had.
+    // (Both sweep in FP32: FP64 runs keep the VALU sweep's sums, from which the matrix sweep's
+    // differ by that sweep's own rounding, up to 1e-5, more than FP64 results may move.)
+    const bool matrix = cfg->precision != HJM_FP64 && S == kMfmaStride && !p->host_rng && D > 1 &&
                         c.sweep.take(sg, false, cc, p->grid.nsteps, c.zs != nullptr, st) == HJM_OK;
     HJM_TRY(plan_launch(p, false, c.zs));
     HJM_HIP(hipEventRecord(e0, st), HJM_ERR_DEVICE);
@@ -518,7 +520,7 @@ int hjm_cva_greeks_reference(const hjm_market* market, const hjm_swap* swap,
         HJM_TRY(dev_alloc(&c.sums, kOut + kTenors));  // then the per-slot sums of gA
         // gA summed over the paths at every slot (the drift gradient's mu terms)
         HJM_HIP(launch_column_sum(c.sap, p->nblocks, kTenors, c.sums + kOut, st), HJM_ERR_LAUNCH);
-        HJM_HIP(launch_ref_adjoint(p->grid, cc, sqrt(dt), p->d_normals, c.gx, c.gA, c.part, st),
+        HJM_HIP(launch_ref_adjoint(p->grid, cc, sqrt(dt), p->d_normals, c.zs, c.gx, c.gA, c.part, st),
                 HJM_ERR_LAUNCH);
         HJM_HIP(launch_column_sum(c.part, nb, kOut, c.sums, st), HJM_ERR_LAUNCH);
         HJM_HIP(hipMemcpyAsync(sums, c.sums, sizeof(double) * (kOut + kTenors), hipMemcpyDeviceToHost, st),

@@ -659,9 +659,11 @@ int hjm_portfolio_cva_greeks(const hjm_market* market, const hjm_portfolio* port
     sg.lo = 0;
     sg.dt = (float)dt;
     sg.paths = P;
-    // the matrix-core sweep for the path kernels' 50-step blocks with in-kernel normals; the
-    // VALU sweep for the others, and where the matrix sweep's buffers cannot be had
-    const bool matrix = p->grid.stride == kMfmaStride && !p->d_normals &&
+    // the matrix-core sweep for FP32 runs of the path kernels' 50-step blocks with in-kernel
+    // normals; the VALU sweep for the others, and where the matrix sweep's buffers cannot be had.
+    // (Both sweep in FP32: FP64 runs keep the VALU sweep's sums, from which the matrix sweep's
+    // differ by that sweep's own rounding, up to 1e-5, more than FP64 results may move.)
+    const bool matrix = !f64 && p->grid.stride == kMfmaStride && !p->d_normals &&
                         c.sweep.take(sg, true, cc, p->grid.nsteps, c.zs != nullptr, st) == HJM_OK;
     HJM_TRY(pplan_enqueue(p, true, c.zs));
     HJM_HIP(hipEventRecord(e0, st), HJM_ERR_DEVICE);
@@ -680,7 +682,7 @@ int hjm_portfolio_cva_greeks(const hjm_market* market, const hjm_portfolio* port
         HJM_TRY(c.sweep.run(sg, true, c.zs, p->grid.nsteps, cfg.seed, cfg.path_offset, c.gbar, c.beta, swept, st));
     } else {
         HJM_TRY(dev_alloc(&c.part, (size_t)nb * kOut));
-        HJM_HIP(launch_pf_adjoint(p->grid, cc, p->d_normals, c.gbar, c.beta, c.part, st), HJM_ERR_LAUNCH);
+        HJM_HIP(launch_pf_adjoint(p->grid, cc, p->d_normals, c.zs, c.gbar, c.beta, c.part, st), HJM_ERR_LAUNCH);
         HJM_HIP(launch_column_sum(c.part, nb, kOut, c.sums, st), HJM_ERR_LAUNCH);
     }
     HJM_HIP(hipEventRecord(e1, st), HJM_ERR_DEVICE);

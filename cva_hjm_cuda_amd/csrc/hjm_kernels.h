@@ -67,12 +67,14 @@ hipError_t launch_pf_paths_mfma(const MfmaGrid& g, const uint16_t* wfrag, float*
 hipError_t launch_ref_adjoint_seed(const ExposureParams& e, double dt, const double* nx,
                                    const double* ny, float* gx, float* gA, double* sa_partials,
                                    hipStream_t st);
-// One-pass VALU sweep, two lanes per path. normals: host FP64 [path][step][3], or null:
-// regenerate. partials: [ref_adjoint_blocks(paths)][5 * 51]
+// One-pass VALU sweep, two lanes per path. normals: host FP64 [path][step][3]; zs: the
+// forward's stored FP32 normals [step][3][path]; both null: regenerate. partials:
+// [ref_adjoint_blocks(paths)][5 * 51]
 // (loading gradients of factors 0, 1, 2, sum of the block-end adjoints, d J / d spot).
 int64_t ref_adjoint_blocks(int64_t paths);
 hipError_t launch_ref_adjoint(const RefGrid& rg, double c, double sqrt_dt, const double* normals,
-                              const float* gx, const float* gA, double* partials, hipStream_t st);
+                              const float* zs, const float* gx, const float* gA, double* partials,
+                              hipStream_t st);
 
 // The reverse sweep on the matrix cores (50 steps per date, in-kernel normals; hjm_adjoint_mfma.hip).
 struct SweepGrid {
@@ -188,8 +190,8 @@ hipError_t launch_pf_adjoint_seed_mfma(const PfValueParams& v, const float* curv
 // One-pass sweep, two lanes per path; partials [pf_adjoint_blocks(paths)][5 * 51] as the
 // reference sweep's.
 int64_t pf_adjoint_blocks(int64_t paths);
-hipError_t launch_pf_adjoint(const PfGrid& g, double c, const double* normals, const float* gbar,
-                             const float* beta, double* partials, hipStream_t st);
+hipError_t launch_pf_adjoint(const PfGrid& g, double c, const double* normals, const float* zs,
+                             const float* gbar, const float* beta, double* partials, hipStream_t st);
 
 // The reference's own GPU design (baseline form).
 hipError_t launch_blockwise_paths(const RefStepConsts<double>& k, const RefGrid& g, int block_index,

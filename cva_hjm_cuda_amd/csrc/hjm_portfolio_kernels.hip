@@ -831,13 +831,14 @@ __global__ __launch_bounds__(kBlock) void pf_adjoint_seed_kernel(const PfValuePa
 // of step n, lambda <- T^T lambda + mu e_0 (mu = dt sum of beta of later dates), + gbar_e at
 // the date steps. The drift gradient comes from the block-end adjoints lambda_e, summed
 // over dates and paths (the host applies sum_{k<S} (T^T)^k to them and the mu terms).
-// Runs whose dates are not 50 steps apart, host normals, and the fallback of the matrix-core
-// sweep (hjm_adjoint_mfma.hip). kSrc: 0 regenerate the in-kernel normals, 1 host-supplied
-// FP64 [path][step][3].
+// FP64 runs, dates not 50 steps apart, host normals, and the fallback of the matrix-core sweep
+// (hjm_adjoint_mfma.hip). kSrc: 0 regenerate the in-kernel normals, 1 host-supplied FP64
+// [path][step][3], 2 the forward pass's stored FP32 normals [step][3][path].
 // partials[workgroup][5 * 51]: g0, g1, g2, sum of lambda_e, d J / d spot.
 template <int kSrc>
 __global__ __launch_bounds__(kBlock) void pf_adjoint_kernel(const PfGrid g, float c,
                                                             const double* __restrict__ normals,
+                                                            const float* __restrict__ zs,
                                                             const float* __restrict__ gbar,
                                                             const float* __restrict__ beta,
                                                             double* __restrict__ partials)
@@ -922,30 +923,54 @@ __global__ __launch_bounds__(kBlock) void pf_adjoint_kernel(const PfGrid g, floa
     };
 
     const int S = g.stride;
+    constexpr int kPre = 5;
+    float zq[kPre][3];
+    auto loadz = [&](int n, float (&d)[3]) {
+        const float* q = zs + (int64_t)n * 3 * P + ic;
+        d[0] = q[0];
+        d[1] = q[P];
+        d[2] = q[2 * P];
+    };
+    if constexpr (kSrc == 2) {
+#pragma unroll
+        for (int u = 0; u < kPre; ++u) loadz(E * S - 1 - u, zq[u]);
+    }
     const int whole = S / kGroupSteps * kGroupSteps;
     for (int e = E - 1; e >= 0; --e) {
         mu += (active && !upper) ? dtf * beta[(int64_t)(e + 1) * P + ic] : 0.f;
 #pragma unroll
         for (int k = 0; k < kHalfSlots; ++k) lacc[k][threadIdx.x] += lam[k];
-        for (int s = S - 1; s >= 0; --s) {
-            const int n = e * S + s;
-            if constexpr (kSrc == 1) {
-                const double* q = normals + (ic * g.nsteps + n) * 3;
-                step((float)q[0], (float)q[1], (float)q[2]);
-            } else {
-                Normals3 z;
-                if (s < whole) {
-                    if ((s & (kGroupSteps - 1)) == kGroupSteps - 1) {
-                        __syncthreads();
-                        fill_group_half(g.seed_lo, g.seed_hi, pid, (uint32_t)e, s / kGroupSteps,
-                                        half, col, kAdjPaths);
-                        __syncthreads();
-                    }
-                    z = group_step(col, kAdjPaths, s);
-                } else {
-                    z = step_normals(g.seed_lo, g.seed_hi, pid, (uint32_t)n, (uint32_t)S);
+        if constexpr (kSrc == 2) {
+            for (int s0 = S - 1; s0 >= 0; s0 -= kPre) {
+#pragma unroll
+                for (int u = 0; u < kPre; ++u) {
+                    const float a0 = zq[u][0], a1 = zq[u][1], a2 = zq[u][2];
+                    const int nn = e * S + s0 - kPre - u;
+                    if (nn >= 0) loadz(nn, zq[u]);
+                    step(a0, a1, a2);
                 }
-                step(z.z0, z.z1, z.z2);
+            }
+        } else {
+            for (int s = S - 1; s >= 0; --s) {
+                const int n = e * S + s;
+                if constexpr (kSrc == 1) {
+                    const double* q = normals + (ic * g.nsteps + n) * 3;
+                    step((float)q[0], (float)q[1], (float)q[2]);
+                } else {
+                    Normals3 z;
+                    if (s < whole) {
+                        if ((s & (kGroupSteps - 1)) == kGroupSteps - 1) {
+                            __syncthreads();
+                            fill_group_half(g.seed_lo, g.seed_hi, pid, (uint32_t)e, s / kGroupSteps,
+                                            half, col, kAdjPaths);
+                            __syncthreads();
+                        }
+                        z = group_step(col, kAdjPaths, s);
+                    } else {
+                        z = step_normals(g.seed_lo, g.seed_hi, pid, (uint32_t)n, (uint32_t)S);
+                    }
+                    step(z.z0, z.z1, z.z2);
+                }
             }
         }
         // date e: the valuation at e depends on f(n_e)
@@ -997,15 +1022,18 @@ hipError_t launch_pf_adjoint_seed_f64(const PfValueParams& v, const double* curv
 
 int64_t pf_adjoint_blocks(int64_t paths) { return (paths + kAdjPaths - 1) / kAdjPaths; }
 
-hipError_t launch_pf_adjoint(const PfGrid& g, double c, const double* normals, const float* gbar,
-                             const float* beta, double* partials, hipStream_t st)
+hipError_t launch_pf_adjoint(const PfGrid& g, double c, const double* normals, const float* zs,
+                             const float* gbar, const float* beta, double* partials, hipStream_t st)
 {
     const dim3 grid((unsigned)pf_adjoint_blocks(g.paths));
     const float cf = step_ratio_f32(c);  // 1 - cf, 1 + cf exact, as in the FP32 forward
+    if (zs && g.stride % 5 != 0) return hipErrorInvalidValue;  // stored-normal read-ahead
     if (normals)
-        pf_adjoint_kernel<1><<<grid, kBlock, 0, st>>>(g, cf, normals, gbar, beta, partials);
+        pf_adjoint_kernel<1><<<grid, kBlock, 0, st>>>(g, cf, normals, zs, gbar, beta, partials);
+    else if (zs)
+        pf_adjoint_kernel<2><<<grid, kBlock, 0, st>>>(g, cf, normals, zs, gbar, beta, partials);
     else
-        pf_adjoint_kernel<0><<<grid, kBlock, 0, st>>>(g, cf, normals, gbar, beta, partials);
+        pf_adjoint_kernel<0><<<grid, kBlock, 0, st>>>(g, cf, normals, zs, gbar, beta, partials);
     return hipGetLastError();
 }
 

@@ -2,10 +2,10 @@
 
 Sizes where it changes shape: paths that leave its waves, 32-path units and workgroups partly
 filled; horizons on both sides of every number of row tiles (mu rows to dates 15, 31, 47, 50)
-and the one-block horizon. The forward is FP64, so that both sides see the same states; the
-seeds and the sweep are FP32 with the paths' terms of either sign: 2e-5 of a gradient's scale
-covers sqrt(25 y x 50 steps) roundings of 2^-24 with a factor of ten. Shocks stored by the
-forward or regenerated in bounded chunks give the same sums bit for bit.
+and the one-block horizon. Seeds and sweep are FP32 with the paths' terms of
+either sign: 2e-5 of a gradient's scale covers sqrt(25 y x 50 steps) roundings of 2^-24 with a
+factor of ten. Shocks stored by the forward or regenerated in bounded chunks give the same
+sums bit for bit. FP64 runs keep the one-pass VALU sweep, with or without stored shocks.
 """
 import numpy as np
 import pytest
@@ -31,12 +31,14 @@ def test_reference_sweep_matches_oracle(oracle, paths, expiry):
                                                   1e6, 0.02, expiry, 0.5, 0.01, z, w)
     swap = hjm.InterestRateSwap(1e6, 0.02, expiry)
     a = hjm.cva_greeks(m, swap, paths, seed=5, precision=hjm.FP64)
-    b = hjm.cva_greeks(m, swap, paths, seed=5, precision=hjm.FP64, path_kernel=hjm.KERNEL_MATRIX)
-    c = hjm.cva_greeks(m, swap, paths, seed=5, precision=hjm.FP64, path_kernel=hjm.KERNEL_MATRIX,
-                       regenerate_normals=True)
-    assert a.stored_normals_bytes == c.stored_normals_bytes == 0 < b.stored_normals_bytes
-    for g in (a, b):
+    d = hjm.cva_greeks(m, swap, paths, seed=5, precision=hjm.FP64, path_kernel=hjm.KERNEL_MATRIX)
+    b = hjm.cva_greeks(m, swap, paths, seed=5, precision=hjm.FP32_KAHAN)
+    c = hjm.cva_greeks(m, swap, paths, seed=5, precision=hjm.FP32_KAHAN, regenerate_normals=True)
+    assert a.stored_normals_bytes == c.stored_normals_bytes == 0
+    assert b.stored_normals_bytes > 0 and d.stored_normals_bytes > 0
+    for g in (a, d):
         assert g.cva == pytest.approx(cva, rel=1e-9)
+    for g in (a, b, d):
         _close((g.d_spot, g.d_vol, g.d_drift), (ds, dv, dm))
     for x, y in ((b.d_spot, c.d_spot), (b.d_vol, c.d_vol), (b.d_drift, c.d_drift)):
         assert np.array_equal(x, y)
@@ -53,8 +55,10 @@ def test_portfolio_sweep_matches_oracle(oracle, paths, horizon):
     cva, ds, dv, dm = oracle.portfolio_cva_greeks(m.spot_rates, m.drifts, m.volatilities, horizon, 0.5,
                                                   0.01, z, pf, w)
     a = hjm.portfolio_cva_greeks(m, pf, paths, horizon=horizon, seed=5, precision=hjm.FP64)
-    b = hjm.portfolio_cva_greeks(m, pf, paths, horizon=horizon, seed=5, precision=hjm.FP64,
+    d = hjm.portfolio_cva_greeks(m, pf, paths, horizon=horizon, seed=5, precision=hjm.FP64,
                                  path_kernel=hjm.KERNEL_MATRIX)
-    for g in (a, b):
+    b = hjm.portfolio_cva_greeks(m, pf, paths, horizon=horizon, seed=5, precision=hjm.FP32_KAHAN)
+    for g in (a, d):
         assert g.cva == pytest.approx(cva, rel=1e-8)
+    for g in (a, b, d):
         _close((g.d_spot, g.d_vol, g.d_drift), (ds, dv, dm))
