@@ -18,7 +18,7 @@ SOURCES = ["hjm_capi.hip", "hjm_ref_kernels.hip", "hjm_baseline_kernels.hip",
            "hjm_adjoint_kernels.hip", "hjm_portfolio_kernels.hip",
            "hjm_capi_portfolio.hip", "hjm_mfma_kernels.hip", "hjm_mfma64_kernels.hip", "hjm_calibration.hip",
            "hjm_select_kernels.hip", "hjm_adjoint_mfma.hip", "hjm_book_kernels.hip",
-           "hjm_pool.hip"]
+           "hjm_map_kernels.hip", "hjm_pool.hip"]
 ARCH = os.environ.get("HJM_OFFLOAD_ARCH", "gfx950")
 
 HIPCC_FLAGS = [

@@ -202,7 +202,6 @@ int plan_init(hjm_plan p, const hjm_market* market, const hjm_swap* swap, const 
         if (wsb) HJM_TRY(dev_alloc(&p->d_selws, wsb));
     }
     // host copies of the block map, kept until the stream is synchronised below
-    std::vector<uint16_t> wf;
     std::vector<double> wf64;
     if (p->use_mfma) {
         int scale = 0;
@@ -216,12 +215,11 @@ int plan_init(hjm_plan p, const hjm_market* market, const hjm_swap* swap, const 
                     HJM_ERR_DEVICE);
         } else {
             HJM_HIP(mfma_kernels_prepare(), HJM_ERR_DEVICE);
-            scale = build_mfma_block_map(market->spot_rates, market->drifts, market->volatilities,
-                                         cfg->dt, swap->dtau, ref_mfma_tiles(D), wf);
-            HJM_TRY(dev_alloc(&p->d_wfrag, wf.size()));
-            HJM_HIP(hipMemcpyAsync(p->d_wfrag, wf.data(), wf.size() * sizeof(uint16_t),
-                                   hipMemcpyHostToDevice, p->stream),
-                    HJM_ERR_DEVICE);
+            const BlockMapParams bm = block_map_params(market->spot_rates, market->drifts, market->volatilities,
+                                                       cfg->dt, swap->dtau, ref_mfma_tiles(D));
+            scale = bm.scale;
+            HJM_TRY(dev_alloc(&p->d_wfrag, block_map_elems(bm.mtiles)));
+            HJM_HIP(launch_block_map(bm, false, p->d_wfrag, p->stream), HJM_ERR_LAUNCH);
         }
         MfmaGrid& mg = p->mg;
         mg.ndates = D;

@@ -299,12 +299,11 @@ int pplan_init(hjm_portfolio_plan p, const hjm_market* market, const hjm_portfol
     int scale = 0;
     if (p->use_mfma) {
         HJM_HIP(mfma_kernels_prepare(), HJM_ERR_DEVICE);
-        std::vector<uint16_t> wf;
-        scale = build_mfma_block_map(market->spot_rates, market->drifts, market->volatilities, cfg->dt,
-                                     pf->dtau, kMfmaPfMTiles, wf, MfmaMap::kPortfolio);
-        HJM_TRY(dev_alloc(&p->d_wfrag, wf.size()));
-        HJM_HIP(hipMemcpy(p->d_wfrag, wf.data(), wf.size() * sizeof(uint16_t), hipMemcpyHostToDevice),
-                HJM_ERR_DEVICE);
+        const BlockMapParams bm = block_map_params(market->spot_rates, market->drifts, market->volatilities,
+                                                   cfg->dt, pf->dtau, kMfmaPfMTiles, MfmaMap::kPortfolio);
+        scale = bm.scale;
+        HJM_TRY(dev_alloc(&p->d_wfrag, block_map_elems(bm.mtiles)));
+        HJM_HIP(launch_block_map(bm, true, p->d_wfrag, p->stream), HJM_ERR_LAUNCH);
     }
     if (p->use_mfma64) {
         HJM_HIP(mfma64_kernels_prepare(), HJM_ERR_DEVICE);

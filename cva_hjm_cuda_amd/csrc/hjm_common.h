@@ -55,7 +55,7 @@ struct RefGrid {
 };
 
 // Matrix-core path kernels (50-step blocks). The FP32 kernels hold the curve and the
-// integrals times 2^k (build_mfma_block_map): spot and a0 carry that factor, dt its inverse,
+// integrals times 2^k (block_map_params): spot and a0 carry that factor, dt its inverse,
 // and `down` = 2^-k scales the curve values that leave the kernel; all of it exact.
 struct MfmaGrid {
     int ndates;

@@ -76,6 +76,12 @@ hipError_t launch_ref_adjoint(const RefGrid& rg, double c, double sqrt_dt, const
                               const float* zs, const float* gx, const float* gA, double* partials,
                               hipStream_t st);
 
+// The block map's fragments of an FP32 matrix plan, block_map_elems(prm.mtiles) elements; the
+// reverse sweep's map and tables (hjm_map_kernels.hip).
+struct BlockMapParams;
+hipError_t launch_block_map(const BlockMapParams& prm, bool pf, uint16_t* frag, hipStream_t st);
+hipError_t launch_sweep_map(double c, bool pf, uint16_t* frag, float* ptab, hipStream_t st);
+
 // The reverse sweep on the matrix cores (50 steps per date, in-kernel normals; hjm_adjoint_mfma.hip).
 struct SweepGrid {
     int hi, lo;               // blocks hi .. lo, swept downwards

@@ -192,7 +192,7 @@ inline std::vector<double> mfma_block_map_dense(const double* drift, const doubl
 }
 
 // bf16 bits of x rounded to nearest (ties to even); x finite.
-inline uint16_t bf16_rne(double x)
+__host__ __device__ inline uint16_t bf16_rne(double x)
 {
     const float f = (float)x;
     uint32_t u;
@@ -201,7 +201,7 @@ inline uint16_t bf16_rne(double x)
     return (uint16_t)(u >> 16);
 }
 
-inline double bf16_value(uint16_t b)
+__host__ __device__ inline double bf16_value(uint16_t b)
 {
     const uint32_t u = (uint32_t)b << 16;
     float f;
@@ -210,7 +210,7 @@ inline double bf16_value(uint16_t b)
 }
 
 // fp16 bits of x rounded to nearest (ties to even); |x| < 65504
-inline uint16_t fp16_rne(float x)
+__host__ __device__ inline uint16_t fp16_rne(float x)
 {
     uint32_t u;
     memcpy(&u, &x, 4);
@@ -224,7 +224,7 @@ inline uint16_t fp16_rne(float x)
     return (uint16_t)(sign | ((u >> 13) - (112u << 10)));
 }
 
-inline double fp16_value(uint16_t h)
+__host__ __device__ inline double fp16_value(uint16_t h)
 {
     const uint32_t e = (h >> 10) & 31u, m = h & 1023u;
     if (!e) return ((h & 0x8000u) ? -0x1p-24 : 0x1p-24) * m;
@@ -234,54 +234,81 @@ inline double fp16_value(uint16_t h)
     return (double)f;
 }
 
-// Fragments of W in the kernel's A-operand order: the curve columns as three bf16 parts, the
-// shock columns (and the drift constant's) times 2^k as two fp16 parts rounded to nearest.
-// Returns k: the power of two that brings the largest shock entry to [2^12, 2^13), where
-// both parts of every entry within 2^-26 of it are normal fp16 numbers (without the scale
-// the entries, 1e-4 .. 1e-2, would leave their low parts to subnormals). The kernels hold the
-// curve and the integrals times 2^k too, so both kinds of products share an accumulator;
-// k is also bounded by the curve's size (max |spot| 2^k <= 2^40), and 0 without shocks.
-// mtiles: the M-tiles built (the reference kernel's live ones).
-inline int build_mfma_block_map(const double* spot, const double* drift, const double* vols, double dt,
-                                double dtau, int mtiles, std::vector<uint16_t>& frag,
-                                MfmaMap map = MfmaMap::kReference)
+// The block map's fragments (block_map_kernel) in the path kernel's A-operand order: row 16 m +
+// lane % 16 and column 32 c + 8 (lane / 16) + i of fragment mfma_frag(m, c, part); the curve
+// columns as three bf16 parts, the shock columns (and the drift constant's) times 2^k as two
+// fp16 parts rounded to nearest.
+struct BlockMapParams {
+    double c, up;            // dt / dtau, 2^k
+    double vec[4][kTenors];  // loadings times sqrt(dt), drift times dt
+    int mtiles;              // the M-tiles built (the reference kernel's live ones)
+    int scale;               // k
+};
+
+// k is the power of two that brings the largest shock entry to [2^12, 2^13), where both parts
+// of every entry within 2^-26 of it are normal fp16 numbers (without the scale the entries,
+// 1e-4 .. 1e-2, would leave their low parts to subnormals). The kernels hold the curve and
+// the integrals times 2^k too, so both kinds of products share an accumulator; k is also
+// bounded by the curve's size (max |spot| 2^k <= 2^40), and 0 without shocks.
+inline BlockMapParams block_map_params(const double* spot, const double* drift, const double* vols, double dt,
+                                       double dtau, int mtiles, MfmaMap map = MfmaMap::kReference)
 {
     const bool pf = map == MfmaMap::kPortfolio;
-    const int rows = pf ? kTenors + 1 : 2 * kTenors;
-    const std::vector<double> W = mfma_block_map_dense(drift, vols, dt, dtau, map);
-    double top = 0.0, curve = 0.0;
-    for (int row = 0; row < rows; ++row)
-        for (int k = 64; k < kMfmaK; ++k) top = std::max(top, fabs(W[(size_t)row * kMfmaK + k]));
-    for (int j = 0; j < kTenors; ++j) curve = std::max(curve, fabs(spot[j]));
-    int scale = 0;
-    if (top > 0.0) {
-        scale = std::max(-120, std::min(120, 12 - ilogb(top)));
-        if (curve > 0.0) scale = std::min(scale, std::max(12 - ilogb(top) - 40, 39 - ilogb(curve)));
+    constexpr int n = kTenors;
+    BlockMapParams p{};
+    p.c = dt / dtau;
+    p.mtiles = mtiles;
+    const double sq = sqrt(dt), c = p.c;
+    for (int j = 0; j < n; ++j) {
+        for (int f = 0; f < 3; ++f) p.vec[f][j] = sq * vols[f * n + j];
+        p.vec[3][j] = drift[j] * dt;
     }
-    const double up = ldexp(1.0, scale);
-    frag.assign((size_t)mtiles * kMfmaTileFrags * kWave * 8, 0);
-    for (int m = 0; m < mtiles; ++m)
-        for (int c = 0; c < kMfmaChunks; ++c)
-            for (int l = 0; l < kWave; ++l)
-                for (int i = 0; i < 8; ++i) {
-                    const int row = 16 * m + l % 16, k = 32 * c + 8 * (l / 16) + i;
-                    const double w = row < rows ? W[(size_t)row * kMfmaK + k] : 0.0;
-                    uint16_t parts[3] = {0, 0, 0};
-                    if (c < 2) {
-                        parts[0] = bf16_rne(w);
-                        const double r1 = w - bf16_value(parts[0]);
-                        parts[1] = bf16_rne(r1);
-                        parts[2] = bf16_rne(r1 - bf16_value(parts[1]));
-                    } else {
-                        parts[0] = fp16_rne((float)(w * up));
-                        parts[1] = fp16_rne((float)(w * up - fp16_value(parts[0])));
-                    }
-                    const int np = c < 2 ? kMfmaParts : kMfmaShockParts;
-                    for (int p = 0; p < np; ++p)
-                        frag[((size_t)mfma_frag(m, c, p) * kWave + l) * 8 + i] = parts[p];
+    // the largest entry of the shock columns and the drift's (mfma_block_map_dense's walks)
+    double tops[n] = {0.0}, left_top = 0.0, curve = 0.0;
+    auto raise = [&tops](const double* x) {
+        for (int j = 0; j < n; ++j) tops[j] = fabs(x[j]) > tops[j] ? fabs(x[j]) : tops[j];
+    };
+    for (int f = 0; f < 4; ++f) {
+        double u[n], t[n], acc[n] = {0.0}, cu[n] = {0.0}, ca[n] = {0.0}, cleft = 0.0;
+        memcpy(u, p.vec[f], sizeof u);
+        for (int q = 0; q < kMfmaStride; ++q) {
+            const double left = acc[0];
+            for (int j = 0; j < n; ++j) acc[j] += u[j];
+            if (f < 3) {
+                raise(u);
+                if (!pf) raise(acc);
+                left_top = fabs(left) > left_top ? fabs(left) : left_top;
+            } else {
+                for (int j = 0; j < n; ++j) {
+                    cu[j] += u[j];
+                    ca[j] += acc[j];
                 }
-    return scale;
+                cleft += left;
+            }
+            for (int j = 0; j < n - 1; ++j) t[j] = (1.0 - c) * u[j] + c * u[j + 1];
+            t[n - 1] = -c * u[n - 2] + (1.0 + c) * u[n - 1];
+            memcpy(u, t, sizeof u);
+        }
+        if (f == 3) {
+            raise(cu);
+            if (!pf) raise(ca);
+            left_top = fabs(cleft) > left_top ? fabs(cleft) : left_top;
+        }
+    }
+    double top = pf ? left_top : 0.0;
+    for (int j = 0; j < n; ++j) {
+        top = std::max(top, tops[j]);
+        curve = std::max(curve, fabs(spot[j]));
+    }
+    if (top > 0.0) {
+        p.scale = std::max(-120, std::min(120, 12 - ilogb(top)));
+        if (curve > 0.0) p.scale = std::min(p.scale, std::max(12 - ilogb(top) - 40, 39 - ilogb(curve)));
+    }
+    p.up = ldexp(1.0, p.scale);
+    return p;
 }
+
+inline size_t block_map_elems(int mtiles) { return (size_t)mtiles * kMfmaTileFrags * kWave * 8; }
 
 // The FP64 block map for v_mfma_f64_16x16x4f64 (ref_paths_mfma64_kernel). One instruction
 // takes K = 4 entries, one per lane group g = lane / 16, from one register of every lane;
@@ -370,40 +397,7 @@ constexpr int kMaxPfMTiles = (HJM_MAX_SETS + 15) / 16;
 // Tables of the matrix-core reverse sweep (hjm_adjoint_mfma.hip): the 64 x 64 map (T^T)^S as
 // [m][c][part][lane][8] bf16 parts of row 16 m + lane % 16 and the curve column of K slot (c,
 // lane / 16, i); and ptab[j][64], column j of sum_{q < S} (T^T)^q (portfolio: j = 0 only).
-inline void build_sweep_maps(double c, bool pf, std::vector<uint16_t>& frag, std::vector<float>& ptab)
-{
-    const int n = kTenors, S = kMfmaStride;
-    // rows of T^T: y_j = (1 - c) x_j + c x_{j-1}, y_49 also - c x_50, y_50 = (1 + c) x_50 + c x_49
-    std::vector<double> A((size_t)n * n, 0.0), next((size_t)n * n), B((size_t)n * n, 0.0);
-    for (int j = 0; j < n; ++j) A[(size_t)j * n + j] = 1.0;
-    for (int q = 0; q < S; ++q) {
-        for (size_t e = 0; e < A.size(); ++e) B[e] += A[e];
-        for (int j = 0; j < n; ++j)
-            for (int m = 0; m < n; ++m) {
-                double v = (j == n - 1 ? 1.0 + c : 1.0 - c) * A[(size_t)j * n + m];
-                if (j > 0) v += c * A[(size_t)(j - 1) * n + m];
-                if (j == n - 2) v -= c * A[(size_t)(n - 1) * n + m];
-                next[(size_t)j * n + m] = v;
-            }
-        A.swap(next);
-    }
-    ptab.assign((size_t)(pf ? 1 : n) * 64, 0.f);
-    for (int j = 0; j < (pf ? 1 : n); ++j)
-        for (int row = 0; row < n; ++row) ptab[(size_t)j * 64 + row] = (float)B[(size_t)row * n + j];
-    frag.assign((size_t)8 * kMfmaParts * kWave * 8, 0);
-    for (int m = 0; m < 4; ++m)
-        for (int ch = 0; ch < 2; ++ch)
-            for (int l = 0; l < kWave; ++l)
-                for (int i = 0; i < 8; ++i) {
-                    const int row = 16 * m + l % 16, k = 16 * (2 * ch + i / 4) + 4 * (l / 16) + i % 4;
-                    if (row >= n || k >= n) continue;
-                    double w = A[(size_t)row * n + k];
-                    for (int p = 0; p < kMfmaParts; ++p) {
-                        const uint16_t h = bf16_rne(w);
-                        frag[((((size_t)m * 2 + ch) * kMfmaParts + p) * kWave + l) * 8 + i] = h;
-                        w -= bf16_value(h);
-                    }
-                }
-}
+constexpr size_t kSweepMapElems = (size_t)8 * kMfmaParts * kWave * 8;
+inline size_t sweep_table_elems(bool pf) { return (size_t)(pf ? 1 : kTenors) * 64; }
 
 }  // namespace hjm

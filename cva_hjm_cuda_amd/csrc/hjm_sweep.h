@@ -1,8 +1,6 @@
 // hjm_sweep.h -- buffers and launches of the matrix-core reverse sweep (host side, shared by
 // the reference and portfolio Greeks).
 #pragma once
-#include <vector>
-
 #include "hjm_host.h"
 #include "hjm_kernels.h"
 #include "hjm_mfma_plan.h"
@@ -23,18 +21,15 @@ struct SweepBuffers {
     int64_t chunk_paths = 0;
     int rows = 0;             // 16 x row tiles
 
-    // Allocates for g.paths paths and uploads the maps; stored: the forward keeps the shocks.
+    // Allocates for g.paths paths and builds the maps; stored: the forward keeps the shocks.
     int take(SweepGrid& g, bool pf, double c, int nsteps, bool stored, hipStream_t st)
     {
         if (g.paths > kSweepMaxPaths) return HJM_ERR_UNSUPPORTED;
         g.units = sweep_units(g.paths);
         const int64_t group = sweep_group(g.paths), groups = (g.paths + group - 1) / group;
         rows = 16 * sweep_row_tiles(pf, g.hi + 1);
-        std::vector<uint16_t> frag;
-        std::vector<float> table;
-        build_sweep_maps(c, pf, frag, table);
-        HJM_TRY(dev_alloc(&map, frag.size()));
-        HJM_TRY(dev_alloc(&ptab, table.size()));
+        HJM_TRY(dev_alloc(&map, kSweepMapElems));
+        HJM_TRY(dev_alloc(&ptab, sweep_table_elems(pf)));
         HJM_TRY(dev_alloc(&partials, (size_t)groups * rows * 160));
         HJM_TRY(dev_alloc(&out, (size_t)rows * 160));
         if (!stored) {
@@ -44,12 +39,7 @@ struct SweepBuffers {
             if (!chunk) HJM_TRY(dev_alloc(&chunk, (size_t)n * per / sizeof(float) + kSweepSlack));
             chunk_paths = n * group;
         }
-        // the host copies go with this call
-        HJM_HIP(hipMemcpyAsync(map, frag.data(), frag.size() * sizeof(uint16_t), hipMemcpyHostToDevice, st),
-                HJM_ERR_DEVICE);
-        HJM_HIP(hipMemcpyAsync(ptab, table.data(), table.size() * sizeof(float), hipMemcpyHostToDevice, st),
-                HJM_ERR_DEVICE);
-        HJM_HIP(hipStreamSynchronize(st), HJM_ERR_DEVICE);
+        HJM_HIP(launch_sweep_map(c, pf, map, ptab, st), HJM_ERR_LAUNCH);
         return HJM_OK;
     }
 
