@@ -136,7 +136,10 @@ void adjoint_mfma_kernel(const SweepGrid g, const u4_t* __restrict__ map, const 
             x[i] = 0.f;
             pm[kPf ? 0 : i] = 0.f;
         }
-        if constexpr (kPf) load_rows(g.hi + 1, x);
+        if constexpr (kPf) {
+            load_rows(g.hi + 1, x);
+            x[13] += x[14];   // row 49: x_49 + x_50
+        }
         load_seeds(g.hi + 1);
         load_tile(g.hi, 0, za[0]);
         load_tile(g.hi, 1, za[1]);
@@ -205,6 +208,7 @@ void adjoint_mfma_kernel(const SweepGrid g, const u4_t* __restrict__ map, const 
 #pragma unroll
                 for (int i = 0; i < 16; ++i)
                     if (i == at) x[i] += v;
+                if (slot == kTenors - 1) x[13] += v;   // (row 49: x_49 + x_50)
                 if (grp == 0) mine[49 + slot] = sa;
                 const float* pr = ptab + slot * 64 + 4 * grp;
 #pragma unroll
@@ -287,6 +291,7 @@ void adjoint_mfma_kernel(const SweepGrid g, const u4_t* __restrict__ map, const 
             }
             f4_t pv[kPf ? 4 : 1];
             if constexpr (kPf) {
+                rows[13] += rows[14];
                 int at = 4 * grp;
                 asm volatile("" : "+v"(at));   // read here each time, not held in registers
 #pragma unroll

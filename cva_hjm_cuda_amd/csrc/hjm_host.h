@@ -202,7 +202,9 @@ inline void sweep_gradients(const double* M, bool pf, int ndates, double c, doub
         for (int j = n - 3; j > 0; --j) x[j] = (1.0 - c) * x[j] + c * x[j - 1];
         x[0] *= 1.0 - c;
     };
-    auto lambda = [&](int j, int col) { return M[(size_t)j * cols + col]; };
+    auto lambda = [&](int j, int col) {   // the sweep's row 49 holds tenors 49 and 50
+        return M[(size_t)j * cols + col] - (j == n - 2 ? M[(size_t)(n - 1) * cols + col] : 0.0);
+    };
     auto mu = [&](int j, int col) {
         if (pf) return j == 0 ? M[(size_t)n * cols + col] : 0.0;
         return j >= 2 && j <= ndates ? M[(size_t)(49 + j) * cols + col] : 0.0;

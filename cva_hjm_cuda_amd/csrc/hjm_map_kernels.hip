@@ -116,16 +116,20 @@ __global__ __launch_bounds__(kWave) void sweep_map_kernel(double c, int tables, 
 #pragma clang fp contract(off)
     constexpr int n = kTenors, S = kMfmaStride;
     const int j = threadIdx.x, m = blockIdx.x;
-    // column m of the powers of T^T: y_j = (1 - c) x_j + c x_{j-1}, y_49 also - c x_50, y_50 =
-    // (1 + c) x_50 + c x_49
-    double a = j == m ? 1.0 : 0.0, b = 0.0;
+    // column m of the powers of T^T with row 49 holding x_49 + x_50: y_j = (1 - c) x_j + c x_{j-1}
+    // below it, y_49 = x_49 + c x_48, y_50 = x_50 + c x_49; b: of their sum, from tenor m
+    // (tenor 50 adds to row 49 too)
+    auto step = [&](double x) {
+        const double below = __shfl_up(x, 1);
+        double y = j < n - 2 ? (1.0 - c) * x : x;
+        if (j > 0) y += c * below;
+        return j < n ? y : 0.0;
+    };
+    double a = j == m ? 1.0 : 0.0, t = j == m || (m == n - 1 && j == n - 2) ? 1.0 : 0.0, b = 0.0;
     for (int q = 0; q < S; ++q) {
-        b += a;
-        const double below = __shfl_up(a, 1), above = __shfl_down(a, 1);
-        double v = (j == n - 1 ? 1.0 + c : 1.0 - c) * a;
-        if (j > 0) v += c * below;
-        if (j == n - 2) v -= c * above;
-        a = j < n ? v : 0.0;
+        b += t;
+        t = step(t);
+        a = step(a);
     }
     if (j >= n) return;
     if (m < tables) ptab[m * 64 + j] = (float)b;
