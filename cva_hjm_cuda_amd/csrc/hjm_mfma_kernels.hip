@@ -869,21 +869,22 @@ __device__ __forceinline__ void value_bonds(const PfValueParams& v, int e, int64
 
 // One M-tile's values for NT N-tiles: acc[n] = a + (-gamma) P over the chunks the tile uses.
 // (A second accumulator for the small split products, as in the path kernels, changed the
-// per-set CVA error by 2 % and cost the valuation a wave per SIMD: not used here.)
+// per-set CVA error by 2 % and cost the valuation a wave per SIMD: not used here. a joins last, by
+// a rounded addition: the matrix cores truncate every group's sum toward zero at the
+// accumulator's size, which with a in it biased V and with it which paths count as
+// positive; spot gradients of a 128-set book 2.3 -> 1.2e-6 off, for 6 % of the valuation's time.)
 template <int NT>
 __device__ __forceinline__ void value_tile(const u4_t* __restrict__ fr0, int lane, int tk, f4_t a4,
                                            const Split8 (&bs)[NT][2], f4_t (&acc)[NT])
 {
 #pragma unroll
-    for (int n = 0; n < NT; ++n) acc[n] = a4;
-#pragma unroll
     for (int c = 0; c < 2; ++c) {
-        if (tk > 32 * c) {
+        if (c == 0 || tk > 32) {
             const u4_t* fr = fr0 + (c * kMfmaParts) * kWave + lane;
             const u4_t ah = fr[0], am = fr[kWave], al = fr[2 * kWave];
             // one product for the N-tiles in turn: no product waits for the one before
 #pragma unroll
-            for (int n = 0; n < NT; ++n) acc[n] = mfma_bf16(ah, bs[n][c].h, acc[n]);
+            for (int n = 0; n < NT; ++n) acc[n] = mfma_bf16(ah, bs[n][c].h, c ? acc[n] : f4_t{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
             for (int n = 0; n < NT; ++n) acc[n] = mfma_bf16(ah, bs[n][c].m, acc[n]);
 #pragma unroll
@@ -896,6 +897,8 @@ __device__ __forceinline__ void value_tile(const u4_t* __restrict__ fr0, int lan
             for (int n = 0; n < NT; ++n) acc[n] = mfma_bf16(am, bs[n][c].m, acc[n]);
         }
     }
+#pragma unroll
+    for (int n = 0; n < NT; ++n) acc[n] += a4;
 }
 
 __device__ __forceinline__ float exposure_of(float V, float disc) { return V > 0.f ? V * disc : 0.f; }
@@ -912,7 +915,7 @@ __device__ __forceinline__ float exposure_of(float V, float disc) { return V > 0
 // waits for the stores: a global load there would, since loads and stores share one counter,
 // so the tile constants and live sets are read once into LDS. Products go round the N-tiles,
 // so none waits for the one before. {2 N-tiles, 8 waves, stage 2} by measurement: at that
-// size 9.86 ms against 10.62 for {4, 4, 8}, at 32 sets x 262144 paths 1.20 against 1.23, at
+// size 10.5 ms against 11.3 for {4, 4, 8}, at 32 sets x 262144 paths 1.20 against 1.23, at
 // 11 x 10007 0.042 against 0.048 (all {4, 4, 8} with the constants in global memory: 12.2,
 // 1.31 and 0.048).
 constexpr int kValMaxStage = 8;  // M-tiles staged at a time, at most

@@ -313,8 +313,8 @@ int hjm_block_map64(const double* drifts, const double* volatilities, double dt,
 /* ---- calibration upstream of the path (no code in the reference; its roadmap,
  * doc/TODO:16, names the volatility and drift calibration of the HJM model) ----------
  * Batched rolling-window PCA of historical forward curves: per window the annualised
- * sample covariance of the daily curve differences, its eigendecomposition (GPU, FP64,
- * cyclic Jacobi), loadings sigma_k = sqrt(lambda_k) v_k of the 3 leading factors (sign:
+ * sample covariance of the daily curve differences, its eigenvalues and leading
+ * eigenvectors (GPU, FP64), loadings sigma_k = sqrt(lambda_k) v_k of the 3 leading factors (sign:
  * components sum > 0), optionally least-squares polynomials in the tenor, and their HJM
  * drift (hjm_hjm_drift). The outputs feed hjm_market directly. */
 typedef struct {
