@@ -83,38 +83,44 @@ __device__ __forceinline__ void for_each_index(F& f, std::integer_sequence<int, 
 
 // One 50-step block: acc = W x [fin; shocks of steps b*50 .. b*50+49; 1]. kStore: also
 // write the block's normals to zs[step][factor][path] (FP32) for a later reverse sweep.
-// kTwoAcc: the small split products (all but Wh xh) accumulate apart from Wh xh and join it
-// once at the end. The matrix cores drop the low bits of products far below the accumulator
-// (measured: C = 1 plus 32 products of 2^-27 returns 1; small positive contributions are
-// lost, small negative ones kept), which biases a single accumulator holding the curve (FP32
-// vs FP64: EE 1.4e-6 -> 3.2e-7 on the 10y precision workload with two). It costs 4 registers
-// per tile and N-tile.
-template <int MT, int NT, bool kStore, bool kInterleave, bool kTwoAcc>
+// kSplitAcc: three accumulators, added up (rounded) once at the end: the curve's Wh xh, the
+// shocks' Wh xh, and every smaller product. The matrix cores truncate a product's sum at the
+// accumulator's size (measured: C = 1 plus 32 products of 2^-27 returns 1; small positive
+// contributions are lost, small negative ones kept). The curve's Wh xh are 16-bit products,
+// which such a sum holds whole; the shocks' are 22 bits wide and are a few percent of the
+// curve, whose accumulator would cut their low bits; with the small products they would cut
+// those. A path's forwards over 10y against FP64, rms relative: 2.1e-7 with the shocks' Wh xh in
+// the curve's accumulator, 1.35e-7 in the small products', 1.26e-7 apart (2.0e-7 with three
+// bf16 parts and two accumulators). It costs 8 registers per tile and N-tile over two
+// accumulators' and 2 % of the reference kernel's time at 131072 paths x 10y (0.43 to 0.44 ms;
+// 12 % where it stores the shocks), 4 % of the portfolio's.
+template <int MT, int NT, bool kStore, bool kInterleave, bool kSplitAcc>
 __device__ __forceinline__ void mfma_block(const u4_t* __restrict__ lds_w, const float (&fin)[NT][16],
                                            f4_t (&acc)[MT][NT], const MfmaGrid& g,
                                            const int64_t (&path)[NT], const bool (&live)[NT],
                                            int b, int grp, int lane, float* __restrict__ zs)
 {
+    constexpr int MS = kSplitAcc ? MT : 1;
+    f4_t shock[MS][NT], small[MS][NT];
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int n = 0; n < NT; ++n) acc[m][n] = f4_t{0.f, 0.f, 0.f, 0.f};
+        for (int n = 0; n < NT; ++n) {
+            acc[m][n] = f4_t{0.f, 0.f, 0.f, 0.f};
+            if constexpr (kSplitAcc) shock[m][n] = small[m][n] = f4_t{0.f, 0.f, 0.f, 0.f};
+        }
     // W's fragments are the same in every block: an opaque offset keeps their LDS reads
     // inside the block instead of hoisted (hundreds of registers) out of the block loop
     uint32_t off = (uint32_t)lane;
     asm volatile("" : "+v"(off));
-    constexpr int MT2 = kTwoAcc ? MT : 1;
-    f4_t acc2[MT2][NT];
-#pragma unroll
-    for (int m = 0; m < MT2; ++m)
-#pragma unroll
-        for (int n = 0; n < NT; ++n) acc2[m][n] = f4_t{0.f, 0.f, 0.f, 0.f};
     // one product for the N-tiles in turn (consecutive MFMAs then write different
-    // accumulators): large = Wh xh, otherwise into the small products' accumulator
-    auto product = [&](int m, bool large, u4_t a, auto fn) {
+    // accumulators)
+    enum Kind { kCurve, kShock, kSmall };
+    auto product = [&](int m, Kind kind, u4_t a, auto fn) {
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
-            if (kTwoAcc && !large) acc2[kTwoAcc ? m : 0][n] = fn(a, n, acc2[kTwoAcc ? m : 0][n]);
+            if (kSplitAcc && kind == kSmall) small[kSplitAcc ? m : 0][n] = fn(a, n, small[kSplitAcc ? m : 0][n]);
+            else if (kSplitAcc && kind == kShock) shock[kSplitAcc ? m : 0][n] = fn(a, n, shock[kSplitAcc ? m : 0][n]);
             else acc[m][n] = fn(a, n, acc[m][n]);
         }
     };
@@ -127,12 +133,12 @@ __device__ __forceinline__ void mfma_block(const u4_t* __restrict__ lds_w, const
             if (mfma_chunk_zero(m, c, false)) continue;
             const u4_t* a = lds_w + mfma_frag(m, c, 0) * kWave + off;
             const u4_t ah = a[0], am = a[kWave], al = a[2 * kWave];
-            product(m, true, ah, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].h, v); });
-            product(m, false, ah, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].m, v); });
-            product(m, false, am, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].h, v); });
-            product(m, false, ah, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].l, v); });
-            product(m, false, al, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].h, v); });
-            product(m, false, am, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].m, v); });
+            product(m, kCurve, ah, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].h, v); });
+            product(m, kSmall, ah, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].m, v); });
+            product(m, kSmall, am, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].h, v); });
+            product(m, kSmall, ah, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].l, v); });
+            product(m, kSmall, al, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].h, v); });
+            product(m, kSmall, am, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].m, v); });
         }
     };
     auto shock_tiles = [&](int c, int m0, int m1, const SplitH8 (&xs)[NT]) {
@@ -140,9 +146,9 @@ __device__ __forceinline__ void mfma_block(const u4_t* __restrict__ lds_w, const
         for (int m = m0; m < m1; ++m) {
             const u4_t* a = lds_w + mfma_frag(m, c, 0) * kWave + off;
             const u4_t ah = a[0], al = a[kWave];
-            product(m, true, ah, [&](u4_t w, int n, f4_t v) { return mfma_f16(w, xs[n].h, v); });
-            product(m, false, ah, [&](u4_t w, int n, f4_t v) { return mfma_f16(w, xs[n].l, v); });
-            product(m, false, al, [&](u4_t w, int n, f4_t v) { return mfma_f16(w, xs[n].h, v); });
+            product(m, kShock, ah, [&](u4_t w, int n, f4_t v) { return mfma_f16(w, xs[n].h, v); });
+            product(m, kSmall, ah, [&](u4_t w, int n, f4_t v) { return mfma_f16(w, xs[n].l, v); });
+            product(m, kSmall, al, [&](u4_t w, int n, f4_t v) { return mfma_f16(w, xs[n].h, v); });
         }
     };
     // split operands: curve chunks from fin (registers 8 c .. 8 c + 7), shock chunk s from
@@ -219,11 +225,11 @@ __device__ __forceinline__ void mfma_block(const u4_t* __restrict__ lds_w, const
     };
     for_each_index(quad, std::make_integer_sequence<int, kMfmaQuads>{});
     shock_tiles(kMfmaChunks - 1, 0, MT, xs[kMfmaChunks - 3]);
-    if constexpr (kTwoAcc) {
+    if constexpr (kSplitAcc) {
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
-            for (int n = 0; n < NT; ++n) acc[m][n] += acc2[m][n];
+            for (int n = 0; n < NT; ++n) acc[m][n] += small[m][n] + shock[m][n];
     }
 }
 
@@ -299,7 +305,7 @@ __attribute__((amdgpu_waves_per_eu(path_waves_per_simd(kNT), path_waves_per_simd
 
     for (int b = 1; b < g.ndates; ++b) {
         f4_t acc[MT][kNT];
-        // two accumulators where registers allow (up to 5 live tiles: 239 VGPRs)
+        // three accumulators where registers allow (up to 5 live tiles: 255 VGPRs)
         mfma_block<MT, kNT, kStore, true, (MT <= 5)>(lds_w, fin, acc, g, path, live, b, grp, lane, zs);
         // integrals: Kahan-add the block's dA (tiles 3 .. MT-1); curve rows become next input
 #pragma unroll
@@ -443,7 +449,7 @@ __global__ __launch_bounds__(tile_waves(MT) * kWave, kStore && MT > 4 ? 3 : 4) v
     double* __restrict__ num_y, float* __restrict__ curves, double* __restrict__ logb,
     float* __restrict__ zs, int64_t begin)
 {
-    constexpr bool kTwoAcc = kPf || MT <= 5;   // as the kernels above
+    constexpr bool kSplitAcc = kPf || MT <= 5;   // as the kernels above
     __shared__ u4_t s_z[2][kShockChunks][2][kWave];
     __shared__ u4_t s_c[2][2][kMfmaParts][kWave];
     const int lane = threadIdx.x & (kWave - 1), wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -540,9 +546,9 @@ __global__ __launch_bounds__(tile_waves(MT) * kWave, kStore && MT > 4 ? 3 : 4) v
         const int buf = i & 1;
         if (i + 1 < nb) shocks(b0 + i + 1, buf ^ 1);
         if (mine) {
-            f4_t acc = {0.f, 0.f, 0.f, 0.f}, acc2 = acc;
+            f4_t acc = {0.f, 0.f, 0.f, 0.f}, acc_shock = acc, acc_small = acc;
             auto small = [&](auto fn, u4_t a, u4_t x) {
-                if constexpr (kTwoAcc) acc2 = fn(a, x, acc2);
+                if constexpr (kSplitAcc) acc_small = fn(a, x, acc_small);
                 else acc = fn(a, x, acc);
             };
 #pragma unroll
@@ -562,11 +568,12 @@ __global__ __launch_bounds__(tile_waves(MT) * kWave, kStore && MT > 4 ? 3 : 4) v
             for (int c = 0; c < kShockChunks; ++c) {
                 const u4_t h = s_z[buf][c][0][lane], l = s_z[buf][c][1][lane];
                 const u4_t* a = w + 6 + 2 * c;
-                acc = mfma_f16(a[0], h, acc);
+                if constexpr (kSplitAcc) acc_shock = mfma_f16(a[0], h, acc_shock);
+                else acc = mfma_f16(a[0], h, acc);
                 small(mfma_f16, a[0], l);
                 small(mfma_f16, a[1], h);
             }
-            if constexpr (kTwoAcc) acc += acc2;
+            if constexpr (kSplitAcc) acc += acc_small + acc_shock;
             if constexpr (!kPf) {
                 if (wv >= 3) {
 #pragma unroll
