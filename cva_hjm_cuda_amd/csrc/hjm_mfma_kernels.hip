@@ -874,38 +874,48 @@ __device__ __forceinline__ void value_bonds(const PfValueParams& v, int e, int64
     }
 }
 
-// One M-tile's values for NT N-tiles: acc[n] = a + (-gamma) P over the chunks the tile uses.
-// (A second accumulator for the small split products, as in the path kernels, changed the
-// per-set CVA error by 2 % and cost the valuation a wave per SIMD: not used here. a joins last, by
-// a rounded addition: the matrix cores truncate every group's sum toward zero at the
-// accumulator's size, which with a in it biased V and with it which paths count as
-// positive; spot gradients of a 128-set book 2.3 -> 1.2e-6 off, for 6 % of the valuation's time.)
+// One M-tile's values for NT N-tiles: acc[n] = a + (-gamma) P over the chunks the tile uses. a and
+// the products Wh xh share an accumulator, the five smaller products of a chunk another, and
+// the two are added up (rounded). The matrix cores truncate a sum at the accumulator's size:
+// beside a, that of the gross book, Wh xh (16 bits) stay whole, and the sum falls to the netted
+// value at once; the small products, a 2^-8 part, lose bits only at their own size. With all
+// products accumulated from zero and a joined last, every small product was truncated at the size
+// of gamma P: PFE of random books 5.6e-7 (relative, over all sets and dates) from the FP64 run,
+// EE 4.9e-7; from a on in one accumulator 3.4 and 3.5e-7, and spot gradients of a book 3 times
+// farther off; now 2.5 and 3.2e-7. At no cost in time: 1048576 paths x 61 dates x 128 sets
+// 10.8 ms before, 10.7 now.
 template <int NT>
 __device__ __forceinline__ void value_tile(const u4_t* __restrict__ fr0, int lane, int tk, f4_t a4,
                                            const Split8 (&bs)[NT][2], f4_t (&acc)[NT])
 {
+    f4_t small[NT];
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
+    for (int n = 0; n < NT; ++n) {
+        acc[n] = a4;
+        small[n] = f4_t{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int c = 1; c >= 0; --c) {
         if (c == 0 || tk > 32) {
             const u4_t* fr = fr0 + (c * kMfmaParts) * kWave + lane;
             const u4_t ah = fr[0], am = fr[kWave], al = fr[2 * kWave];
             // one product for the N-tiles in turn: no product waits for the one before
 #pragma unroll
-            for (int n = 0; n < NT; ++n) acc[n] = mfma_bf16(ah, bs[n][c].h, c ? acc[n] : f4_t{0.f, 0.f, 0.f, 0.f});
+            for (int n = 0; n < NT; ++n) small[n] = mfma_bf16(am, bs[n][c].m, small[n]);
 #pragma unroll
-            for (int n = 0; n < NT; ++n) acc[n] = mfma_bf16(ah, bs[n][c].m, acc[n]);
+            for (int n = 0; n < NT; ++n) small[n] = mfma_bf16(ah, bs[n][c].l, small[n]);
 #pragma unroll
-            for (int n = 0; n < NT; ++n) acc[n] = mfma_bf16(am, bs[n][c].h, acc[n]);
+            for (int n = 0; n < NT; ++n) small[n] = mfma_bf16(al, bs[n][c].h, small[n]);
 #pragma unroll
-            for (int n = 0; n < NT; ++n) acc[n] = mfma_bf16(ah, bs[n][c].l, acc[n]);
+            for (int n = 0; n < NT; ++n) acc[n] = mfma_bf16(ah, bs[n][c].h, acc[n]);
 #pragma unroll
-            for (int n = 0; n < NT; ++n) acc[n] = mfma_bf16(al, bs[n][c].h, acc[n]);
+            for (int n = 0; n < NT; ++n) small[n] = mfma_bf16(ah, bs[n][c].m, small[n]);
 #pragma unroll
-            for (int n = 0; n < NT; ++n) acc[n] = mfma_bf16(am, bs[n][c].m, acc[n]);
+            for (int n = 0; n < NT; ++n) small[n] = mfma_bf16(am, bs[n][c].h, small[n]);
         }
     }
 #pragma unroll
-    for (int n = 0; n < NT; ++n) acc[n] += a4;
+    for (int n = 0; n < NT; ++n) acc[n] += small[n];
 }
 
 __device__ __forceinline__ float exposure_of(float V, float disc) { return V > 0.f ? V * disc : 0.f; }
@@ -922,9 +932,9 @@ __device__ __forceinline__ float exposure_of(float V, float disc) { return V > 0
 // waits for the stores: a global load there would, since loads and stores share one counter,
 // so the tile constants and live sets are read once into LDS. Products go round the N-tiles,
 // so none waits for the one before. {2 N-tiles, 8 waves, stage 2} by measurement: at that
-// size 10.5 ms against 11.3 for {4, 4, 8}, at 32 sets x 262144 paths 1.20 against 1.23, at
-// 11 x 10007 0.042 against 0.048 (all {4, 4, 8} with the constants in global memory: 12.2,
-// 1.31 and 0.048).
+// size 10.7 ms against 12.4 for {4, 4, 8} and 11.9 for {2, 4, 2}, at 32 sets x 262144 paths 1.32
+// against 1.49 and 1.39, at 11 x 10007 0.046 .. 0.049 against 0.054 and 0.046. (Stages 1 .. 8 differ
+// by less than runs do.)
 constexpr int kValMaxStage = 8;  // M-tiles staged at a time, at most
 
 template <int NT, int WAVES>
