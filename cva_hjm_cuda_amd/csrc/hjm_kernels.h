@@ -94,12 +94,16 @@ struct SweepGrid {
 constexpr int64_t kSweepMaxPaths = (int64_t)1 << 26;   // 32-bit lane offsets: 48 B x paths
 constexpr int kSweepSlack = 32;              // floats of zeros the sweep needs past zs
 int sweep_row_tiles(bool pf, int ndates);    // rows of a partial: 16 x this, 160 columns
+// units of a pair of waves, 1 or 2: its FP32 sums then cover at most 2 units' blocks, for any
+// number of paths, before they join the FP64 ones
 int sweep_units(int64_t paths);
 int64_t sweep_group(int64_t paths);          // paths of a workgroup: one partial each
 hipError_t launch_adjoint_mfma(const SweepGrid& g, bool pf, const uint16_t* map, const float* ptab,
                                const float* zs, const float* seed_a, const float* seed_b, float* partials,
                                hipStream_t st);
-hipError_t launch_sweep_sum(const float* partials, int64_t rows, int cols, double* out, hipStream_t st);
+// out[c] = (add ? out[c] : 0) + the FP64 sum of partials[r][c] over the rows, in a fixed order
+hipError_t launch_sweep_sum(const float* partials, int64_t rows, int cols, bool add, double* out,
+                            hipStream_t st);
 hipError_t launch_sweep_shocks(uint64_t seed, int64_t path0, const SweepGrid& g, float* zs, hipStream_t st);
 
 // A book's swaps on the device, grouped by netting set (the caller's order within a set):

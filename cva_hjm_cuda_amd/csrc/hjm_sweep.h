@@ -11,6 +11,9 @@ namespace hjm_host {
 // number of workgroups' paths at a time (the sums do not depend on it: every workgroup writes
 // its own partial).
 constexpr size_t kSweepChunkBytes = (size_t)1 << 30;
+// Partials of at most this many workgroups (40 to 72 KB each) are held at a time; each such
+// segment is summed into the FP64 result before the next.
+constexpr int64_t kSweepSegment = 4096;
 
 struct SweepBuffers {
     uint16_t* map = nullptr;
@@ -30,11 +33,12 @@ struct SweepBuffers {
         rows = 16 * sweep_row_tiles(pf, g.hi + 1);
         HJM_TRY(dev_alloc(&map, kSweepMapElems));
         HJM_TRY(dev_alloc(&ptab, sweep_table_elems(pf)));
-        HJM_TRY(dev_alloc(&partials, (size_t)groups * rows * 160));
+        HJM_TRY(dev_alloc(&partials, (size_t)std::min(groups, kSweepSegment) * rows * 160));
         HJM_TRY(dev_alloc(&out, (size_t)rows * 160));
         if (!stored) {
             const size_t per = (size_t)group * nsteps * 3 * sizeof(float);
-            int64_t n = std::min<int64_t>(groups, std::max<int64_t>(1, (int64_t)(kSweepChunkBytes / per)));
+            int64_t n = std::min<int64_t>(std::min(groups, kSweepSegment),
+                                          std::max<int64_t>(1, (int64_t)(kSweepChunkBytes / per)));
             while (n > 1 && dev_alloc(&chunk, (size_t)n * per / sizeof(float) + kSweepSlack) != HJM_OK) n /= 2;
             if (!chunk) HJM_TRY(dev_alloc(&chunk, (size_t)n * per / sizeof(float) + kSweepSlack));
             chunk_paths = n * group;
@@ -56,18 +60,25 @@ struct SweepBuffers {
     {
         const int64_t group = sweep_group(g.paths), groups = (g.paths + group - 1) / group;
         const int cols = rows * 160;
-        const int64_t step = zs ? g.paths : chunk_paths;
-        for (int64_t p = 0; p < g.paths; p += step) {
-            g.begin = p;
-            g.end = std::min(g.paths, p + step);
-            g.zld = zs ? g.paths : g.end - g.begin;
-            HJM_TRY(clear_slack(zs ? zs : chunk, (size_t)g.zld * nsteps * 3, st));
-            if (!zs) HJM_HIP(launch_sweep_shocks(seed, path0, g, chunk, st), HJM_ERR_LAUNCH);
-            HJM_HIP(launch_adjoint_mfma(g, pf, map, ptab, zs ? zs : chunk, seed_a, seed_b,
-                                        partials + (size_t)(p / group) * cols, st),
+        const int64_t segment = kSweepSegment * group, step = zs ? segment : chunk_paths;
+        if (zs) HJM_TRY(clear_slack(zs, (size_t)g.paths * nsteps * 3, st));
+        for (int64_t first = 0; first < groups; first += kSweepSegment) {
+            const int64_t end = std::min(g.paths, first * group + segment);
+            for (int64_t p = first * group; p < end; p += step) {
+                g.begin = p;
+                g.end = std::min(end, p + step);
+                g.zld = zs ? g.paths : g.end - g.begin;
+                if (!zs) {
+                    HJM_TRY(clear_slack(chunk, (size_t)g.zld * nsteps * 3, st));
+                    HJM_HIP(launch_sweep_shocks(seed, path0, g, chunk, st), HJM_ERR_LAUNCH);
+                }
+                HJM_HIP(launch_adjoint_mfma(g, pf, map, ptab, zs ? zs + p : chunk, seed_a, seed_b,
+                                            partials + (size_t)(p / group - first) * cols, st),
+                        HJM_ERR_LAUNCH);
+            }
+            HJM_HIP(launch_sweep_sum(partials, std::min(groups - first, kSweepSegment), cols, first > 0, out, st),
                     HJM_ERR_LAUNCH);
         }
-        HJM_HIP(launch_sweep_sum(partials, groups, cols, out, st), HJM_ERR_LAUNCH);
         HJM_HIP(hipMemcpyAsync(sums, out, sizeof(double) * cols, hipMemcpyDeviceToHost, st), HJM_ERR_DEVICE);
         return HJM_OK;
     }
