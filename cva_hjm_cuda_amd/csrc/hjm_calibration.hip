@@ -562,15 +562,10 @@ int hjm_calibrate_pca(const hjm_calibration* c, hjm_calibration_results* r)
         (void)hipEventElapsedTime(&ms, e0, e1);
         r->timings_ms[0] = ms;
     }
-    (void)hipStreamSynchronize(nullptr);
+    const bool clean = hipStreamSynchronize(nullptr) == hipSuccess;
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
-    dev_free(d_curves);
-    dev_free(d_ev);
-    dev_free(d_ld);
-    dev_free(d_raw);
-    dev_free(d_cov);
-    dev_free(d_drift);
+    dev_free(clean, d_curves, d_ev, d_ld, d_raw, d_cov, d_drift);
     return rc;
 }
 

@@ -88,17 +88,9 @@ void plan_release(hjm_plan p)
     (void)hipGetDevice(&prev);
     (void)hipSetDevice(p->device);
     const bool clean = p->ctx.quiesce();
-    dev_free(p->d_normals);
-    dev_free(p->d_wfrag);
-    dev_free(p->d_wfrag64);
-    dev_free(p->d_nx);
-    dev_free(p->d_ny);
-    dev_free(p->d_ex);
-    dev_free(p->d_partials);
-    dev_free(p->d_sums);
-    dev_free(p->d_selws);
+    dev_free(clean, p->d_normals, p->d_wfrag, p->d_wfrag64, p->d_nx, p->d_ny, p->d_ex, p->d_partials, p->d_sums,
+             p->d_selws);
     p->ctx.give();
-    if (!clean) pool_release_all();
     if (prev >= 0) (void)hipSetDevice(prev);
     delete p;
 }
@@ -469,14 +461,9 @@ int hjm_cva_greeks_reference(const hjm_market* market, const hjm_swap* swap,
         SweepBuffers sweep;
         ~Cleanup()
         {
-            (void)p->ctx.quiesce();
-            dev_free(gx);
-            dev_free(zs);
-            dev_free(gA);
-            dev_free(part);
-            dev_free(sums);
-            dev_free(sap);
-            sweep.free();
+            const bool clean = p->ctx.quiesce();
+            dev_free(clean, gx, zs, gA, part, sums, sap);
+            sweep.free(clean);
             hjm_plan_destroy(p);
         }
     } c{p};
@@ -610,15 +597,8 @@ int hjm_simulate_reference_blockwise(const hjm_market* market, const hjm_swap* s
         hipEvent_t ev[5] = {};
         ~Bufs()
         {
-            if (st) (void)hipStreamSynchronize(st);
-            dev_free(normals);
-            dev_free(s0);
-            dev_free(s1);
-            dev_free(integ);
-            dev_free(nx);
-            dev_free(ny);
-            dev_free(ex);
-            dev_free(sums);
+            const bool clean = !st || hipStreamSynchronize(st) == hipSuccess;
+            dev_free(clean, normals, s0, s1, integ, nx, ny, ex, sums);
             for (auto& x : ev)
                 if (x) (void)hipEventDestroy(x);
             if (st) (void)hipStreamDestroy(st);
@@ -741,8 +721,7 @@ int hjm_generate_normals(uint64_t seed, int64_t path_offset, int64_t paths, int3
         rc = HJM_ERR_LAUNCH;
     else if (hipMemcpy(out, d, n * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess)
         rc = HJM_ERR_DEVICE;
-    (void)hipStreamSynchronize(nullptr);
-    dev_free(d);
+    dev_free(hipStreamSynchronize(nullptr) == hipSuccess, d);
     return rc;
 }
 
@@ -768,10 +747,8 @@ int hjm_box_muller_parts(const uint32_t* words, int64_t n, int32_t device, float
                  hipMemcpy(cosine, d + n, b, hipMemcpyDeviceToHost) != hipSuccess ||
                  hipMemcpy(sine, d + 2 * n, b, hipMemcpyDeviceToHost) != hipSuccess)
             rc = HJM_ERR_DEVICE;
-        (void)hipStreamSynchronize(nullptr);
-        dev_free(d);
     }
-    dev_free(dw);
+    dev_free(hipStreamSynchronize(nullptr) == hipSuccess, d, dw);
     return rc;
 }
 
@@ -798,10 +775,7 @@ int hjm_select_kth(const double* values, int32_t rows, int64_t n, int64_t k, int
     if (rc == HJM_OK && hipDeviceSynchronize() != hipSuccess) rc = HJM_ERR_LAUNCH;
     if (rc == HJM_OK && hipMemcpy(out, d_out, rows * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess)
         rc = HJM_ERR_DEVICE;
-    (void)hipStreamSynchronize(nullptr);
-    dev_free(d);
-    dev_free(d_out);
-    dev_free(ws);
+    dev_free(hipStreamSynchronize(nullptr) == hipSuccess, d, d_out, ws);
     return rc;
 }
 

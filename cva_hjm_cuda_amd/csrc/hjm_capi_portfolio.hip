@@ -72,27 +72,10 @@ void pplan_release(hjm_portfolio_plan p)
     const bool clean = p->ctx.quiesce();
     if (p->exec) (void)hipGraphExecDestroy(p->exec);
     if (p->graph) (void)hipGraphDestroy(p->graph);
-    dev_free(p->d_normals);
-    dev_free(p->d_curves);
-    dev_free(p->d_logb);
-    dev_free(p->d_ex);
-    dev_free(p->d_partials);
-    dev_free(p->d_sums);
-    dev_free(p->d_selws);
-    dev_free(p->d_loparts);
-    dev_free(p->d_coef);
-    dev_free(p->d_book_ints);
-    dev_free(p->d_book_reals);
-    dev_free(p->d_vfrag);
-    dev_free(p->d_apad);
-    dev_free(p->d_tilek);
-    dev_free(p->d_a);
-    dev_free(p->d_kmax);
-    dev_free(p->d_w);
-    dev_free(p->d_wfrag);
-    dev_free(p->d_wfrag64);
+    dev_free(clean, p->d_normals, p->d_curves, p->d_logb, p->d_ex, p->d_partials, p->d_sums, p->d_selws,
+             p->d_loparts, p->d_coef, p->d_book_ints, p->d_book_reals, p->d_vfrag, p->d_apad, p->d_tilek,
+             p->d_a, p->d_kmax, p->d_w, p->d_wfrag, p->d_wfrag64);
     p->ctx.give();
-    if (!clean) pool_release_all();
     if (prev >= 0) (void)hipSetDevice(prev);
     delete p;
 }
@@ -612,15 +595,9 @@ int hjm_portfolio_cva_greeks(const hjm_market* market, const hjm_portfolio* port
         SweepBuffers sweep;
         ~Cleanup()
         {
-            (void)p->ctx.quiesce();
-            dev_free(zs);
-            dev_free(gbar);
-            dev_free(beta);
-            dev_free(part);
-            dev_free(sums);
-            dev_free(bp);
-            dev_free(tfrag);
-            sweep.free();
+            const bool clean = p->ctx.quiesce();
+            dev_free(clean, zs, gbar, beta, part, sums, bp, tfrag);
+            sweep.free(clean);
             hjm_portfolio_plan_destroy(p);
         }
     } c{p};

@@ -54,12 +54,13 @@ inline int dev_alloc(T** p, size_t count)
     return HJM_OK;
 }
 
-// Only once the work that used the block is done (hjm_pool.h).
-template <typename T>
-inline void dev_free(T*& p)
+// Blocks whose work is done (idle), or may not be: the stream that used them is in error, and
+// they are not kept for other plans (hjm_pool.h).
+template <typename... T>
+inline void dev_free(bool idle, T*&... p)
 {
-    pool_free((void*)p);
-    p = nullptr;
+    (pool_free((void*)p, idle), ...);
+    ((p = nullptr), ...);
 }
 
 // A plan's stream, events and pinned buffer, returned to the cache when the plan goes. Waits
@@ -71,8 +72,8 @@ struct ContextHolder {
         c = context_acquire(device, host_bytes);
         return c ? HJM_OK : HJM_ERR_DEVICE;
     }
-    // false: the stream is in error and nothing that it used may be handed out again
-    bool quiesce() { return !c || hipStreamSynchronize(c->stream) == hipSuccess; }
+    // false: the stream is in error and nothing that it used may be handed out again (dev_free)
+    [[nodiscard]] bool quiesce() { return !c || hipStreamSynchronize(c->stream) == hipSuccess; }
     void give()
     {
         context_release(c);

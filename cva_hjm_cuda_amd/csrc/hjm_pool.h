@@ -8,7 +8,8 @@
 //     beyond that; larger blocks never enter), gives everything back when an allocation
 //     fails (which is then tried again) and on hjm_release_cached_memory;
 //   * takes a block only when no work on it is outstanding: whoever frees one has
-//     synchronised the stream that used it (hipFree used to wait for the device);
+//     synchronised the stream that used it (hipFree used to wait for the device), and says so
+//     if that failed: such a block goes back to the device and to no other plan;
 //   * is behind one mutex: any thread may allocate and free on any device.
 // Blocks come back with their old contents, as undefined as hipMalloc's.
 #pragma once
@@ -22,7 +23,8 @@ constexpr int kPoolContexts = 8;                // idle plan contexts per device
 
 // Memory of the current device; hipErrorOutOfMemory (or the runtime's error) on failure.
 hipError_t pool_alloc(void** p, size_t bytes);
-void pool_free(void* p);
+// idle: the work that used the block is known to be done, so it may be kept.
+void pool_free(void* p, bool idle);
 void pool_release_all();
 
 // A plan's stream (non-blocking, default priority), timing events and pinned host buffer.

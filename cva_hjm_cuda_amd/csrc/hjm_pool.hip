@@ -114,7 +114,7 @@ hipError_t pool_alloc(void** out, size_t bytes)
     }
 }
 
-void pool_free(void* p)
+void pool_free(void* p, bool idle)
 {
     if (!p) return;
     Pool& q = pool();
@@ -126,7 +126,7 @@ void pool_free(void* p)
         if (it != q.live.end()) {
             b = it->second;
             q.live.erase(it);
-            if (b.bytes <= kPoolBytes) {
+            if (idle && b.bytes <= kPoolBytes) {
                 size_t held = b.bytes;
                 for (const Block& x : q.idle) held += x.device == b.device ? x.bytes : 0;
                 for (auto x = q.idle.begin(); held > kPoolBytes && x != q.idle.end();) {

@@ -83,14 +83,7 @@ struct SweepBuffers {
         return HJM_OK;
     }
 
-    void free()
-    {
-        dev_free(map);
-        dev_free(ptab);
-        dev_free(partials);
-        dev_free(out);
-        dev_free(chunk);
-    }
+    void free(bool idle) { dev_free(idle, map, ptab, partials, out, chunk); }
 };
 
 }  // namespace hjm_host
