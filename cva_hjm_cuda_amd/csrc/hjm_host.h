@@ -69,8 +69,7 @@ struct ContextHolder {
     PlanContext* c = nullptr;
     int take(int device, size_t host_bytes)
     {
-        c = context_acquire(device, host_bytes);
-        return c ? HJM_OK : HJM_ERR_DEVICE;
+        return context_acquire(device, host_bytes, &c);
     }
     // false: the stream is in error and nothing that it used may be handed out again (dev_free)
     [[nodiscard]] bool quiesce() { return !c || hipStreamSynchronize(c->stream) == hipSuccess; }

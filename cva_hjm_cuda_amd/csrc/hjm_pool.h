@@ -35,8 +35,9 @@ struct PlanContext {
     void* host = nullptr;      // pinned, host_bytes long
     size_t host_bytes = 0;
 };
-// A context of the current device (an idle one if there is), or null.
-PlanContext* context_acquire(int device, size_t host_bytes);
+// A context of the current device (an idle one if there is); HJM_ERR_ALLOC if its pinned
+// buffer cannot be had, after the cache was given back, HJM_ERR_DEVICE if its stream cannot.
+int context_acquire(int device, size_t host_bytes, PlanContext** out);
 // Waits for the context's stream, then keeps the context for the next plan.
 void context_release(PlanContext* c);
 

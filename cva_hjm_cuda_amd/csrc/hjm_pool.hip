@@ -166,8 +166,9 @@ void pool_release_all()
     for (PlanContext* c : contexts) context_destroy(c);
 }
 
-PlanContext* context_acquire(int device, size_t host_bytes)
+int context_acquire(int device, size_t host_bytes, PlanContext** out)
 {
+    *out = nullptr;
     Pool& q = pool();
     PlanContext* c = nullptr;
     {
@@ -181,29 +182,37 @@ PlanContext* context_acquire(int device, size_t host_bytes)
     }
     if (!c) {
         c = new (std::nothrow) PlanContext();
-        if (!c) return nullptr;
+        if (!c) return HJM_ERR_ALLOC;
         c->device = device;
         bool ok = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) == hipSuccess;
         for (auto& e : c->ev) ok = ok && hipEventCreate(&e) == hipSuccess;
         if (!ok) {
             (void)hipGetLastError();
             context_destroy(c);
-            return nullptr;
+            return HJM_ERR_DEVICE;
         }
     }
     if (c->host_bytes < host_bytes) {
         if (c->host) (void)hipHostFree(c->host);
         c->host = nullptr;
         c->host_bytes = 0;
-        if (hipHostMalloc(&c->host, host_bytes, hipHostMallocDefault) != hipSuccess) {
+        auto take = [&] {
+            if (hipHostMalloc(&c->host, host_bytes, hipHostMallocDefault) == hipSuccess) return true;
             (void)hipGetLastError();
             c->host = nullptr;
-            context_destroy(c);
-            return nullptr;
+            return false;
+        };
+        if (!take()) {
+            pool_release_all();   // the idle contexts' buffers
+            if (!take()) {
+                context_destroy(c);
+                return HJM_ERR_ALLOC;
+            }
         }
         c->host_bytes = host_bytes;
     }
-    return c;
+    *out = c;
+    return HJM_OK;
 }
 
 void context_release(PlanContext* c)

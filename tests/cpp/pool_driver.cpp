@@ -37,12 +37,27 @@ static void blocks_of_a_failed_stream()
     CHECK(h.take(0, 64) == HJM_OK && !h.c->stream->bad);
 }
 
+// A pinned buffer that cannot be had is an allocation failure, as a device block is, and is
+// reported only after the idle contexts' buffers were given back.
+static void pinned_buffers_that_cannot_be_had()
+{
+    ContextHolder a, b, c, d;
+    CHECK(a.take(0, 1 << 20) == HJM_OK && b.take(0, 1 << 20) == HJM_OK);
+    a.give();
+    b.give();
+    fake::pinned_budget = 5 << 19;   // two and a half such buffers
+    CHECK(c.take(0, 2 << 20) == HJM_OK);   // one context's buffer grows, the other's goes
+    CHECK(d.take(0, 1 << 20) == HJM_ERR_ALLOC);
+    CHECK(d.c == nullptr && fake::streams.size() == 1 && fake::pinned.size() == 1 && fake::bad_frees == 0);
+}
+
 int main(int argc, char** argv)
 {
     const struct {
         const char* name;
         void (*run)();
-    } checks[] = {{"blocks_of_a_failed_stream", blocks_of_a_failed_stream}};
+    } checks[] = {{"blocks_of_a_failed_stream", blocks_of_a_failed_stream},
+                  {"pinned_buffers_that_cannot_be_had", pinned_buffers_that_cannot_be_had}};
     for (const auto& c : checks)
         if (argc == 2 && !strcmp(argv[1], c.name)) {
             c.run();
