@@ -1,6 +1,7 @@
 // hjm_pool.hip -- the device-memory and plan-context cache of hjm_pool.h (host code).
 #include "hjm_pool.h"
 
+#include <algorithm>
 #include <deque>
 #include <mutex>
 #include <new>
@@ -32,13 +33,21 @@ Pool& pool()
     return *p;
 }
 
-// Sizes in steps of 1/8 of their power of two, at least 512 bytes: repeated calls of nearby
-// sizes share blocks, and a block is at most 1/8 larger than asked for.
+// Sizes in steps of 1/8 of their power of two, at least 512 bytes and at most 2 MB: repeated
+// calls of nearby sizes share blocks. What is too large to be kept is not rounded.
 size_t rounded(size_t bytes)
 {
+    if (bytes > kPoolBytes) return bytes;
     size_t step = 512;
-    while (step * 16 < bytes) step *= 2;
+    while (step * 16 < bytes && step < ((size_t)2 << 20)) step *= 2;
     return (bytes + step - 1) / step * step;
+}
+
+// A kept block serves a request of `want` bytes if it is larger by no more than 1/8, or 16 MB:
+// what a plan holds beyond its needs does not decide whether it fits the card.
+bool serves(size_t bytes, size_t want)
+{
+    return bytes >= want && bytes - want <= std::min(want / 8, (size_t)16 << 20);
 }
 
 void device_free(const Block& b)
@@ -71,14 +80,14 @@ hipError_t pool_alloc(void** out, size_t bytes)
     int device = -1;
     hipError_t err = hipGetDevice(&device);
     if (err != hipSuccess) return err;
-    const size_t want = rounded(bytes);
+    size_t want = rounded(bytes);
     Pool& q = pool();
     try {
         {
             std::lock_guard<std::mutex> lock(q.m);
             auto best = q.idle.end();
             for (auto it = q.idle.begin(); it != q.idle.end(); ++it)
-                if (it->device == device && it->bytes >= want && it->bytes <= want + want / 8 &&
+                if (it->device == device && serves(it->bytes, want) &&
                     (best == q.idle.end() || it->bytes < best->bytes))
                     best = it;
             if (best != q.idle.end()) {
@@ -94,7 +103,7 @@ hipError_t pool_alloc(void** out, size_t bytes)
         if (err != hipSuccess) {
             (void)hipGetLastError();
             pool_release_all();
-            err = hipMalloc(&p, want);
+            err = hipMalloc(&p, want = bytes);
             if (err != hipSuccess) {
                 (void)hipGetLastError();
                 return err;

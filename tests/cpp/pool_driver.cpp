@@ -51,12 +51,36 @@ static void pinned_buffers_that_cannot_be_had()
     CHECK(d.c == nullptr && fake::streams.size() == 1 && fake::pinned.size() == 1 && fake::bad_frees == 0);
 }
 
+// What fits the card is not refused for being rounded up: one block too large to be kept, several
+// that could be, and a card with less than a rounding left.
+static void memory_close_to_the_cards()
+{
+    const size_t gb = (size_t)1 << 30;
+    char *a = nullptr, *b[10] = {}, *c = nullptr;
+    fake::budget = 20 * gb - gb / 20;
+    CHECK(dev_alloc(&a, 20 * gb - gb / 10) == HJM_OK);
+    dev_free(true, a);
+    CHECK(fake::device.empty());
+    fake::budget = 43 * gb + 10 * ((size_t)2 << 20);
+    for (auto& p : b) CHECK(dev_alloc(&p, 43 * (gb / 10)) == HJM_OK);
+    // blocks kept are not handed to requests far smaller
+    const int before = fake::mallocs;
+    for (auto& p : b) dev_free(true, p);
+    CHECK(dev_alloc(&c, 4 * gb) == HJM_OK && fake::mallocs > before);
+    dev_free(true, c);
+    pool_release_all();
+    CHECK(fake::device.empty());
+    fake::budget = 1000001;   // rounded: 1048576
+    CHECK(dev_alloc(&c, 1000001) == HJM_OK);
+}
+
 int main(int argc, char** argv)
 {
     const struct {
         const char* name;
         void (*run)();
     } checks[] = {{"blocks_of_a_failed_stream", blocks_of_a_failed_stream},
+                  {"memory_close_to_the_cards", memory_close_to_the_cards},
                   {"pinned_buffers_that_cannot_be_had", pinned_buffers_that_cannot_be_had}};
     for (const auto& c : checks)
         if (argc == 2 && !strcmp(argv[1], c.name)) {
