@@ -72,7 +72,7 @@ struct ContextHolder {
         return context_acquire(device, host_bytes, &c);
     }
     // false: the stream is in error and nothing that it used may be handed out again (dev_free)
-    [[nodiscard]] bool quiesce() { return !c || hipStreamSynchronize(c->stream) == hipSuccess; }
+    [[nodiscard]] bool quiesce() { return !c || context_quiesce(c); }
     void give()
     {
         context_release(c);

@@ -17,6 +17,7 @@ struct Block {
     void* p;
     size_t bytes;
     int device;
+    unsigned long long id;   // the runtime's number of the allocation; 0: unknown
 };
 
 struct Pool {
@@ -50,8 +51,25 @@ bool serves(size_t bytes, size_t want)
     return bytes >= want && bytes - want <= std::min(want / 8, (size_t)16 << 20);
 }
 
+// The number of the allocation that p belongs to (an address comes back, its number does not);
+// 0 if it belongs to none.
+unsigned long long buffer_id(void* p)
+{
+    unsigned long long id = 0;
+    if (hipPointerGetAttribute(&id, HIP_POINTER_ATTRIBUTE_BUFFER_ID, (hipDeviceptr_t)p) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    return id;
+}
+
+// a device reset has ended it
+bool gone(const Block& b) { return b.id != 0 && buffer_id(b.p) != b.id; }
+bool gone(const PlanContext& c) { return c.mark_id != 0 && buffer_id(c.mark) != c.mark_id; }
+
 void device_free(const Block& b)
 {
+    if (gone(b)) return;
     int prev = -1;
     (void)hipGetDevice(&prev);
     if (prev != b.device) (void)hipSetDevice(b.device);
@@ -64,10 +82,13 @@ void context_destroy(PlanContext* c)
     int prev = -1;
     (void)hipGetDevice(&prev);
     if (prev != c->device) (void)hipSetDevice(c->device);
-    if (c->host) (void)hipHostFree(c->host);
-    for (auto& e : c->ev)
-        if (e) (void)hipEventDestroy(e);
-    if (c->stream) (void)hipStreamDestroy(c->stream);
+    if (c->host && buffer_id(c->host) == c->host_id) (void)hipHostFree(c->host);
+    if (!gone(*c)) {
+        for (auto& e : c->ev)
+            if (e) (void)hipEventDestroy(e);
+        if (c->stream) (void)hipStreamDestroy(c->stream);
+        if (c->mark) (void)hipFree(c->mark);
+    }
     if (prev >= 0 && prev != c->device) (void)hipSetDevice(prev);
     delete c;
 }
@@ -85,15 +106,18 @@ hipError_t pool_alloc(void** out, size_t bytes)
     try {
         {
             std::lock_guard<std::mutex> lock(q.m);
-            auto best = q.idle.end();
-            for (auto it = q.idle.begin(); it != q.idle.end(); ++it)
-                if (it->device == device && serves(it->bytes, want) &&
-                    (best == q.idle.end() || it->bytes < best->bytes))
-                    best = it;
-            if (best != q.idle.end()) {
+            for (;;) {
+                auto best = q.idle.end();
+                for (auto it = q.idle.begin(); it != q.idle.end(); ++it)
+                    if (it->device == device && serves(it->bytes, want) &&
+                        (best == q.idle.end() || it->bytes < best->bytes))
+                        best = it;
+                if (best == q.idle.end()) break;
                 const Block b = *best;
-                q.live.emplace(b.p, b);
+                const bool usable = !gone(b);
+                if (usable) q.live.insert_or_assign(b.p, b);
                 q.idle.erase(best);
+                if (!usable) continue;
                 *out = b.p;
                 return hipSuccess;
             }
@@ -111,7 +135,8 @@ hipError_t pool_alloc(void** out, size_t bytes)
         }
         try {
             std::lock_guard<std::mutex> lock(q.m);
-            q.live.emplace(p, Block{p, want, device});
+            // (an entry of that address is of a plan that a device reset has outlived)
+            q.live.insert_or_assign(p, Block{p, want, device, buffer_id(p)});
         } catch (...) {
             (void)hipFree(p);
             return hipErrorOutOfMemory;
@@ -128,14 +153,14 @@ void pool_free(void* p, bool idle)
     if (!p) return;
     Pool& q = pool();
     std::vector<Block> drop;
-    Block b{p, 0, 0};
+    Block b{p, 0, 0, 0};
     try {
         std::lock_guard<std::mutex> lock(q.m);
         const auto it = q.live.find(p);
         if (it != q.live.end()) {
             b = it->second;
             q.live.erase(it);
-            if (idle && b.bytes <= kPoolBytes) {
+            if (idle && b.bytes <= kPoolBytes && b.id != 0 && !gone(b)) {
                 size_t held = b.bytes;
                 for (const Block& x : q.idle) held += x.device == b.device ? x.bytes : 0;
                 for (auto x = q.idle.begin(); held > kPoolBytes && x != q.idle.end();) {
@@ -180,14 +205,22 @@ int context_acquire(int device, size_t host_bytes, PlanContext** out)
     *out = nullptr;
     Pool& q = pool();
     PlanContext* c = nullptr;
-    {
-        std::lock_guard<std::mutex> lock(q.m);
-        for (size_t i = q.contexts.size(); i-- > 0;)
-            if (q.contexts[i]->device == device) {
-                c = q.contexts[i];
-                q.contexts.erase(q.contexts.begin() + (std::ptrdiff_t)i);
-                break;
-            }
+    for (bool found = true; found && !c;) {
+        {
+            std::lock_guard<std::mutex> lock(q.m);
+            found = false;
+            for (size_t i = q.contexts.size(); i-- > 0;)
+                if (q.contexts[i]->device == device) {
+                    c = q.contexts[i];
+                    q.contexts.erase(q.contexts.begin() + (std::ptrdiff_t)i);
+                    found = true;
+                    break;
+                }
+        }
+        if (c && gone(*c)) {
+            context_destroy(c);
+            c = nullptr;
+        }
     }
     if (!c) {
         c = new (std::nothrow) PlanContext();
@@ -195,6 +228,8 @@ int context_acquire(int device, size_t host_bytes, PlanContext** out)
         c->device = device;
         bool ok = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) == hipSuccess;
         for (auto& e : c->ev) ok = ok && hipEventCreate(&e) == hipSuccess;
+        ok = ok && hipMalloc(&c->mark, 512) == hipSuccess;
+        c->mark_id = ok ? buffer_id(c->mark) : 0;
         if (!ok) {
             (void)hipGetLastError();
             context_destroy(c);
@@ -219,16 +254,19 @@ int context_acquire(int device, size_t host_bytes, PlanContext** out)
             }
         }
         c->host_bytes = host_bytes;
+        c->host_id = buffer_id(c->host);
     }
     *out = c;
     return HJM_OK;
 }
 
+bool context_quiesce(PlanContext* c) { return gone(*c) || hipStreamSynchronize(c->stream) == hipSuccess; }
+
 void context_release(PlanContext* c)
 {
     if (!c) return;
-    const bool idle = hipStreamSynchronize(c->stream) == hipSuccess;
-    if (idle) {
+    const bool idle = context_quiesce(c);
+    if (idle && c->mark_id != 0 && !gone(*c)) {
         Pool& q = pool();
         try {
             std::lock_guard<std::mutex> lock(q.m);

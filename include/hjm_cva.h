@@ -121,7 +121,9 @@ int hjm_device_count(int* count);
 /* The library keeps up to 8 GB per device of the memory that destroyed plans and finished
  * calls used, with a few streams, for those that follow (mapping fresh device memory costs
  * more than most runs). This returns all of it to the device; plans in use are not touched.
- * A failed allocation does the same by itself before it is reported. */
+ * A failed allocation does the same by itself before it is reported. hipDeviceReset ends what
+ * is kept as it ends everything else on the device; the library notices and starts afresh
+ * (plans from before it must not be used any more, only destroyed). */
 void hjm_release_cached_memory(void);
 
 /* CVA weights w_j = (1-R) * trapezoid share of the default probability of

@@ -27,6 +27,7 @@ struct FakeStream {
 struct FakeEvent {};
 typedef FakeStream* hipStream_t;
 typedef FakeEvent* hipEvent_t;
+typedef void* hipDeviceptr_t;
 enum { hipStreamNonBlocking = 1, hipHostMallocDefault = 0 };
 enum hipPointer_attribute { HIP_POINTER_ATTRIBUTE_BUFFER_ID = 7 };
 

@@ -21,7 +21,7 @@ def driver(tmp_path_factory):
 
 
 @pytest.mark.parametrize("check", ["blocks_of_a_failed_stream", "pinned_buffers_that_cannot_be_had",
-                                   "memory_close_to_the_cards"])
+                                   "memory_close_to_the_cards", "a_device_reset"])
 def test_pool(driver, check):
     r = subprocess.run([driver, check], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout + r.stderr
