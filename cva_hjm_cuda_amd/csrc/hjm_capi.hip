@@ -68,6 +68,7 @@ struct hjm_plan_s {
     MfmaGrid mg{};
     uint16_t* d_wfrag = nullptr;  // bf16 parts of the block map (FP32 plans)
     double* d_wfrag64 = nullptr;  // the block map's FP64 fragments (FP64 plans)
+    std::vector<double> wfrag64;  // what its asynchronous upload reads, also if creation fails
     double* d_normals = nullptr;
     double* d_nx = nullptr;
     double* d_ny = nullptr;
@@ -193,16 +194,14 @@ int plan_init(hjm_plan p, const hjm_market* market, const hjm_swap* swap, const 
             kTenors, bracket_plan(cfg->paths, p->pfe_rank, sizeof(double)), sizeof(double));
         if (wsb) HJM_TRY(dev_alloc(&p->d_selws, wsb));
     }
-    // host copies of the block map, kept until the stream is synchronised below
-    std::vector<double> wf64;
     if (p->use_mfma) {
         int scale = 0;
         if (cfg->precision == HJM_FP64) {
             HJM_HIP(mfma64_kernels_prepare(), HJM_ERR_DEVICE);
             build_mfma64_block_map(market->drifts, market->volatilities, cfg->dt, swap->dtau,
-                                   ref_mfma_tiles(D), wf64);
-            HJM_TRY(dev_alloc(&p->d_wfrag64, wf64.size()));
-            HJM_HIP(hipMemcpyAsync(p->d_wfrag64, wf64.data(), wf64.size() * sizeof(double),
+                                   ref_mfma_tiles(D), p->wfrag64);
+            HJM_TRY(dev_alloc(&p->d_wfrag64, p->wfrag64.size()));
+            HJM_HIP(hipMemcpyAsync(p->d_wfrag64, p->wfrag64.data(), p->wfrag64.size() * sizeof(double),
                                    hipMemcpyHostToDevice, p->stream),
                     HJM_ERR_DEVICE);
         } else {

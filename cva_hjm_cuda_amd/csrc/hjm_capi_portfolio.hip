@@ -52,8 +52,12 @@ struct hjm_pplan_s {
     uint32_t* d_loparts = nullptr;  // counts below the bracket per row and statistics workgroup
     double* d_coef = nullptr;
     double* d_a = nullptr;
-    int* d_book_ints = nullptr;      // the swap list: set offsets, periods
-    double* d_book_reals = nullptr;  // signed notionals, coupons
+    // the swap list: set offsets, periods; signed notionals, coupons. The host copies are the
+    // plan's, since an asynchronous upload may still read them when its creation fails
+    std::vector<int> book_ints;
+    std::vector<double> book_reals;
+    int* d_book_ints = nullptr;
+    double* d_book_reals = nullptr;
     int* d_kmax = nullptr;
     double* d_w = nullptr;
     uint16_t* d_vfrag = nullptr;  // FP32: bf16 parts of -gamma (matrix-core valuation)
@@ -190,8 +194,11 @@ int pplan_init(hjm_portfolio_plan p, const hjm_market* market, const hjm_portfol
         cva_weights(nd, pf->dtau, pf->hazard_rate[s], pf->recovery, &p->w[(size_t)s * nd]);
     // the swaps grouped by set, in the caller's order within a set
     const int G = pf->nsets, N = pf->nswaps;
-    std::vector<int> order((size_t)N), ints((size_t)G + 1 + N, 0);
-    std::vector<double> reals(2 * (size_t)N);
+    std::vector<int> order((size_t)N);
+    std::vector<int>& ints = p->book_ints;
+    std::vector<double>& reals = p->book_reals;
+    ints.assign((size_t)G + 1 + N, 0);
+    reals.resize(2 * (size_t)N);
     int* first = ints.data();
     for (int s = 0; s < N; ++s) ++first[pf->netting_set[s] + 1];
     for (int g = 0; g < G; ++g) first[g + 1] += first[g];
@@ -311,7 +318,6 @@ int pplan_init(hjm_portfolio_plan p, const hjm_market* market, const hjm_portfol
             mg.spot64[j] = market->spot_rates[j];
         }
     }
-    // the host copies above go with this call
     HJM_HIP(hipStreamSynchronize(st), HJM_ERR_DEVICE);
     return HJM_OK;
 }
