@@ -25,7 +25,20 @@ struct SweepBuffers {
     int rows = 0;             // 16 x row tiles
 
     // Allocates for g.paths paths and builds the maps; stored: the forward keeps the shocks.
+    // What could be had of the memory is given back if the rest cannot (the VALU sweep's
+    // buffers are allocated then).
     int take(SweepGrid& g, bool pf, double c, int nsteps, bool stored, hipStream_t st)
+    {
+        const int rc = allocate(g, pf, nsteps, stored);
+        if (rc != HJM_OK) {
+            free(true);
+            return rc;
+        }
+        HJM_HIP(launch_sweep_map(c, pf, map, ptab, st), HJM_ERR_LAUNCH);
+        return HJM_OK;
+    }
+
+    int allocate(SweepGrid& g, bool pf, int nsteps, bool stored)
     {
         if (g.paths > kSweepMaxPaths) return HJM_ERR_UNSUPPORTED;
         g.units = sweep_units(g.paths);
@@ -43,7 +56,6 @@ struct SweepBuffers {
             if (!chunk) HJM_TRY(dev_alloc(&chunk, (size_t)n * per / sizeof(float) + kSweepSlack));
             chunk_paths = n * group;
         }
-        HJM_HIP(launch_sweep_map(c, pf, map, ptab, st), HJM_ERR_LAUNCH);
         return HJM_OK;
     }
 

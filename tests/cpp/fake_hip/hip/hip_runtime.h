@@ -105,6 +105,9 @@ inline hipError_t hipPointerGetAttribute(void* out, hipPointer_attribute, void* 
     }
     return hipErrorInvalidValue;
 }
+enum hipMemcpyKind { hipMemcpyHostToDevice, hipMemcpyDeviceToHost };
+inline hipError_t hipMemsetAsync(void*, int, size_t, hipStream_t) { return hipSuccess; }
+inline hipError_t hipMemcpyAsync(void*, const void*, size_t, hipMemcpyKind, hipStream_t) { return hipSuccess; }
 inline hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned)
 {
     fake::streams.insert(*s = new FakeStream());
