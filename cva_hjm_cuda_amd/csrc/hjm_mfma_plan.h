@@ -245,11 +245,13 @@ struct BlockMapParams {
     int scale;               // k
 };
 
-// k is the power of two that brings the largest shock entry to [2^12, 2^13), where both parts
-// of every entry within 2^-26 of it are normal fp16 numbers (without the scale the entries,
-// 1e-4 .. 1e-2, would leave their low parts to subnormals). The kernels hold the curve and
-// the integrals times 2^k too, so both kinds of products share an accumulator; k is also
-// bounded by the curve's size (max |spot| 2^k <= 2^40), and 0 without shocks.
+// k is the power of two that brings the largest shock entry (the drift's and the integral rows'
+// among them) to [2^12, 2^13); without it the entries, 1e-4 .. 1e-2, would leave their low parts
+// to fp16's subnormals. An entry down to 2^-14 of the largest keeps 22 bits in its two parts, a
+// smaller one an absolute 2^-37 of the largest. The kernels hold the curve and the integrals times
+// 2^k too, so both kinds of products share the final sum; k is bounded by the curve's size
+// (max |spot| 2^k < 2^40, so that 25 years of integrals stay far from FP32's end; shocks that
+// this leaves below 2^12 are under 2^-27 of the curve), and 0 without shocks.
 inline BlockMapParams block_map_params(const double* spot, const double* drift, const double* vols, double dt,
                                        double dtau, int mtiles, MfmaMap map = MfmaMap::kReference)
 {
@@ -302,7 +304,7 @@ inline BlockMapParams block_map_params(const double* spot, const double* drift, 
     }
     if (top > 0.0) {
         p.scale = std::max(-120, std::min(120, 12 - ilogb(top)));
-        if (curve > 0.0) p.scale = std::min(p.scale, std::max(12 - ilogb(top) - 40, 39 - ilogb(curve)));
+        if (curve > 0.0) p.scale = std::min(p.scale, 39 - ilogb(curve));
     }
     p.up = ldexp(1.0, p.scale);
     return p;
