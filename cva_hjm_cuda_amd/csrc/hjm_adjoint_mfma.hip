@@ -146,9 +146,13 @@ void adjoint_mfma_kernel(const SweepGrid g, const u4_t* __restrict__ map, const 
         load_tile(g.hi, 2, zb[0]);
         load_tile(g.hi, 3, zb[1]);
         __syncthreads();   // the unit before is read (and the map and table are there)
-        // rows 48 .. 16 R - 1 start at zero: the mu rows not yet injected, and the padding
+        // rows 48 .. 16 R - 1 start at zero: the mu rows not yet injected, and the padding; by the
+        // lane that also writes them
+        if (grp == 0) {
 #pragma unroll
-        for (int m = 3; m < R; ++m) *reinterpret_cast<f4_t*>(mine + 16 * m + 4 * grp) = f4_t{0.f, 0.f, 0.f, 0.f};
+            for (int q = 0; q < 4 * (R - 3); ++q)
+                *reinterpret_cast<f4_t*>(mine + 48 + 4 * q) = f4_t{0.f, 0.f, 0.f, 0.f};
+        }
 
         auto write_rows = [&]() {
 #pragma unroll
