@@ -512,7 +512,7 @@ def calculate_exposure_multi_gpu(expected_exposure: np.ndarray, payOff: Interest
 @dataclass
 class Tuning:
     """Launch shapes of a portfolio plan (0: the kernel's default; see hjm_tuning)."""
-    block_size: int = 256          # VALU path kernel
+    block_size: int = 256          # path kernel of one path per lane
     blocks_per_cu: int = 0         # persistent path kernel (matrix-core: 0 or 1)
     use_graph: bool = False
     fuse_statistics: bool = False  # FP32: valuation and statistics in one pass
@@ -622,9 +622,8 @@ def autotune_portfolio(market: Market, portfolio, paths: int, horizon: float = 3
     """Fastest launch shapes for this problem, measured on the device: returns (Tuning
     with use_graph set, eager ms of one execute with it). Matrix-core FP32 plans tune the
     path kernel (N-tiles, waves, persistent grid), the valuation (N-tiles, waves, LDS
-    stage) and the fused against the exposure pass; VALU path kernels their block size
-    and persistent grid; FP64 plans on the matrix cores keep the defaults
-    (hjm_portfolio_autotune)."""
+    stage) and the fused against the exposure pass; FP32 paths of one per lane their block
+    size and persistent grid; FP64 plans keep the defaults (hjm_portfolio_autotune)."""
     mk = market._c()
     pfc = _pf_c(portfolio, horizon, recovery)
     cfg = _config(paths, dt, precision, RNG_PHILOX, seed, None, 0.0, recovery, pfe_quantile,

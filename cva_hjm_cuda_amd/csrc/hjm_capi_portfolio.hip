@@ -721,7 +721,11 @@ int hjm_portfolio_autotune(const hjm_market* market, const hjm_portfolio* portfo
 {
     if (!best || !config || !portfolio) return HJM_ERR_NULL;
     hjm_config cfg = *config;
-    if (cfg.rng == HJM_RNG_HOST) cfg.rng = HJM_RNG_PHILOX;
+    // FP64 runs on host normals have a path kernel of their own, the one that FP64's launch fields
+    // are for; it is tuned on the first of the caller's normals. The others are tuned on the
+    // generator's.
+    const bool host64 = cfg.precision == HJM_FP64 && cfg.path_kernel != HJM_KERNEL_MATRIX && cfg.host_normals;
+    if (cfg.rng == HJM_RNG_HOST && !host64) cfg.rng = HJM_RNG_PHILOX;
     // the VALU path kernel's cost is linear in the horizon: it is tuned on two dates
     hjm_portfolio short_pf = *portfolio;
     std::vector<int32_t> per;
@@ -731,7 +735,7 @@ int hjm_portfolio_autotune(const hjm_market* market, const hjm_portfolio* portfo
     int nd = 0;
     HJM_TRY(check_portfolio(portfolio, &nd));
     if (!mfma) {
-        short_pf.horizon = 2.0 * portfolio->dtau;
+        short_pf.horizon = std::min(portfolio->horizon, 2.0 * portfolio->dtau);
         per.assign(portfolio->periods, portfolio->periods + portfolio->nswaps);
         for (auto& x : per) x = std::min(x, 2);
         short_pf.periods = per.data();
@@ -804,8 +808,8 @@ int hjm_portfolio_autotune(const hjm_market* market, const hjm_portfolio* portfo
             if (rc == HJM_OK) passes[fuse] = ms[4] - ms[0];
         }
         bt.fuse_statistics = passes[1] < passes[0] ? 1 : 0;
-    } else if (p->precision != HJM_FP64) {
-        // (the FP64 path kernels choose their shape by the path count: nothing to sweep)
+    } else if (p->precision != HJM_FP64 || p->d_normals) {
+        // (FP64 path kernels on the generator's normals have a shape by path count, or one shape)
         double bv = 1e300;
         for (int bs : {64, 128, 256})
             for (int bpc : {0, 1, 2, 4, 8}) {

@@ -215,14 +215,16 @@ typedef struct {
 } hjm_portfolio;
 
 /* Launch shapes of the portfolio plan's kernels (0 in a field: its default). The VALU
- * path kernel (FP64, host normals, or path_kernel = VECTOR) uses block_size and
- * blocks_per_cu; the matrix-core FP32 path kernel path_tiles, path_waves and
- * blocks_per_cu (0 or 1: one workgroup per CU); the
- * matrix-core valuation value_tiles, value_waves and value_stage. The FP64 matrix-core
- * path kernel (FP64 with path_kernel = MATRIX) has a fixed shape. Results do not depend
- * on the shapes. hjm_portfolio_autotune measures them. */
+ * path kernel of one path per lane (host normals, or FP32 with path_kernel = VECTOR) uses
+ * block_size and blocks_per_cu; the matrix-core FP32 path kernel path_tiles, path_waves and
+ * blocks_per_cu (0 or 1: one workgroup per CU); the matrix-core valuation value_tiles,
+ * value_waves and value_stage. FP64 plans on the generator's normals ignore the path fields
+ * (they are checked all the same): several lanes per path by path count, or the one shape of the
+ * FP64 matrix-core kernel (path_kernel = MATRIX). Results do not depend on the shapes.
+ * hjm_portfolio_autotune measures them. */
 typedef struct {
-    int32_t block_size;     /* threads per workgroup of the VALU path kernel: 64, 128 or 256 */
+    int32_t block_size;     /* threads per workgroup of the path kernel of one path per lane:
+                               64, 128 or 256 */
     int32_t blocks_per_cu;  /* persistent path kernel: grid = blocks_per_cu x CUs workgroups
                                looping over the groups of paths; 0 = one workgroup per group */
     int32_t use_graph;      /* capture all passes in one hipGraph, replay it per execute */
@@ -272,9 +274,9 @@ int hjm_portfolio_cva_greeks(const hjm_market* market, const hjm_portfolio* port
  * (use_graph set) and the eager time of one execute with it into *best_ms. Matrix-core
  * FP32 plans: the path kernel over its four shapes x {one workgroup per group, persistent
  * one per CU}, the valuation over tiles x waves x LDS stage, then the exposure pass
- * against the fused valuation-statistics pass. VALU path kernels: block sizes {64, 128,
- * 256} x persistent grids {0, 1, 2, 4, 8 workgroups per CU} on a 2-date horizon. FP64
- * plans on the matrix cores (path_kernel = MATRIX) have no shape to choose: defaults. */
+ * against the fused valuation-statistics pass. Path kernels of one path per lane: block sizes {64, 128,
+ * 256} x persistent grids {0, 1, 2, 4, 8 workgroups per CU} on a 2-date horizon (FP64: on the
+ * first host normals). FP64 plans on the generator's normals have no shape to choose: defaults. */
 int hjm_portfolio_autotune(const hjm_market* market, const hjm_portfolio* portfolio,
                            const hjm_config* config, hjm_tuning* best, double* best_ms);
 
