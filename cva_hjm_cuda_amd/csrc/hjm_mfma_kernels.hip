@@ -4,10 +4,10 @@
 // (hjm_mfma_plan.h), computed on the matrix cores with split operands: the curve columns with
 // v_mfma_f32_16x16x32_bf16 as six products of three-way bf16 splits (W's parts precomputed,
 // the operand split exactly in registers), the shock columns with v_mfma_f32_16x16x32_f16 as
-// three products of two-way fp16 splits (22 bits of a term that is a few percent of the
-// curve; 258 products per wave-block at 5 M-tiles against 408 with bf16 throughout, and 1.5
-// instead of 5.5 VALU instructions to split a shock: the 10y path kernel at 131072 paths went
-// from 0.51 to 0.42 ms, its results' error against FP64 unchanged). The split products
+// three products of two-way fp16 splits (258 products per wave-block at 5 M-tiles against 408
+// with bf16 throughout, and 1.5 instead of 5.5 VALU instructions to split a shock: the 10y path
+// kernel at 131072 paths went from 0.55 to 0.44 ms; its forwards' error against FP64, with the
+// accumulators apart, from 2.0e-7 to 1.26e-7). The split products
 // keep FP32 accuracy while running on the matrix cores concurrently with the VALU
 // (FP32 MFMA on gfx950 shares the vector pipeline and gains nothing over it). A wave owns
 // 32 paths = 2 N-tiles of 16 (the portfolio kernel's shape is a launch choice). The
@@ -49,9 +49,9 @@ __host__ __device__ constexpr int shock_chunk_last_quad(int s)
 // Issue plan: the matrix-core work of the block is spread over the quads that generate
 // shocks, so that their RNG (VALU) runs beside a share of the MFMAs: chunk c's M-tiles
 // [m0, m1) go to quad q. Quads 3, 7 and 11 make no Philox call (their shocks come from
-// calls made earlier) and get no MFMA work; curve chunks 0, 1 (six products a tile) are
-// ready at the start, shock chunk s (three products) once its last shock's call is made
-// (quads 1, 4, 6, 9, 12); shock chunk 4 completes with the last quad and runs after it.
+// calls made earlier) and get no MFMA work; curve chunks 0, 1 (six products a
+// tile, or five and the sixth, Wh xh, last) are ready at the start, shock chunk s (three
+// products) once its last shock's call is made (quads 1, 4, 6, 9, 12); shock chunk 4 completes with the last quad and runs after it.
 struct IssueSlot {
     int chunk, m0, m1;
 };
@@ -83,49 +83,53 @@ __device__ __forceinline__ void for_each_index(F& f, std::integer_sequence<int, 
 
 // One 50-step block: acc = W x [fin; shocks of steps b*50 .. b*50+49; 1]. kStore: also
 // write the block's normals to zs[step][factor][path] (FP32) for a later reverse sweep.
-// kSplitAcc: three accumulators, added up (rounded) once at the end: the curve's Wh xh, the
-// shocks' Wh xh, and every smaller product. The matrix cores truncate a product's sum at the
-// accumulator's size (measured: C = 1 plus 32 products of 2^-27 returns 1; small positive
-// contributions are lost, small negative ones kept). The curve's Wh xh are 16-bit products,
-// which such a sum holds whole; the shocks' are 22 bits wide and are a few percent of the
-// curve, whose accumulator would cut their low bits; with the small products they would cut
-// those. A path's forwards over 10y against FP64, rms relative: 2.1e-7 with the shocks' Wh xh in
-// the curve's accumulator, 1.35e-7 in the small products', 1.26e-7 apart (2.0e-7 with three
-// bf16 parts and two accumulators). It costs 8 registers per tile and N-tile over two
-// accumulators' and 2 % of the reference kernel's time at 131072 paths x 10y (0.43 to 0.44 ms;
-// 12 % where it stores the shocks), 4 % of the portfolio's.
-template <int MT, int NT, bool kStore, bool kInterleave, bool kSplitAcc>
+// Three accumulators, added up (rounded) once at the end: the curve's Wh xh, the shocks' Wh xh,
+// and every smaller product (kSplitAcc; otherwise, past 5 live M-tiles, for want of registers, the
+// last two are one). The matrix cores truncate a product's sum at the accumulator's size
+// (measured: C = 1 plus 32 products of 2^-27 returns 1; small positive contributions are
+// lost, small negative ones kept). The curve's Wh xh are 16-bit products, which such a sum
+// holds whole; the shocks' are 22 bits wide, and the curve's accumulator would cut their low
+// bits; with the small products they would cut those. Forwards against FP64, rms relative:
+//   10y (5 tiles) 2.1e-7 with the shocks' Wh xh in the curve's accumulator, 1.35e-7 in the small
+//     products', 1.26e-7 apart (2.0e-7 with three bf16 parts and two accumulators);
+//   25y (7 tiles) 6.1e-6 with one accumulator, 1.2e-6 with two; EE 6.6e-7 and 3.6e-7, PFE 3.0e-6 and
+//     5.9e-7 (three bf16 parts and one accumulator 1.2e-6 and 4.0e-6).
+// kLate: the curve's products come last, a tile at a time, in registers that nothing else needs
+// by then; for the reference kernels, which have none to spare (stored shocks at 65536 paths x
+// 10y: 0.295 ms, 0.325 with 8 more registers per tile and N-tile). The portfolio's, with 4
+// tiles and no MFMA schedule of its own, spills less the other way ({1, 16} at 262144 paths x 30y:
+// 2.13 ms, 2.29 late). The same sums either way.
+template <int MT, int NT, bool kStore, bool kInterleave, bool kSplitAcc, bool kLate>
 __device__ __forceinline__ void mfma_block(const u4_t* __restrict__ lds_w, const float (&fin)[NT][16],
                                            f4_t (&acc)[MT][NT], const MfmaGrid& g,
                                            const int64_t (&path)[NT], const bool (&live)[NT],
                                            int b, int grp, int lane, float* __restrict__ zs)
 {
     constexpr int MS = kSplitAcc ? MT : 1;
-    f4_t shock[MS][NT], small[MS][NT];
+    f4_t small[MS][NT], curve[kLate ? 1 : MT][NT];
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
             acc[m][n] = f4_t{0.f, 0.f, 0.f, 0.f};
-            if constexpr (kSplitAcc) shock[m][n] = small[m][n] = f4_t{0.f, 0.f, 0.f, 0.f};
+            if constexpr (kSplitAcc) small[m][n] = f4_t{0.f, 0.f, 0.f, 0.f};
+            if constexpr (!kLate) curve[m][n] = f4_t{0.f, 0.f, 0.f, 0.f};
         }
     // W's fragments are the same in every block: an opaque offset keeps their LDS reads
     // inside the block instead of hoisted (hundreds of registers) out of the block loop
     uint32_t off = (uint32_t)lane;
     asm volatile("" : "+v"(off));
     // one product for the N-tiles in turn (consecutive MFMAs then write different
-    // accumulators)
-    enum Kind { kCurve, kShock, kSmall };
-    auto product = [&](int m, Kind kind, u4_t a, auto fn) {
+    // accumulators): large = the shocks' Wh xh
+    auto product = [&](int m, bool large, u4_t a, auto fn) {
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
-            if (kSplitAcc && kind == kSmall) small[kSplitAcc ? m : 0][n] = fn(a, n, small[kSplitAcc ? m : 0][n]);
-            else if (kSplitAcc && kind == kShock) shock[kSplitAcc ? m : 0][n] = fn(a, n, shock[kSplitAcc ? m : 0][n]);
+            if (kSplitAcc && !large) small[kSplitAcc ? m : 0][n] = fn(a, n, small[kSplitAcc ? m : 0][n]);
             else acc[m][n] = fn(a, n, acc[m][n]);
         }
     };
-    // M-tiles [m0, m1) of curve chunk c, less the structurally zero ones (the reference and
-    // portfolio maps share tiles 0..3, whose zeros agree; c and m are constants once
+    // M-tiles [m0, m1) of curve chunk c (kLate: without Wh xh), less the structurally zero ones (the
+    // reference and portfolio maps share tiles 0..3, whose zeros agree; c and m are constants once
     // unrolled), and of a shock chunk
     auto curve_tiles = [&](int c, int m0, int m1, const Split8 (&xs)[NT]) {
 #pragma unroll
@@ -133,12 +137,14 @@ __device__ __forceinline__ void mfma_block(const u4_t* __restrict__ lds_w, const
             if (mfma_chunk_zero(m, c, false)) continue;
             const u4_t* a = lds_w + mfma_frag(m, c, 0) * kWave + off;
             const u4_t ah = a[0], am = a[kWave], al = a[2 * kWave];
-            product(m, kCurve, ah, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].h, v); });
-            product(m, kSmall, ah, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].m, v); });
-            product(m, kSmall, am, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].h, v); });
-            product(m, kSmall, ah, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].l, v); });
-            product(m, kSmall, al, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].h, v); });
-            product(m, kSmall, am, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].m, v); });
+            if constexpr (!kLate)
+#pragma unroll
+                for (int n = 0; n < NT; ++n) curve[m][n] = mfma_bf16(ah, xs[n].h, curve[m][n]);
+            product(m, false, ah, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].m, v); });
+            product(m, false, am, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].h, v); });
+            product(m, false, ah, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].l, v); });
+            product(m, false, al, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].h, v); });
+            product(m, false, am, [&](u4_t w, int n, f4_t v) { return mfma_bf16(w, xs[n].m, v); });
         }
     };
     auto shock_tiles = [&](int c, int m0, int m1, const SplitH8 (&xs)[NT]) {
@@ -146,9 +152,9 @@ __device__ __forceinline__ void mfma_block(const u4_t* __restrict__ lds_w, const
         for (int m = m0; m < m1; ++m) {
             const u4_t* a = lds_w + mfma_frag(m, c, 0) * kWave + off;
             const u4_t ah = a[0], al = a[kWave];
-            product(m, kShock, ah, [&](u4_t w, int n, f4_t v) { return mfma_f16(w, xs[n].h, v); });
-            product(m, kSmall, ah, [&](u4_t w, int n, f4_t v) { return mfma_f16(w, xs[n].l, v); });
-            product(m, kSmall, al, [&](u4_t w, int n, f4_t v) { return mfma_f16(w, xs[n].h, v); });
+            product(m, true, ah, [&](u4_t w, int n, f4_t v) { return mfma_f16(w, xs[n].h, v); });
+            product(m, false, ah, [&](u4_t w, int n, f4_t v) { return mfma_f16(w, xs[n].l, v); });
+            product(m, false, al, [&](u4_t w, int n, f4_t v) { return mfma_f16(w, xs[n].h, v); });
         }
     };
     // split operands: curve chunks from fin (registers 8 c .. 8 c + 7), shock chunk s from
@@ -214,7 +220,7 @@ __device__ __forceinline__ void mfma_block(const u4_t* __restrict__ lds_w, const
             if constexpr (kInterleave) {
                 // within the quad: one MFMA, then a share of the RNG's VALU instructions
 #pragma unroll
-                for (int i = 0; i < (is.m1 - is.m0) * NT * (is.chunk < 2 ? 6 : 3); ++i) {
+                for (int i = 0; i < (is.m1 - is.m0) * NT * (is.chunk < 2 ? (kLate ? 5 : 6) : 3); ++i) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                     __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);
                 }
@@ -225,11 +231,25 @@ __device__ __forceinline__ void mfma_block(const u4_t* __restrict__ lds_w, const
     };
     for_each_index(quad, std::make_integer_sequence<int, kMfmaQuads>{});
     shock_tiles(kMfmaChunks - 1, 0, MT, xs[kMfmaChunks - 3]);
-    if constexpr (kSplitAcc) {
 #pragma unroll
-        for (int m = 0; m < MT; ++m)
+    for (int m = 0; m < MT; ++m) {
+        f4_t(&own)[NT] = curve[kLate ? 0 : m];
+        if constexpr (kLate) {
 #pragma unroll
-            for (int n = 0; n < NT; ++n) acc[m][n] += small[m][n] + shock[m][n];
+            for (int n = 0; n < NT; ++n) own[n] = f4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                if (mfma_chunk_zero(m, c, false)) continue;
+                const u4_t ah = lds_w[mfma_frag(m, c, 0) * kWave + off];
+#pragma unroll
+                for (int n = 0; n < NT; ++n) own[n] = mfma_bf16(ah, xc[c][n].h, own[n]);
+            }
+        }
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            if constexpr (kSplitAcc) acc[m][n] += small[m][n];
+            acc[m][n] += own[n];
+        }
     }
 }
 
@@ -305,8 +325,8 @@ __attribute__((amdgpu_waves_per_eu(path_waves_per_simd(kNT), path_waves_per_simd
 
     for (int b = 1; b < g.ndates; ++b) {
         f4_t acc[MT][kNT];
-        // three accumulators where registers allow (up to 5 live tiles: 255 VGPRs)
-        mfma_block<MT, kNT, kStore, true, (MT <= 5)>(lds_w, fin, acc, g, path, live, b, grp, lane, zs);
+        // three accumulators where registers allow (up to 5 live tiles: 251 VGPRs)
+        mfma_block<MT, kNT, kStore, true, (MT <= 5), true>(lds_w, fin, acc, g, path, live, b, grp, lane, zs);
         // integrals: Kahan-add the block's dA (tiles 3 .. MT-1); curve rows become next input
 #pragma unroll
         for (int n = 0; n < kNT; ++n) {
@@ -418,7 +438,7 @@ __global__ __launch_bounds__((WAVES ? WAVES : max_waves(NT)) * kWave) void pf_pa
             }
             if (e + 1 >= g.ndates) break;
             f4_t acc[kMfmaPfMTiles][NT];
-            mfma_block<kMfmaPfMTiles, NT, kStore, false, true>(lds_w, fin, acc, g, path, live, e, grp, lane,
+            mfma_block<kMfmaPfMTiles, NT, kStore, false, true, false>(lds_w, fin, acc, g, path, live, e, grp, lane,
                                                                zs);
 #pragma unroll
             for (int n = 0; n < NT; ++n) {
@@ -546,7 +566,7 @@ __global__ __launch_bounds__(tile_waves(MT) * kWave, kStore && MT > 4 ? 3 : 4) v
         const int buf = i & 1;
         if (i + 1 < nb) shocks(b0 + i + 1, buf ^ 1);
         if (mine) {
-            f4_t acc = {0.f, 0.f, 0.f, 0.f}, acc_shock = acc, acc_small = acc;
+            f4_t curve = {0.f, 0.f, 0.f, 0.f}, acc = curve, acc_small = curve;
             auto small = [&](auto fn, u4_t a, u4_t x) {
                 if constexpr (kSplitAcc) acc_small = fn(a, x, acc_small);
                 else acc = fn(a, x, acc);
@@ -556,7 +576,7 @@ __global__ __launch_bounds__(tile_waves(MT) * kWave, kStore && MT > 4 ? 3 : 4) v
                 if (c < 1 || !mfma_chunk_zero(wv, c, false)) {
                     const u4_t h = s_c[buf][c][0][lane], m = s_c[buf][c][1][lane], l = s_c[buf][c][2][lane];
                     const u4_t* a = w + 3 * c;
-                    acc = mfma_bf16(a[0], h, acc);
+                    curve = mfma_bf16(a[0], h, curve);
                     small(mfma_bf16, a[0], m);
                     small(mfma_bf16, a[1], h);
                     small(mfma_bf16, a[0], l);
@@ -568,12 +588,12 @@ __global__ __launch_bounds__(tile_waves(MT) * kWave, kStore && MT > 4 ? 3 : 4) v
             for (int c = 0; c < kShockChunks; ++c) {
                 const u4_t h = s_z[buf][c][0][lane], l = s_z[buf][c][1][lane];
                 const u4_t* a = w + 6 + 2 * c;
-                if constexpr (kSplitAcc) acc_shock = mfma_f16(a[0], h, acc_shock);
-                else acc = mfma_f16(a[0], h, acc);
+                acc = mfma_f16(a[0], h, acc);
                 small(mfma_f16, a[0], l);
                 small(mfma_f16, a[1], h);
             }
-            if constexpr (kSplitAcc) acc += acc_small + acc_shock;
+            if constexpr (kSplitAcc) acc += acc_small;
+            acc += curve;
             if constexpr (!kPf) {
                 if (wv >= 3) {
 #pragma unroll
@@ -661,15 +681,15 @@ hipError_t mfma_kernels_prepare()
 // The launch that takes the paths from `begin` on (one after another to the last path; every
 // path's result is the same whichever takes it): N-tiles per wave (0: a workgroup per
 // N-tile), waves per workgroup, workgroups. t = N-tiles per CU of the paths left. Path kernel
-// times in us by t, {workgroup per N-tile / 1 per wave / 2 per wave}, 10y reference (4
+// times in us by t, {workgroup per N-tile / 1 per wave / 2 per wave}, 10y reference (5
 // M-tiles) | 25y (7) | portfolio over 30y:
-//   t = 1   33 / 79 / 181  |  74 / 233 / 550 |  77 / 183 / 506
-//   t = 3   64 / 79 / 181  | 152 / 237 / 557 | 152 / 185 / 510
-//   t = 4   99 / 82 / 123  | 192 / 242 / 380 | 245 / 190 / 340
-//   t = 5  104 / 114 / 126 | 235 / 330 / 389 | 252 / 295 / 343
-//   t = 8  172 / 113 / 126 | 402 / 333 / 387 | 422 / 300 / 345
-//   t = 12 237 / 152 / 190 | 580 / 436 / 566 | 613 / 402 / 518
-//   t = 16 312 / 282 / 193 | 746 / 832 / 567 | 806 / 745 / 530
+//   t = 1   36 /  86 / 127 |  75 / 259 / 383 |  78 / 213 / 333
+//   t = 3   68 /  85 / 128 | 161 / 265 / 386 | 162 / 209 / 328
+//   t = 4  103 /  82 / 126 | 198 / 260 / 382 | 253 / 208 / 327
+//   t = 5  106 / 111 / 124 | 239 / 323 / 381 | 254 / 291 / 328
+//   t = 8  166 / 114 / 126 | 391 / 328 / 380 | 419 / 293 / 330
+//   t = 12 250 / 156 / 190 | 565 / 439 / 557 | 613 / 415 / 504
+//   t = 16 321 / 288 / 194 | 732 / 836 / 561 | 804 / 729 / 528
 // so: a workgroup per N-tile where its three to a CU (or a fuller second turn) serve, then a
 // wave each, then two to a wave. Past 16, whole turns of the chip go to {2, 8} and the rest
 // by the same rule (100000 paths: 368 -> 337 us, 25y 1114 -> 977; 80000: 366 -> 268).

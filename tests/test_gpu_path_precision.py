@@ -57,3 +57,15 @@ def test_blocks_add_their_roundings(expiry):
     assert np.all(x[inner] <= tol[inner])
     assert np.all(lny[inner] <= tol[inner])
     assert math.sqrt(float((x[inner] ** 2).mean())) <= 1.7e-7   # without the third accumulator 1.7 .. 2.3e-7
+
+
+@pytest.mark.parametrize("expiry", [15.0, 20.0, 25.0])
+def test_long_runs_add_their_roundings(expiry):
+    # the kernels of 6 and 7 tiles, for all slots that the backward difference does not reach
+    print("[gpu] %gy of blocks" % expiry, flush=True)
+    x, lny = _rms(expiry, 20000, 17)
+    blocks = np.arange(1, x.size + 1)
+    inner = blocks < 24
+    tol = 2.0 * np.sqrt(blocks) * 2.0 ** -24
+    assert np.all(x[inner] <= tol[inner])
+    assert np.all(lny[inner] <= tol[inner])
