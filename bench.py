@@ -475,7 +475,7 @@ def main():
                                "51 tenors, 3 factors, FP32 evolution + Kahan-compensated "
                                "integrals, EE/PFE97.5/CVA in FP64" % (PATHS, S),
                    "paths": PATHS, "steps_per_path": S, "tenors": 51, "factors": 3,
-                   "parallelism": "single GPU, one path per lane"},
+                   "parallelism": "single GPU"},
         "roofline": {"bound": "mfma" if args.path_kernel == "matrix" else "valu",
                      "achieved": achieved, "peak": PEAK_TFLOPS["f32"],
                      "unit": "TFLOP/s", "frac": achieved / PEAK_TFLOPS["f32"],

@@ -161,9 +161,10 @@ __device__ __forceinline__ void householder(double (&a)[kN], int lane, double* s
 }
 
 // Number of eigenvalues of the tridiagonal {d_j, e_{j-1}^2} below x: sign changes of the leading
-// minors' recurrence (3 FP64 instructions a row), rescaled every 8 rows: entries are at most
-// about 1 in magnitude, and e^2 has a floor of 2^-118, far below rounding, so that 8 rows lose
-// at most 2^-480 and a zero minor is followed by one of the opposite sign.
+// minors' recurrence (3 FP64 instructions a row), rescaled every 8 rows: the matrix's entries are
+// scaled to at most 1, so d, e and x are at most 51 or so (a parallel shift's d), and 8 rows
+// gain at most 2^64; e^2 has a floor of 2^-118, far below rounding, so that they lose at most
+// 2^-480, and a zero minor is followed by one of the opposite sign.
 __device__ __forceinline__ int sturm_count(const d2_t* s_de, double x)
 {
     // an opaque offset: the entries stay in LDS rather than in 204 registers across the calls
