@@ -52,7 +52,10 @@ __global__ __launch_bounds__(kWave) void block_map_kernel(const BlockMapParams p
         const size_t at = (size_t)(row % 16 + 16 * (k % 32 / 8)) * 8 + k % 8;
         auto part = [&](int p) -> uint16_t& { return frag[(size_t)mfma_frag(m, ch, p) * kWave * 8 + at]; };
         if (ch < 2) {
-            part(0) = bf16_part(w);
+            // an entry far below its row's largest has no part among the leading ones, whose
+            // products the matrix cores drop below 2^-24 of the largest beside them
+            const bool minor = fabs(w) < (row < n ? kMinorCurve : kMinorSum);
+            part(0) = minor ? (uint16_t)0 : bf16_part(w);
             part(1) = bf16_part(w);
             part(2) = bf16_part(w);
         } else {

@@ -312,6 +312,17 @@ inline BlockMapParams block_map_params(const double* spot, const double* drift, 
     return p;
 }
 
+// Curve columns: an entry below 2^-16 of its row's largest takes only the second and third part
+// (16 bits, 2^-32 of the largest). As a leading part its product would lie so far below the
+// others that the matrix cores drop it: with dt = 0.01f instead of 0.01 the last tenors' map has
+// entries of 2e-8 beside 1, which carry what the others lack to a row sum of 1, and without them
+// the last forwards drift, quadratically in time (mean error of EE over 10 curves against FP64:
+// 20y 1.8e-6, 25y 4.3e-6; with them 3.3e-7 and 3.5e-7). Lines from 2^-12 to 2^-20 measure the
+// same; at 2^-8 the products among the small ones are large enough that their truncation
+// shows (10y 3.3e-7 -> 4.5e-7). With dt / dtau = 1 / 50 the largest entries are 0.37 to 2 in
+// the curve's rows and 31 in the sums'.
+constexpr double kMinorCurve = 0x1p-17, kMinorSum = 0x1p-11;
+
 inline size_t block_map_elems(int mtiles) { return (size_t)mtiles * kMfmaTileFrags * kWave * 8; }
 
 // The FP64 block map for v_mfma_f64_16x16x4f64 (ref_paths_mfma64_kernel). One instruction

@@ -69,3 +69,21 @@ def test_long_runs_add_their_roundings(expiry):
     tol = 2.0 * np.sqrt(blocks) * 2.0 ** -24
     assert np.all(x[inner] <= tol[inner])
     assert np.all(lny[inner] <= tol[inner])
+
+
+@pytest.mark.parametrize("expiry", [20.0, 25.0])
+@pytest.mark.parametrize("spot,vol", [(1.0, 1.0), (1.1, 0.95), (0.9, 1.05)])
+def test_a_float_step_keeps_the_last_forwards(expiry, spot, vol):
+    # dt = 0.01f: c = 2 dt is not 0.02, and the last tenors' map has entries of 2e-8 that carry
+    # the rest of a row's sum. EE is a mean of sums of forwards less the rate, three times as
+    # sensitive as a forward, whose tolerance is the one of b blocks
+    print("[gpu] float step %gy, curve x %g, loadings x %g" % (expiry, spot, vol), flush=True)
+    m = hjm.benchmark_market()
+    vols = vol * m.volatilities
+    m = hjm.Market(spot * m.spot_rates, hjm.hjm_drift(vols), vols, m.accrual)
+    swap = hjm.InterestRateSwap(1e6, 0.025, expiry)
+    kw = dict(seed=19, pfe_quantile=0.975, dt=float(np.float32(0.01)))
+    a = hjm.simulate_reference(m, swap, 9000, precision=hjm.FP64, **kw).expected_exposure
+    b = hjm.simulate_reference(m, swap, 9000, precision=hjm.FP32_KAHAN, **kw).expected_exposure
+    tol = 3.0 * 2.0 * math.sqrt(2.0 * expiry) * 2.0 ** -24
+    assert np.linalg.norm(b - a) <= tol * np.linalg.norm(a)
