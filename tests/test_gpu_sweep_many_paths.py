@@ -67,3 +67,17 @@ def test_portions_do_not_change_the_sums(paths, expiry):
     assert a.stored_normals_bytes > 0 == b.stored_normals_bytes
     for k in FIELDS:
         assert np.array_equal(getattr(a, k), getattr(b, k))
+
+
+def test_a_large_book_of_many_paths_against_fp64():
+    # 65536 paths x 30y, 1024 swaps in 128 sets: the documented 1e-4 of the largest component
+    m, pf = hjm.benchmark_market(), hjm.synthetic_portfolio(1024, 128, seed=7)
+
+    def run(precision):
+        print("[gpu] book Greeks: 65536 paths x 30y, precision %d" % precision, flush=True)
+        return hjm.portfolio_cva_greeks(m, pf, 65536, horizon=30.0, precision=precision, seed=5)
+
+    a, b = run(hjm.FP64), run(hjm.FP32_KAHAN)
+    for k in FIELDS:
+        x, y = getattr(b, k), getattr(a, k)
+        assert np.max(np.abs(x - y)) <= 1e-4 * np.max(np.abs(y))
