@@ -7,7 +7,7 @@
 // three products of two-way fp16 splits (258 products per wave-block at 5 M-tiles against 408
 // with bf16 throughout, and 1.5 instead of 5.5 VALU instructions to split a shock: the 10y path
 // kernel at 131072 paths went from 0.55 to 0.44 ms; its forwards' error against FP64, with the
-// accumulators apart, from 2.0e-7 to 1.26e-7). The split products
+// accumulators apart, from 2.0e-7 to 1.24e-7). The split products
 // keep FP32 accuracy while running on the matrix cores concurrently with the VALU
 // (FP32 MFMA on gfx950 shares the vector pipeline and gains nothing over it). A wave owns
 // 32 paths = 2 N-tiles of 16 (the portfolio kernel's shape is a launch choice). The
@@ -91,7 +91,7 @@ __device__ __forceinline__ void for_each_index(F& f, std::integer_sequence<int, 
 // holds whole; the shocks' are 22 bits wide, and the curve's accumulator would cut their low
 // bits; with the small products they would cut those. Forwards against FP64, rms relative:
 //   10y (5 tiles) 2.1e-7 with the shocks' Wh xh in the curve's accumulator, 1.35e-7 in the small
-//     products', 1.26e-7 apart (2.0e-7 with three bf16 parts and two accumulators);
+//     products', 1.24e-7 apart (2.0e-7 with three bf16 parts and two accumulators);
 //   25y (7 tiles) 6.1e-6 with one accumulator, 1.2e-6 with two; EE 6.6e-7 and 3.6e-7, PFE 3.0e-6 and
 //     5.9e-7 (three bf16 parts and one accumulator 1.2e-6 and 4.0e-6).
 // kLate: the curve's products come last, a tile at a time, in registers that nothing else needs
